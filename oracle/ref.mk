@@ -17,7 +17,11 @@ LDFLAGS = -L$(TORCH_LIB) -Wl,-rpath,$(TORCH_LIB) -ltorch -ltorch_cpu -lc10
 HERE := $(dir $(abspath $(lastword $(MAKEFILE_LIST))))
 OUT := $(HERE)_ref
 
-all: $(OUT)/knn_ref.so $(OUT)/fps_ref.so
+# a checkout without its sources (an empty folder) leaves nothing to build
+KNN_SRC := $(wildcard $(REF)/torch_point_ops/knn/csrc/knn.cpp)
+FPS_SRC := $(wildcard $(REF)/torch_point_ops/fps/csrc/fps.cpp)
+
+all: $(if $(KNN_SRC),$(OUT)/knn_ref.so) $(if $(FPS_SRC),$(OUT)/fps_ref.so)
 
 $(OUT)/knn_ref.so: $(REF)/torch_point_ops/knn/csrc/knn.cpp
 	mkdir -p $(OUT)
