@@ -210,6 +210,20 @@ int tpo_knn_gather(int dtype, const void* x, const int64_t* idx,
                    int64_t U, void* out, void* stream);
 
 /*
+ * knn_gather backward: grad_x (N,M,U) = the sum of grad_out (N,L,K,U) over the
+ * entries (l, k), k < lengths[n], by row idx[n,l,k] (clamped to [0, M)); every
+ * row is written.  F32/F64/F16; half sums are taken in float and rounded once.
+ * The workspace size is 0 where the call does not apply (U > 7, very long
+ * clouds, no entries) and the call then returns TPO_ERR_ARG.
+ */
+int64_t tpo_knn_gather_bwd_workspace_size(int dtype, int64_t N, int64_t M, int64_t L, int64_t K,
+                                          int64_t U);
+int tpo_knn_gather_bwd(int dtype, const void* grad_out, const int64_t* idx,
+                       const int64_t* lengths, int64_t N, int64_t M, int64_t L, int64_t K,
+                       int64_t U, void* grad_x, void* workspace, int64_t workspace_bytes,
+                       void* stream);
+
+/*
  * KNN backward.  Replaces knn_cuda_backward (knn.cu:469-534),
  * torch_point_ops_knn::knn_backward (knn.cpp:170-171).
  *   idxs / grad_dists (N,P1,K); grad_p1 (N,P1,D), grad_p2 (N,P2,D) `dtype`.

@@ -358,6 +358,69 @@ def test_knn_gather_kernel_matches_torch_ops(tpo, dev, dtype, U, L):
         assert torch.allclose(ga, gb, rtol=1e-6, atol=1e-6)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.float16])
+@pytest.mark.parametrize("U,M,L,K,terms", [
+    (3, 513, 73, 7, "normal"),    # 511 entries, a second bucket of one row
+    (3, 1, 512, 1, "normal"),     # one row takes every entry of one workgroup
+    (1, 5000, 171, 3, "normal"),  # 513 entries: a workgroup with one
+    (4, 2000, 700, 5, "wide"),    # terms of 2^-60 .. 2^60: no common fixed point
+    (7, 140000, 40, 16, "normal"),  # buckets of more than 512 rows
+    (2, 600, 300, 4, "infinite"),
+    (3, 100, 60, 4, "zero"),
+    (8, 300, 90, 6, "normal"),    # longer rows: torch's scatter
+])
+def test_knn_gather_backward_vs_float64(tpo, dev, dtype, U, M, L, K, terms):
+    """Each row's gradient within the error of a float sum in any order,
+    (terms + 1) u sum|term|, of the float64 sum (half sums are taken in float and
+    rounded once; torch's own scatter rounds them at every addition)."""
+    g = torch.Generator().manual_seed(U * M + L)
+    N = 3
+    idx = torch.randint(0, M, (N, L, K), generator=g)
+    idx[0, :, 0] = M // 2  # many entries of one row
+    idx[1, 0, 0] = -1  # padding slots of the forward: clamped
+    go = torch.randn(N, L, K, U, generator=g, dtype=torch.float64)
+    if terms == "wide":
+        span = 7 if dtype == torch.float16 else 60
+        go = go * 2.0 ** torch.randint(-span, span + 1, go.shape, generator=g)
+    go = go.to(dtype)
+    if terms == "infinite":
+        go[0, 5, 1, 0] = float("inf")
+        go[2, 6, 0, 1] = float("nan")
+    if terms == "zero":
+        go.zero_()
+    lengths = torch.tensor([M, min(2, M), M])
+    keep = (torch.arange(K)[None] < lengths[:, None])[:, None, :, None]
+    t = torch.where(keep, go.double(), torch.zeros((), dtype=torch.float64)).reshape(N, L * K, U)
+    j = idx.clamp(0, M - 1).reshape(N, L * K, 1).expand(-1, -1, U)
+    want = torch.zeros(N, M, U, dtype=torch.float64).scatter_add(1, j, t)
+    mass = torch.zeros(N, M, U, dtype=torch.float64).scatter_add(1, j, t.abs())
+    many = torch.zeros(N, M, U, dtype=torch.float64).scatter_add(1, j, (t != 0).double())
+    x = torch.randn(N, M, U, generator=g).to(dev, dtype).requires_grad_(True)
+    (got,) = torch.autograd.grad(tpo.knn_gather(x, idx.to(dev), lengths.to(dev)), (x,), go.to(dev))
+    got = got.cpu().double()
+    fin = torch.isfinite(want)
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    inf = ~fin & ~torch.isnan(want)
+    assert torch.equal(got[inf], want[inf])
+    u = 2.0 ** (-53 if dtype == torch.float64 else -24)
+    bound = (many + 1) * u * mass
+    if dtype == torch.float16:
+        bound = (many if U > 7 else 0) * 2.0 ** -11 * mass + bound + want.abs() * 2.0 ** -11 + 2.0 ** -25
+    over = want.abs() > (65000 if dtype == torch.float16 else 1e300)
+    assert ((got - want).abs() <= bound)[fin & ~over].all()
+
+
+def test_knn_gather_gradient_of_the_gradient(tpo, dev):
+    g = torch.Generator().manual_seed(5)
+    x = torch.randn(2, 30, 3, generator=g, dtype=torch.float64).to(dev).requires_grad_(True)
+    idx = torch.randint(0, 30, (2, 9, 4), generator=g).to(dev)
+    lengths = torch.tensor([30, 2], device=dev)
+    assert torch.autograd.gradgradcheck(lambda t: tpo.knn_gather(t, idx, lengths).square(), (x,))
+    torch.library.opcheck(torch.ops.torch_point_ops_knn.knn_gather_backward.default,
+                          (torch.randn(2, 9, 4, 3, device=dev, requires_grad=True), idx, lengths, 30),
+                          raise_exception=True)
+
+
 def test_knn_points_sorted_and_gather(tpo, O, dev):
     g = torch.Generator().manual_seed(22)
     p1 = torch.randn(3, 40, 3, generator=g)

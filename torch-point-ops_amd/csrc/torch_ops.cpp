@@ -356,6 +356,47 @@ at::Tensor knn_gather_hip(const at::Tensor& x_in, const at::Tensor& idx_in,
   return out;
 }
 
+// knn_gather's gradient in x: records grouped by row and summed in LDS where
+// the rows are short (tpo_knn_gather_bwd), torch's scatter otherwise.
+at::Tensor knn_gather_backward_hip(const at::Tensor& go_in, const at::Tensor& idx_in,
+                                   const at::Tensor& lengths_in, int64_t M) {
+  check_hip(go_in, "grad_out");
+  c10::OptionalDeviceGuard guard(go_in.device());
+  TORCH_CHECK(go_in.dim() == 4 && idx_in.dim() == 3,
+              "knn_gather_backward expects (N,L,K,U) and (N,L,K)");
+  const int64_t N = go_in.size(0), L = go_in.size(1), K = go_in.size(2), U = go_in.size(3);
+  TORCH_CHECK(idx_in.size(0) == N && idx_in.size(1) == L && idx_in.size(2) == K,
+              "idx shape differs from grad_out");
+  TORCH_CHECK(idx_in.scalar_type() == at::kLong && lengths_in.scalar_type() == at::kLong,
+              "idx and lengths must be int64");
+  TORCH_CHECK(lengths_in.numel() == N, "lengths must have one entry per cloud");
+  TORCH_CHECK(go_in.device() == idx_in.device() && go_in.device() == lengths_in.device(),
+              "grad_out, idx and lengths must be on the same device");
+  TORCH_CHECK(M >= 0, "M must be non-negative");
+  const at::Tensor go = go_in.contiguous(), idx = idx_in.contiguous();
+  const at::Tensor lengths = lengths_in.contiguous();
+  int dt = -1;
+  if (go.scalar_type() == at::kFloat) dt = TPO_F32;
+  if (go.scalar_type() == at::kDouble) dt = TPO_F64;
+  if (go.scalar_type() == at::kHalf) dt = TPO_F16;
+  const int64_t wsb = dt < 0 ? 0 : tpo_knn_gather_bwd_workspace_size(dt, N, M, L, K, U);
+  if (wsb > 0) {
+    at::Tensor gx = at::empty({N, M, U}, go.options());
+    at::Tensor ws = at::empty({wsb}, go.options().dtype(at::kByte));
+    check_rc(tpo_knn_gather_bwd(dt, go.data_ptr(), idx.data_ptr<int64_t>(),
+                                lengths.data_ptr<int64_t>(), N, M, L, K, U, gx.data_ptr(),
+                                ws.data_ptr(), wsb, stream_of(go)),
+             "knn_gather_backward");
+    return gx;
+  }
+  at::Tensor gx = at::zeros({N, M, U}, go.options());
+  if (go.numel() == 0 || gx.numel() == 0) return gx;
+  const at::Tensor keep = at::arange(K, idx.options()).unsqueeze(0).lt(lengths.view({N, 1}));
+  const at::Tensor g = at::where(keep.view({N, 1, K, 1}), go, at::zeros({}, go.options()));
+  const at::Tensor j = idx.clamp(0, M - 1).view({N, L * K, 1}).expand({N, L * K, U});
+  return gx.scatter_add_(1, j, g.reshape({N, L * K, U}));
+}
+
 std::tuple<at::Tensor, at::Tensor> knn_backward_hip(const at::Tensor& p1_in,
                                                     const at::Tensor& p2_in,
                                                     const at::Tensor& lengths1_in,
@@ -588,11 +629,13 @@ TORCH_LIBRARY(torch_point_ops_knn, m) {
   m.def("knn_forward_sorted(Tensor p1, Tensor p2, Tensor lengths1, Tensor lengths2, "
         "int norm, int K, int version) -> (Tensor, Tensor)");
   m.def("knn_gather(Tensor x, Tensor idx, Tensor lengths) -> Tensor");
+  m.def("knn_gather_backward(Tensor grad_out, Tensor idx, Tensor lengths, int M) -> Tensor");
 }
 TORCH_LIBRARY_IMPL(torch_point_ops_knn, CUDA, m) {
   m.impl("knn_forward", &knn_forward_hip);
   m.impl("knn_forward_sorted", &knn_forward_sorted_hip);
   m.impl("knn_gather", &knn_gather_hip);
+  m.impl("knn_gather_backward", &knn_gather_backward_hip);
   m.impl("knn_backward", &knn_backward_hip);
 }
 

@@ -56,16 +56,11 @@ _SORTED_IN_KERNEL = (torch.float32, torch.float64, torch.float16)
 
 
 def _knn_gather_backward(ctx, grad_out):
-    # gather's gradient: scatter-add the rows back (the masked slots carry none)
+    # gather's gradient: the rows added back (the masked slots carry none)
     idx, lengths = ctx.saved_tensors
     if grad_out is None or not ctx.needs_input_grad[0]:
         return None, None, None
-    N, L, K, U = grad_out.shape
-    keep = (torch.arange(K, device=idx.device)[None] < lengths[:, None])[:, None, :, None]
-    g = (grad_out * keep).reshape(N, L * K, U)
-    j = idx.clamp(0, ctx.M - 1).reshape(N, L * K, 1).expand(-1, -1, U)
-    grad_x = torch.zeros(N, ctx.M, U, dtype=grad_out.dtype, device=grad_out.device)
-    return grad_x.scatter_add_(1, j, g), None, None
+    return torch.ops.torch_point_ops_knn.knn_gather_backward(grad_out, idx, lengths, ctx.M), None, None
 
 
 def _knn_gather_setup_context(ctx, inputs, output):
@@ -78,6 +73,31 @@ torch.library.register_autograd(
     "torch_point_ops_knn::knn_gather", _knn_gather_backward,
     setup_context=_knn_gather_setup_context,
 )
+
+
+def _knn_gather_backward_backward(ctx, grad_grad_x):
+    # linear in grad_out: its gradient is the gather itself
+    idx, lengths = ctx.saved_tensors
+    if grad_grad_x is None or not ctx.needs_input_grad[0]:
+        return None, None, None, None
+    gg = torch.ops.torch_point_ops_knn.knn_gather(grad_grad_x, idx.clamp(0, ctx.M - 1), lengths)
+    return gg, None, None, None
+
+
+def _knn_gather_backward_setup_context(ctx, inputs, output):
+    _grad_out, idx, lengths, ctx.M = inputs
+    ctx.save_for_backward(idx, lengths)
+
+
+torch.library.register_autograd(
+    "torch_point_ops_knn::knn_gather_backward", _knn_gather_backward_backward,
+    setup_context=_knn_gather_backward_setup_context,
+)
+
+
+@torch.library.register_fake("torch_point_ops_knn::knn_gather_backward")
+def _knn_gather_backward_fake(grad_out, idx, lengths, M):
+    return grad_out.new_empty(grad_out.shape[0], M, grad_out.shape[3])
 
 
 @torch.library.register_fake("torch_point_ops_knn::knn_gather")
