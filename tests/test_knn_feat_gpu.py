@@ -1,0 +1,103 @@
+"""knn_points rows of float points with many dimensions: candidates from the
+matrix cores by an exact bound, equal distances replayed.  Every row must be
+the reference-order forward's row as the module's sort leaves it, bit for bit."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _sorted_by_module(idxs, dists, lengths2, K):
+    # knn_points' sort after the forward (reference knn/__init__.py:111-131)
+    pad = (lengths2[:, None] <= torch.arange(K, device=dists.device)[None])[:, None].expand_as(dists)
+    ds, order = dists.masked_fill(pad, float("inf")).sort(dim=2)
+    return idxs.gather(2, order), ds.masked_fill(pad, 0.0)
+
+
+def _check(tpo, dev, p1, p2, l1, l2, K):
+    a, b, la, lb = p1.to(dev), p2.to(dev), l1.to(dev), l2.to(dev)
+    for version in (-1, 0):
+        si, sd = tpo.knn_points(a, b, la, lb, K=K, version=version)
+        ri, rd = torch.ops.torch_point_ops_knn.knn_forward(a, b, la, lb, 2, K, version)
+        ei, ed = _sorted_by_module(ri, rd, lb, K)
+        assert torch.equal(sd.isnan(), ed.isnan())
+        assert torch.equal(torch.nan_to_num(sd), torch.nan_to_num(ed))
+        assert torch.equal(si, ei)
+
+
+# widths at the edges of the 16-wide k-steps with six more entries for the
+# norms, and not multiples of 4; reference counts at the edges of the tiles
+# (32), of the all-candidates lists (192), of the fine groups (31 tiles) and of
+# several tiles a group (over 128 tiles a wave)
+@pytest.mark.parametrize("D,P1,P2,K", [
+    (4, 70, 1, 3), (9, 64, 31, 5), (10, 65, 33, 20), (11, 130, 192, 32), (26, 63, 193, 32),
+    (27, 200, 255, 16), (35, 333, 992, 20), (42, 1, 993, 2), (58, 128, 1024, 10),
+    (64, 500, 2048, 20), (74, 96, 3000, 32), (90, 33, 5000, 5), (106, 40, 700, 8),
+    (122, 64, 4128, 31), (128, 257, 9001, 16), (64, 30, 33000, 32), (16, 700, 4095, 12),
+])
+@pytest.mark.parametrize("case", ["normal", "offset", "self"])
+def test_feature_rows_match_the_reference_order(tpo, dev, D, P1, P2, K, case):
+    g = torch.Generator().manual_seed(D * P2 + K)
+    N = 2
+    p2 = torch.randn(N, P2, D, generator=g)
+    p1 = torch.randn(N, P1, D, generator=g)
+    if case == "offset":  # far from the origin, widths of very different sizes
+        scale = 2.0 ** torch.randint(-6, 7, (D,), generator=g)
+        p1, p2 = (p1 * scale + 50).float(), (p2 * scale + 50).float()
+    if case == "self":
+        p1 = p2[:, torch.randint(0, P2, (P1,), generator=g)].contiguous()
+    l1 = torch.tensor([P1, max(1, P1 - 5)])
+    l2 = torch.tensor([P2, max(1, (2 * P2) // 3)])
+    _check(tpo, dev, p1, p2, l1, l2, K)
+
+
+@pytest.mark.parametrize("case", ["few_ties", "all_ties", "runs", "nonfinite_query",
+                                  "nonfinite_cloud", "huge", "tiny", "short", "far_cloud"])
+@pytest.mark.parametrize("D,K", [(64, 20), (9, 5)])
+def test_feature_rows_replayed_and_edge_values(tpo, dev, case, D, K):
+    g = torch.Generator().manual_seed(len(case) + D)
+    N, P1, P2 = 3, 900, 1500
+    p1 = torch.randn(N, P1, D, generator=g)
+    p2 = torch.randn(N, P2, D, generator=g)
+    l1, l2 = torch.tensor([P1, P1, 500]), torch.tensor([P2, 1100, P2])
+    if case == "few_ties":  # copies of a few references, queries beside them
+        p2[:, 700:710] = p2[:, 100:110]
+        p1[:, :10] = p2[:, 100:110] + 1e-3
+    elif case == "all_ties":  # every row: more than the replay takes
+        p1 = torch.randint(0, 2, (N, P1, D), generator=g).float()
+        p2 = torch.randint(0, 2, (N, P2, D), generator=g).float()
+    elif case == "runs":  # all neighbours of a query next to each other in the cloud
+        c = torch.randn(N, P2 // 50, 1, D, generator=g) * 10
+        p2 = (c + 0.1 * torch.randn(N, P2 // 50, 50, D, generator=g)).reshape(N, P2, D)
+        p1 = (c[:, torch.randint(0, P2 // 50, (P1,), generator=g), 0]
+              + 0.1 * torch.randn(N, P1, D, generator=g))
+    elif case == "nonfinite_query":
+        p1[0, 3, 2] = float("nan")
+        p1[1, 4, 0] = float("inf")
+    elif case == "nonfinite_cloud":
+        p2[0, 5, 1] = float("inf")
+        p2[1, 7, 1] = float("nan")
+        p2[2, 0, 0] = float("nan")
+    elif case == "huge":  # distances that overflow to infinity
+        p2[0, ::3] *= 1e25
+        p1[1] *= 1e30
+    elif case == "tiny":
+        p1, p2 = p1 * 1e-22, p2 * 1e-22
+    elif case == "short":
+        l2 = torch.tensor([K - 1, 0, 3])
+    else:
+        p1 = p1 + 1e4
+    _check(tpo, dev, p1, p2, l1, l2, K)
+
+
+@pytest.mark.parametrize("D,P2", [(4, 3), (16, 500), (64, 2100)])
+def test_single_nearest_takes_the_lower_index(tpo, O, dev, D, P2):
+    g = torch.Generator().manual_seed(P2)
+    p2 = torch.randint(0, 3, (2, P2, D), generator=g).float()  # many equal rows
+    p1 = torch.randint(0, 3, (2, 150, D), generator=g).float()
+    l1, l2 = torch.tensor([150, 90]), torch.tensor([P2, 0])
+    for version in (-1, 0):
+        i, d = tpo.knn_points(p1.to(dev), p2.to(dev), l1.to(dev), l2.to(dev), K=1, version=version)
+        ei, ed = O.knn_fwd(p1.numpy(), p2.numpy(), l1.numpy(), l2.numpy(), K=1, version=version)
+        assert np.array_equal(i.cpu().numpy(), ei) and np.array_equal(d.cpu().numpy(), ed)

@@ -26,7 +26,7 @@ INCLUDE = os.path.join(REPO, "include")
 ROCM = os.environ.get("ROCM_PATH", "/opt/rocm")
 ARCH = "gfx950"
 
-HIP_SOURCES = ["capi.hip", "chamfer.hip", "chamfer_grid.hip", "knn.hip", "knn_hd.hip", "knn_bwd.hip", "knn_grid.hip", "knn_bf16.hip", "fps.hip", "gather.hip", "emd.hip"]
+HIP_SOURCES = ["capi.hip", "chamfer.hip", "chamfer_grid.hip", "knn.hip", "knn_hd.hip", "knn_bwd.hip", "knn_grid.hip", "knn_feat.hip", "knn_redo.hip", "knn_bf16.hip", "fps.hip", "gather.hip", "emd.hip"]
 
 HIPCC_FLAGS = [
     f"--offload-arch={ARCH}",
@@ -45,9 +45,11 @@ HIPCC_FLAGS = [
 ]
 
 # fps.hip: its one-lane LDS atomic needs no wave-level pre-reduction.
-# knn_bf16.hip: MFMA results in VGPRs, read by the VALU without AGPR copies.
+# knn_bf16.hip, knn_feat.hip: MFMA results in VGPRs, read by the VALU without
+# AGPR copies.
 HIPCC_FILE_FLAGS: dict = {"fps.hip": ["-mllvm", "-amdgpu-atomic-optimizer-strategy=None"],
-                          "knn_bf16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
+                          "knn_bf16.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"],
+                          "knn_feat.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form"]}
 
 
 def _run(cmd, verbose):

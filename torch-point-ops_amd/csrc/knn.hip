@@ -25,7 +25,7 @@
 //   reference's global-memory MinK.
 #include <utility>
 
-#include "knn_common.hpp"
+#include "knn_replay.hpp"
 
 namespace tpo {
 // knn_bf16.hip
@@ -40,6 +40,12 @@ int64_t hd_workspace_bytes(int64_t rows, int64_t S, int64_t K);
 void launch_hd(const void* p1, const void* p2, const int64_t* l1, const int64_t* l2, int N, int P1,
                int P2, int D, int K, int norm, int S, int pad, bool sort, int64_t* idxs,
                void* dists, void* ws, hipStream_t s);
+// knn_feat.hip
+bool knn_feat_applies(int dtype, int64_t N, int64_t P1, int64_t P2, int64_t D, int64_t K, int norm);
+int64_t knn_feat_workspace(int64_t N, int64_t P1, int64_t P2, int64_t D);
+RedoList launch_knn_feat(const void* p1, const void* p2, const int64_t* l1, const int64_t* l2,
+                         int N, int P1, int P2, int D, int K, int pad, bool sort, int64_t* idxs,
+                         void* dists, void* ws, hipStream_t s);
 // knn_grid.hip
 bool knn_grid_applies(int dtype, int64_t D, int64_t K, int64_t P2);
 int64_t knn_grid_workspace(int64_t N, int64_t P2);
@@ -155,12 +161,15 @@ __global__ __launch_bounds__(1024) void knn_order_kernel(const T* __restrict__ p
 
 // mode bit 0: RegisterMinK<2> (version 3, K = 2); bit 1 (= SORT): rows
 // sorted as knn_points(return_sorted=True) returns them (knn_sort_row).
+// redo: the counts of a RedoList whose queries `order` holds, or null.  With
+// one, the listed rows alone are processed, when there are over REDO_LIMIT.
 template <typename T, int DT, int NORM, int KC, bool SORT>
 __global__ __launch_bounds__(256) void knn_fwd_kernel(
     const T* __restrict__ p1, const T* __restrict__ p2, const int64_t* __restrict__ len1,
     const int64_t* __restrict__ len2, const int32_t* __restrict__ order, int P1, int P2, int D,
-    int K, int nqb, int pad_sentinel, int mode, int64_t* __restrict__ idxs,
-    T* __restrict__ dists) {
+    int K, int nqb, int pad_sentinel, int mode, const uint32_t* __restrict__ redo,
+    int64_t* __restrict__ idxs, T* __restrict__ dists) {
+  if (redo && redo[0] <= REDO_LIMIT) return;
   const int sorted2 = mode & 1;
   // float D=3: reference points reach the lanes through a wave-private LDS
   // block (each lane stages one, every lane reads them back as broadcasts),
@@ -170,7 +179,7 @@ __global__ __launch_bounds__(256) void knn_fwd_kernel(
   __shared__ float4 s_ref[STAGED ? 4 : 1][64];
   const int n = blockIdx.x / nqb;
   const int i = (blockIdx.x - n * nqb) * 256 + threadIdx.x;  // position in processing order
-  const bool in_range = i < P1;
+  const bool in_range = i < (redo ? (int)redo[1 + n] : P1);
   if (!STAGED && !in_range) return;
   const int q = in_range ? (order ? order[(size_t)n * P1 + i] : i) : 0;  // query row of this lane
   int64_t l1 = len1[n], l2 = len2[n];
@@ -412,62 +421,63 @@ __global__ __launch_bounds__(256) void knn_fwd_global_kernel(
 template <typename T, int DT, int NORM, int KC>
 void launch_fwd_kc(const void* p1, const void* p2, const int64_t* l1, const int64_t* l2,
                    const int32_t* order, int N, int P1, int P2, int D, int K, int pad,
-                   int sorted2, int64_t* idxs, void* dists, hipStream_t s) {
+                   int sorted2, const uint32_t* redo, int64_t* idxs, void* dists, hipStream_t s) {
   const int nqb = (P1 + 255) / 256;
   if (sorted2 & 2)
     hipLaunchKernelGGL((knn_fwd_kernel<T, DT, NORM, KC, true>), dim3(N * nqb), dim3(256), 0, s,
                        (const T*)p1, (const T*)p2, l1, l2, order, P1, P2, D, K, nqb, pad, sorted2,
-                       idxs, (T*)dists);
+                       redo, idxs, (T*)dists);
   else
     hipLaunchKernelGGL((knn_fwd_kernel<T, DT, NORM, KC, false>), dim3(N * nqb), dim3(256), 0, s,
                        (const T*)p1, (const T*)p2, l1, l2, order, P1, P2, D, K, nqb, pad, sorted2,
-                       idxs, (T*)dists);
+                       redo, idxs, (T*)dists);
 }
 
 template <typename T, int DT, int NORM>
 void launch_fwd_dt(const void* p1, const void* p2, const int64_t* l1, const int64_t* l2,
                    const int32_t* order, int N, int P1, int P2, int D, int K, int pad,
-                   int sorted2, int64_t* idxs, void* dists, hipStream_t s) {
-  if (K <= 4) launch_fwd_kc<T, DT, NORM, 4>(p1, p2, l1, l2, order, N, P1, P2, D, K, pad, sorted2, idxs, dists, s);
-  else if (K <= 8) launch_fwd_kc<T, DT, NORM, 8>(p1, p2, l1, l2, order, N, P1, P2, D, K, pad, sorted2, idxs, dists, s);
-  else if (K <= 16) launch_fwd_kc<T, DT, NORM, 16>(p1, p2, l1, l2, order, N, P1, P2, D, K, pad, sorted2, idxs, dists, s);
-  else launch_fwd_kc<T, DT, NORM, 32>(p1, p2, l1, l2, order, N, P1, P2, D, K, pad, sorted2, idxs, dists, s);
+                   int sorted2, const uint32_t* redo, int64_t* idxs, void* dists, hipStream_t s) {
+  if (K <= 4) launch_fwd_kc<T, DT, NORM, 4>(p1, p2, l1, l2, order, N, P1, P2, D, K, pad, sorted2, redo, idxs, dists, s);
+  else if (K <= 8) launch_fwd_kc<T, DT, NORM, 8>(p1, p2, l1, l2, order, N, P1, P2, D, K, pad, sorted2, redo, idxs, dists, s);
+  else if (K <= 16) launch_fwd_kc<T, DT, NORM, 16>(p1, p2, l1, l2, order, N, P1, P2, D, K, pad, sorted2, redo, idxs, dists, s);
+  else launch_fwd_kc<T, DT, NORM, 32>(p1, p2, l1, l2, order, N, P1, P2, D, K, pad, sorted2, redo, idxs, dists, s);
 }
 
 template <typename T, int NORM>
 void launch_fwd_norm(const void* p1, const void* p2, const int64_t* l1, const int64_t* l2,
                      int32_t* order, int N, int P1, int P2, int D, int K, int pad, int sorted2,
-                     int64_t* idxs, void* dists, hipStream_t s) {
+                     const uint32_t* redo, int64_t* idxs, void* dists, hipStream_t s) {
   if (K > 32) {
     const int nqb = (P1 + 255) / 256;
     hipLaunchKernelGGL((knn_fwd_global_kernel<T, NORM>), dim3(N * nqb), dim3(256), 0, s,
                        (const T*)p1, (const T*)p2, l1, l2, P1, P2, D, K, nqb, idxs, (T*)dists);
   } else if (D == 3) {
-    if (order)
+    if (order && !redo)
       hipLaunchKernelGGL(knn_order_kernel<T>, dim3(N), dim3(1024), 0, s, (const T*)p1, l1, P1,
                          order);
-    launch_fwd_dt<T, 3, NORM>(p1, p2, l1, l2, order, N, P1, P2, D, K, pad, sorted2, idxs, dists, s);
+    launch_fwd_dt<T, 3, NORM>(p1, p2, l1, l2, order, N, P1, P2, D, K, pad, sorted2, redo, idxs, dists, s);
   } else {
+    if (!redo) order = nullptr;
     if constexpr (sizeof(T) == 4) {  // common high-D widths: float query held in VGPRs
       if (D == 128) {
-        launch_fwd_dt<T, 128, NORM>(p1, p2, l1, l2, nullptr, N, P1, P2, D, K, pad, sorted2, idxs, dists, s);
+        launch_fwd_dt<T, 128, NORM>(p1, p2, l1, l2, order, N, P1, P2, D, K, pad, sorted2, redo, idxs, dists, s);
         return;
       }
       if (D == 64) {
-        launch_fwd_dt<T, 64, NORM>(p1, p2, l1, l2, nullptr, N, P1, P2, D, K, pad, sorted2, idxs, dists, s);
+        launch_fwd_dt<T, 64, NORM>(p1, p2, l1, l2, order, N, P1, P2, D, K, pad, sorted2, redo, idxs, dists, s);
         return;
       }
     }
-    launch_fwd_dt<T, 0, NORM>(p1, p2, l1, l2, nullptr, N, P1, P2, D, K, pad, sorted2, idxs, dists, s);
+    launch_fwd_dt<T, 0, NORM>(p1, p2, l1, l2, order, N, P1, P2, D, K, pad, sorted2, redo, idxs, dists, s);
   }
 }
 
 template <typename T>
 void launch_fwd(const void* p1, const void* p2, const int64_t* l1, const int64_t* l2,
                 int32_t* order, int N, int P1, int P2, int D, int K, int norm, int pad,
-                int sorted2, int64_t* idxs, void* dists, hipStream_t s) {
-  if (norm == 1) launch_fwd_norm<T, 1>(p1, p2, l1, l2, order, N, P1, P2, D, K, pad, sorted2, idxs, dists, s);
-  else launch_fwd_norm<T, 2>(p1, p2, l1, l2, order, N, P1, P2, D, K, pad, sorted2, idxs, dists, s);
+                int sorted2, const uint32_t* redo, int64_t* idxs, void* dists, hipStream_t s) {
+  if (norm == 1) launch_fwd_norm<T, 1>(p1, p2, l1, l2, order, N, P1, P2, D, K, pad, sorted2, redo, idxs, dists, s);
+  else launch_fwd_norm<T, 2>(p1, p2, l1, l2, order, N, P1, P2, D, K, pad, sorted2, redo, idxs, dists, s);
 }
 
 // dispatch.cuh:114-147
@@ -497,7 +507,9 @@ extern "C" int64_t tpo_knn_workspace_size(int dtype, int64_t N, int64_t P1, int6
   if (knn_grid_applies(dtype, D, K, P2)) order += knn_grid_workspace(N, P2);
   const int S = hd_slices(dtype, N, P1, P2, D, K);
   const int64_t hd = S > 0 ? hd_workspace_bytes(N * P1, S, K) : 0;
-  return order > hd ? order : hd;
+  const int64_t feat =
+      knn_feat_applies(dtype, N, P1, P2, D, K, norm) ? knn_feat_workspace(N, P1, P2, D) : 0;
+  return std::max(order, std::max(hd, feat));
 }
 
 static int knn_fwd_impl(int dtype, const void* p1, const void* p2, const int64_t* lengths1,
@@ -534,6 +546,19 @@ static int knn_fwd_impl(int dtype, const void* p1, const void* p2, const int64_t
   const int pad = v <= 1;
   const int sorted2 = (v == 3 && K == 2) | (sort_rows ? 2 : 0);  // the kernel's mode bits
   hipStream_t s = (hipStream_t)stream;
+  // rows by distance, many dimensions: candidates from the matrix cores
+  if ((sort_rows || K == 1) && !(sorted2 & 1) && D != 3 && workspace &&
+      knn_feat_applies(dtype, N, P1, P2, D, K, norm) &&
+      workspace_bytes >= knn_feat_workspace(N, P1, P2, D)) {
+    const RedoList r =
+        launch_knn_feat(p1, p2, lengths1, lengths2, (int)N, (int)P1, (int)P2, (int)D, (int)K, pad,
+                        sort_rows, idxs, dists, workspace, s);
+    launch_knn_redo(p1, p2, lengths1, lengths2, (int)N, (int)P1, (int)P2, (int)D, (int)K, norm, pad,
+                    sort_rows, r, idxs, dists, s);
+    launch_fwd<float>(p1, p2, lengths1, lengths2, r.queries, (int)N, (int)P1, (int)P2, (int)D,
+                      (int)K, norm, pad, sorted2, r.total, idxs, dists, s);
+    return check_launch("tpo_knn_fwd");
+  }
   {  // long reference clouds, few queries: references sliced over workgroups
     const int S = hd_slices(dtype, N, P1, P2, D, K);
     if (S > 0 && workspace && workspace_bytes >= hd_workspace_bytes(N * P1, S, K) && v <= 1) {
@@ -553,9 +578,9 @@ static int knn_fwd_impl(int dtype, const void* p1, const void* p2, const int64_t
     return check_launch("tpo_knn_fwd");
   }
   switch (dtype) {
-    case TPO_F32: launch_fwd<float>(p1, p2, lengths1, lengths2, order, (int)N, (int)P1, (int)P2, (int)D, (int)K, norm, pad, sorted2, idxs, dists, s); break;
-    case TPO_F64: launch_fwd<double>(p1, p2, lengths1, lengths2, order, (int)N, (int)P1, (int)P2, (int)D, (int)K, norm, pad, sorted2, idxs, dists, s); break;
-    case TPO_F16: launch_fwd<half_t>(p1, p2, lengths1, lengths2, order, (int)N, (int)P1, (int)P2, (int)D, (int)K, norm, pad, sorted2, idxs, dists, s); break;
+    case TPO_F32: launch_fwd<float>(p1, p2, lengths1, lengths2, order, (int)N, (int)P1, (int)P2, (int)D, (int)K, norm, pad, sorted2, nullptr, idxs, dists, s); break;
+    case TPO_F64: launch_fwd<double>(p1, p2, lengths1, lengths2, order, (int)N, (int)P1, (int)P2, (int)D, (int)K, norm, pad, sorted2, nullptr, idxs, dists, s); break;
+    case TPO_F16: launch_fwd<half_t>(p1, p2, lengths1, lengths2, order, (int)N, (int)P1, (int)P2, (int)D, (int)K, norm, pad, sorted2, nullptr, idxs, dists, s); break;
     default: return set_error(TPO_ERR_DTYPE, "tpo_knn_fwd: unsupported dtype %d", dtype);
   }
   return check_launch("tpo_knn_fwd");

@@ -4,7 +4,7 @@
 // MinK slot layout of mink.cuh:77-121), references sliced over the GPU.
 #include <utility>
 
-#include "knn_common.hpp"
+#include "knn_replay.hpp"
 
 #pragma clang fp contract(off)
 
@@ -223,31 +223,9 @@ __global__ __launch_bounds__(256) void knn_hd_slice_kernel(
   if (q < P1) cnt[cs] = act ? count : 0;
 }
 
-// The merge runs one wave per query row.  The replay's K slots live one per
-// lane (lanes 0 .. K-1) as a list ordered by (value, slot descending), NaN
-// values first: the last lane then holds the slot that first_max picks (the
-// first slot holding the largest value; a NaN never becomes the maximum
-// unless it sits in slot 0, and then the threshold is NaN and nothing is
-// ever inserted).  Inserting (d, j) below the threshold puts it into the
-// last element's slot: the lanes whose key exceeds the new one shift up one
-// lane (DPP wave_shr) and the new entry lands in the gap.  Candidates come
-// 64 at a time, one per lane; a ballot against the threshold finds the next
-// insertion in index order, and is taken again after each one.
-
-// order key of a distance: the compare-equal floats share one (-0 as +0),
-// NaN below every number
-__device__ __forceinline__ uint32_t hd_ord(float v) {
-  const uint32_t u = __float_as_uint(v == 0.f ? 0.f : v);
-  return v != v ? 0u : ((u & 0x80000000u) ? ~u : (u | 0x80000000u));
-}
-__device__ __forceinline__ int hd_shr1(int x) {  // lane i takes lane i-1 (lane 0: 0)
-  return __builtin_amdgcn_mov_dpp(x, 0x138, 0xF, 0xF, true);
-}
-__device__ __forceinline__ int hd_lane(int x, int l) { return __builtin_amdgcn_readlane(x, l); }
-__device__ __forceinline__ float hd_lane(float x, int l) {
-  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x), l));
-}
-
+// The merge runs one wave per query row (ReplayRow, knn_replay.hpp).
+// Candidates come 64 at a time, one per lane; a ballot against the threshold
+// finds the next insertion in index order, and is taken again after each one.
 template <int DT, int NORM, int KC, bool SORT>
 __global__ __launch_bounds__(256) void knn_hd_merge_kernel(
     const float* __restrict__ p1, const float* __restrict__ p2, const int64_t* __restrict__ len1,
@@ -278,52 +256,14 @@ __global__ __launch_bounds__(256) void knn_hd_merge_kernel(
   // lane s < K: slot s of the fill (with more than K references the first
   // slice stored its distances)
   const int fill = L2 < K ? L2 : K;
-  float v = Lim<float>::inf();
-  int ix = -1;
+  ReplayRow rr;
+  rr.v = Lim<float>::inf();
+  rr.ix = -1;
   if (lane < fill) {
-    v = L2 > K ? fd[row * K + lane] : dist(lane);
-    ix = lane;
+    rr.v = L2 > K ? fd[row * K + lane] : dist(lane);
+    rr.ix = lane;
   }
-  if (L2 > K && hd_lane(v, 0) == hd_lane(v, 0)) {
-    // the fill as the ordered list: lane s moves to its rank.  An entry is
-    // (value, slot << 26 | index) (references fewer than 2^26).
-    const uint64_t key = ((uint64_t)hd_ord(v) << 32) | (uint32_t)(63 - lane);
-    int rank = 0;
-#pragma unroll
-    for (int t = 0; t < KC; ++t) {
-      if (t < K) {
-        const uint64_t kt = ((uint64_t)(uint32_t)hd_lane((int)(key >> 32), t) << 32) |
-                            (uint32_t)hd_lane((int)(uint32_t)key, t);
-        rank += kt < key ? 1 : 0;
-      }
-    }
-    const int to = 4 * (lane < K ? rank : lane);
-    v = __int_as_float(__builtin_amdgcn_ds_permute(to, __float_as_int(v)));
-    int pk = __builtin_amdgcn_ds_permute(to, (lane << 26) | ix);
-    float thr = hd_lane(v, K - 1);
-    // (d, j) takes the last entry's slot; the entries after it in the order
-    // (a larger value, or an equal one in a lower slot) move up one lane
-    auto insert = [&](float d, int j) {
-      const int sr = hd_lane(pk, K - 1) & ~0x3ffffff;
-      const float vp = __int_as_float(hd_shr1(__float_as_int(v)));
-      const int pp = hd_shr1(pk);
-      // bitwise, not short-circuit: no branches in the wave-wide step
-      const bool in = lane < K;
-      const bool gt = in & ((v > d) | ((v == d) & (pk < sr)));
-      const bool gtp = in & (lane > 0) & ((vp > d) | ((vp == d) & (pp < sr)));
-      v = gtp ? vp : (gt ? d : v);
-      pk = gtp ? pp : (gt ? (sr | j) : pk);
-      thr = hd_lane(v, K - 1);
-    };
-    // one candidate per lane, in index order across the lanes
-    auto batch = [&](float di, int ji, bool ok) {
-      uint64_t m = __ballot(ok && di < thr);
-      while (m != 0) {
-        const int e = __builtin_ctzll(m);
-        insert(hd_lane(di, e), hd_lane(ji, e));
-        m &= __ballot(ok && di < thr) & ~((2ull << e) - 1ull);
-      }
-    };
+  if (L2 > K && rr.begin(K, lane)) {
     for (int sl = 0; sl < S; ++sl) {
       const int a = K + sl * slen, b = min(L2, a + slen);
       if (a >= b) break;
@@ -333,49 +273,24 @@ __global__ __launch_bounds__(256) void knn_hd_merge_kernel(
         const int32_t* __restrict__ cip = ci + (row * S + sl) * HD_CAP;
         for (int k0 = 0; k0 < c; k0 += 64) {
           const int k = min(k0 + lane, c - 1);  // lanes past the list repeat its last entry
-          batch(cdp[k], cip[k], k0 + lane < c);
+          rr.batch<true>(replay_ord(cdp[k]), cip[k], k0 + lane < c, K);
         }
       } else {  // the slice's list overflowed: recompute it in order
         for (int j0 = a; j0 < b; j0 += 64) {
           const int j = min(j0 + lane, b - 1);
-          batch(dist(j), j, j0 + lane < b);
+          rr.batch<false>(replay_ord(dist(j)), j0, j0 + lane < b, K);
         }
       }
     }
-    // back to slot order: lane s takes slot s
-    const int back = 4 * (lane < K ? (pk >> 26) : lane);
-    v = __int_as_float(__builtin_amdgcn_ds_permute(back, __float_as_int(v)));
-    ix = __builtin_amdgcn_ds_permute(back, pk) & 0x3ffffff;
+    rr.end(K, lane);
   }
   const int size = fill;
   const int64_t pad_i = pad_sentinel ? -1 : 0;
   const float pad_d = pad_sentinel ? Lim<float>::inf() : 0.f;
   if constexpr (SORT) {
-    // knn_sort_row's network with position p in lane p: an exchange of
-    // positions (a, a + stride) runs in both lanes, which agree on it
-    float d = lane < size ? v : Lim<float>::inf();
-    int x = lane < size ? ix : (int)pad_i;
-    int va = lane < K ? 1 : 0;
-    auto cas = [&](int stride, bool up) {
-      const float pd = __shfl_xor(d, stride);
-      const int px = __shfl_xor(x, stride), pv = __shfl_xor(va, stride);
-      const bool lo = (lane & stride) == 0;
-      const float da = lo ? d : pd, db = lo ? pd : d;
-      const bool vA = (lo ? va : pv) != 0, vB = (lo ? pv : va) != 0;
-      const bool lt = !knn_isnan(da) && (knn_isnan(db) || da < db);
-      const bool sw = ((lt && vA) || !vB) == up;
-      if ((lane | stride) < KC && sw) {
-        d = pd;
-        x = px;
-        va = pv;
-      }
-    };
-#pragma unroll
-    for (int sz = 2; sz < 32; sz *= 2)
-#pragma unroll
-      for (int stride = sz / 2; stride > 0; stride /= 2) cas(stride, (lane & sz) != 0);
-#pragma unroll
-    for (int stride = 16; stride > 0; stride /= 2) cas(stride, false);
+    float d;
+    int x;
+    rr.sort<KC>(K, size, (int)pad_i, lane, d, x);
     if (lane < K) {
       io[lane] = (int64_t)x;
       dout[lane] = lane < size ? d : 0.f;
@@ -383,8 +298,8 @@ __global__ __launch_bounds__(256) void knn_hd_merge_kernel(
     return;
   }
   if (lane < K) {
-    io[lane] = lane < size ? (int64_t)ix : pad_i;
-    dout[lane] = lane < size ? v : pad_d;
+    io[lane] = lane < size ? (int64_t)rr.ix : pad_i;
+    dout[lane] = lane < size ? rr.v : pad_d;
   }
 }
 

@@ -1,0 +1,225 @@
+// knn_redo.hip -- the MinK process (knn.cu:113-168, mink.cuh:77-121) of the few
+// query rows whose result the sorted distances do not decide: equal distances
+// come out in an order that depends on the whole insertion history, so those
+// rows are replayed.  The KNN kernels that select by distance list them
+// (RedoList); random clouds leave a few rows a call.
+//
+// A workgroup a row: its waves compute the distances of a window of
+// references into LDS, then one wave replays them in index order (ReplayRow).
+// Bound by the row's serial insertions (about K ln(P2 / K) of them); the
+// rows run side by side.
+#include "knn_replay.hpp"
+
+#pragma clang fp contract(off)
+
+namespace tpo {
+namespace {
+
+constexpr int KR_THREADS = 1024;
+constexpr int KR_GRID = 256;
+constexpr int KR_DC = 32;          // dimensions a wave stages at once
+constexpr int KR_DS = KR_DC + 4;   // floats between staged rows (16-byte reads, distinct banks)
+constexpr int KR_DIRECT = 8;       // up to this width a lane reads its row itself
+// distances held in LDS at once: with staged rows beside them, and without
+constexpr int KR_WIN = 2048, KR_WIN_DIRECT = 32768;
+constexpr int KR_STAGE = KR_THREADS / 64 * 64 * KR_DS;
+constexpr int KR_LDS = KR_WIN + KR_STAGE > KR_WIN_DIRECT ? KR_WIN + KR_STAGE : KR_WIN_DIRECT;
+
+// Distances (knn.cu:148-158) of references [w0, w0 + wn) to the query q (zeros
+// past D), as replay_ord, into s_d: each wave batches of 64 references, a
+// lane a reference.  A lane's sum runs over its row's dimensions in order, so
+// wider rows pass through LDS 32 dimensions at a time: loads cover whole
+// 128-byte lines (a lane a row would touch 64 lines an instruction), and the
+// next step's are in flight while one is summed.  The sums start at 0 and run
+// on over zeros past D, which changes no bit.  Loops stay rolled: this code is
+// cold at each launch, and fetching it takes longer than running it.
+template <int NORM>
+__device__ __forceinline__ void kr_distances(const float* q, const float* __restrict__ rp, int w0,
+                                             int wn, int D, bool vec4, float* st, int w, int lane,
+                                             uint32_t* s_d) {
+  auto step = [](float acc, float a, float b) {
+    const float d = a - b;
+    return NORM == 2 ? knn_acc2(acc, d, false) : knn_acc1(acc, d, false);
+  };
+  const int last = wn - 1;
+  const float* __restrict__ base = rp + (size_t)w0 * D;
+  if (D <= KR_DIRECT) {  // rows of neighbouring lanes share lines: four batches at once
+#pragma unroll 1
+    for (int j0 = 64 * w; j0 < wn; j0 += 4 * KR_THREADS) {
+      float acc[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+      for (int k = 0; k < D; ++k)
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+          acc[u] = step(acc[u], q[k], base[(size_t)min(j0 + u * KR_THREADS + lane, last) * D + k]);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (j0 + u * KR_THREADS + lane < wn) s_d[j0 + u * KR_THREADS + lane] = replay_ord(acc[u]);
+    }
+    return;
+  }
+  // steps: 32 dimensions of a batch; lane l loads 16 bytes (4 words) of row
+  // 8 u + l / 8, or one word of row 2 u + l / 32
+  const int nk = (D + KR_DC - 1) / KR_DC;
+  int lj = 64 * w, lk = 0;  // the next step to load (past the last batch: its last row again)
+  float4 b[8];
+  auto load = [&]() {
+    if (vec4) {
+      const int k = lk * KR_DC + 4 * (lane & 7);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        b[u] = *reinterpret_cast<const float4*>(
+            base + (size_t)min(lj + 8 * u + (lane >> 3), last) * D + min(k, D - 4));
+        if (k >= D) b[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+      }
+    } else {
+      const int k = lk * KR_DC + (lane & 31);
+      auto at = [&](int u) {
+        const float v = base[(size_t)min(lj + 2 * u + (lane >> 5), last) * D + min(k, D - 1)];
+        return k < D ? v : 0.f;
+      };
+#pragma unroll
+      for (int u = 0; u < 8; ++u) b[u] = make_float4(at(4 * u), at(4 * u + 1), at(4 * u + 2), at(4 * u + 3));
+    }
+    if (++lk == nk) {
+      lk = 0;
+      lj += KR_THREADS;
+    }
+  };
+  int j0 = 64 * w, kc = 0;
+  float acc = 0.f;
+  if (j0 < wn) load();
+#pragma unroll 1
+  while (j0 < wn) {
+    if (vec4) {
+#pragma unroll
+      for (int u = 0; u < 8; ++u)
+        *reinterpret_cast<float4*>(st + (8 * u + (lane >> 3)) * KR_DS + 4 * (lane & 7)) = b[u];
+    } else {
+      float* __restrict__ o = st + (lane >> 5) * KR_DS + (lane & 31);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        o[(8 * u + 0) * KR_DS] = b[u].x;
+        o[(8 * u + 2) * KR_DS] = b[u].y;
+        o[(8 * u + 4) * KR_DS] = b[u].z;
+        o[(8 * u + 6) * KR_DS] = b[u].w;
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    load();
+#pragma unroll 2
+    for (int k = 0; k < KR_DC; k += 4) {
+      const float4 r = *reinterpret_cast<const float4*>(st + lane * KR_DS + k);
+      const float4 a = *reinterpret_cast<const float4*>(q + kc * KR_DC + k);
+      acc = step(step(step(step(acc, a.x, r.x), a.y, r.y), a.z, r.z), a.w, r.w);
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    if (++kc == nk) {
+      if (j0 + lane < wn) s_d[j0 + lane] = replay_ord(acc);
+      kc = 0;
+      acc = 0.f;
+      j0 += KR_THREADS;
+    }
+  }
+}
+
+template <int NORM, bool SORT>
+__global__ __launch_bounds__(KR_THREADS) void knn_redo_kernel(
+    const float* __restrict__ p1, const float* __restrict__ p2, const int64_t* __restrict__ len2,
+    int P1, int P2, int D, int K, int pad_sentinel, bool vec4, RedoList list,
+    int64_t* __restrict__ idxs, float* __restrict__ dists) {
+  __shared__ __align__(16) uint32_t s_d[KR_LDS];  // distances, then the waves' staged rows
+  __shared__ __align__(16) float s_q[128 + KR_DC];
+  const uint32_t total = *list.total;
+  if (total == 0 || total > REDO_LIMIT) return;
+  const int tid = threadIdx.x, lane = tid & 63, w = wave_id();
+  float* st = reinterpret_cast<float*>(s_d + KR_WIN) + w * 64 * KR_DS;
+  const int win = D <= KR_DIRECT ? KR_WIN_DIRECT : KR_WIN;
+  for (uint32_t r = blockIdx.x; r < total; r += gridDim.x) {
+    const size_t row = list.rows[r];
+    const int n = (int)(row / (uint32_t)P1);
+    int64_t l2 = len2[n];
+    l2 = l2 < 0 ? 0 : (l2 > P2 ? P2 : l2);
+    const int L2 = (int)l2, fill = min(L2, K);
+    const float* __restrict__ rp = p2 + (size_t)n * P2 * D;
+    for (int d = tid; d < 128 + KR_DC; d += KR_THREADS) s_q[d] = d < D ? p1[row * D + d] : 0.f;
+    __syncthreads();
+    ReplayRow rr;
+    rr.v = Lim<float>::inf();
+    rr.ix = -1;
+    bool live = false;
+    for (int w0 = 0; w0 < L2; w0 += win) {
+      const int wn = min(win, L2 - w0);
+      kr_distances<NORM>(s_q, rp, w0, wn, D, vec4, st, w, lane, s_d);
+      __syncthreads();
+      if (tid < 64) {
+        int e0 = 0;
+        if (w0 == 0) {  // the fill: K <= 32 references of the first window
+          if (lane < fill) {
+            rr.v = __uint_as_float(s_d[lane] - 1u);
+            rr.ix = lane;
+          }
+          live = L2 > K && rr.begin(K, lane);
+          e0 = fill;
+        }
+        if (live) {
+          uint32_t d = s_d[min(e0 + lane, wn - 1)];
+#pragma unroll 1
+          for (; e0 < wn; e0 += 64) {  // the next batch is read ahead
+            const uint32_t dn = s_d[min(e0 + 64 + lane, wn - 1)];
+            rr.batch<false>(d, w0 + e0, e0 + lane < wn, K);
+            d = dn;
+          }
+        }
+      }
+      __syncthreads();
+    }
+    if (tid < 64) {
+      if (live) rr.end(K, lane);
+      const int64_t pad_i = pad_sentinel ? -1 : 0;
+      int64_t* __restrict__ io = idxs + row * K;
+      float* __restrict__ dout = dists + row * K;
+      if constexpr (SORT) {
+        float d;
+        int x;
+        rr.sort<32>(K, fill, (int)pad_i, lane, d, x);
+        if (lane < K) {
+          io[lane] = (int64_t)x;
+          dout[lane] = lane < fill ? d : 0.f;
+        }
+      } else if (lane < K) {
+        io[lane] = lane < fill ? (int64_t)rr.ix : pad_i;
+        dout[lane] = lane < fill ? rr.v : (pad_sentinel ? Lim<float>::inf() : 0.f);
+      }
+    }
+    __syncthreads();  // s_q before the next row's
+  }
+}
+
+}  // namespace
+
+void launch_knn_redo(const void* p1, const void* p2, const int64_t* l1, const int64_t* l2, int N,
+                     int P1, int P2, int D, int K, int norm, int pad, bool sort, const RedoList& r,
+                     int64_t* idxs, void* dists, hipStream_t s) {
+  (void)l1;
+  const int64_t rows = (int64_t)N * P1;
+  const bool vec4 = D % 4 == 0 && (((uintptr_t)p2) & 15) == 0;
+  const dim3 g((unsigned)(rows < KR_GRID ? rows : KR_GRID)), b(KR_THREADS);
+#define KNN_REDO(NORM, SORT)                                                                  \
+  hipLaunchKernelGGL((knn_redo_kernel<NORM, SORT>), g, b, 0, s, (const float*)p1,             \
+                     (const float*)p2, l2, P1, P2, D, K, pad, vec4, r, idxs, (float*)dists)
+  if (norm == 1) {
+    if (sort) KNN_REDO(1, true);
+    else KNN_REDO(1, false);
+  } else {
+    if (sort) KNN_REDO(2, true);
+    else KNN_REDO(2, false);
+  }
+#undef KNN_REDO
+}
+
+}  // namespace tpo

@@ -1,0 +1,153 @@
+// knn_replay.hpp -- one query row's MinK process by one wave: the K slots
+// as an ordered list in the lanes, insertions in index order from batches of
+// 64 distances, and the row sort of knn_points(return_sorted=True) across
+// the lanes (knn.cu:113-168, mink.cuh:77-121, knn/__init__.py:111-131).
+//
+// The slots live one per lane (lanes 0 .. K-1) as a list ordered by 64-bit
+// keys (value, slot descending), NaN values first: the last lane then holds
+// the slot that first_max picks (the first slot holding the largest value; a
+// NaN never becomes the maximum unless it sits in slot 0, and then the
+// threshold is NaN and nothing is ever inserted).  Inserting (d, j) below the
+// threshold puts it into the last element's slot: the lanes whose key exceeds
+// the new one shift up one lane (DPP wave_shr) and the new entry lands in the
+// gap.  An insertion is a chain of dependent wave-wide steps; the evicted
+// entries simply move on into the lanes past K, which nothing reads.
+#pragma once
+
+#include "knn_common.hpp"
+
+#pragma clang fp contract(off)
+
+namespace tpo {
+
+// A distance (>= +0, +inf or NaN) as an unsigned that orders like it; list
+// entries put NaN (0) below every number, candidates above.
+__device__ __forceinline__ uint32_t replay_ord(float v) { return __float_as_uint(v) + 1u; }
+__device__ __forceinline__ uint32_t replay_shr1(uint32_t x) {  // lane i takes lane i-1 (lane 0: 0)
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x138, 0xF, 0xF, true);
+}
+__device__ __forceinline__ uint32_t replay_lane(uint32_t x, int l) {
+  return (uint32_t)__builtin_amdgcn_readlane((int)x, l);
+}
+
+struct ReplayRow {
+  float v;  // lane s < K: slot s, before begin() and after end()
+  int ix;
+  // between them the ordered list: value, (63 - slot) << 26 | index
+  // (references fewer than 2^26), and the last lane's value
+  uint32_t hi, lo, thr;
+
+  // lanes 0 .. K-1 hold the fill (slot s = reference s); orders them.
+  // Returns false when nothing can ever be inserted (a NaN in slot 0).
+  __device__ __forceinline__ bool begin(int K, int lane) {
+    hi = v != v ? 0u : replay_ord(v);
+    if (replay_lane(hi, 0) == 0u) return false;
+    lo = (uint32_t)(63 - lane) << 26 | (uint32_t)ix;
+    const uint64_t key = (uint64_t)hi << 32 | lo;
+    int rank = 0;
+#pragma unroll 1
+    for (int t = 0; t < K; ++t) {
+      const uint64_t kt = (uint64_t)replay_lane(hi, t) << 32 | replay_lane(lo, t);
+      rank += kt < key ? 1 : 0;
+    }
+    const int to = 4 * (lane < K ? rank : lane);
+    hi = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)hi);
+    lo = (uint32_t)__builtin_amdgcn_ds_permute(to, (int)lo);
+    thr = replay_lane(hi, K - 1);
+    return true;
+  }
+  // 64 candidates in index order, lane l holding reference ji (BY_LANE) or
+  // ji + l (a wave-uniform ji) at the ordered distance o; ok: the lane has one
+  template <bool BY_LANE>
+  __device__ __forceinline__ void batch(uint32_t o, int ji, bool ok, int K) {
+    o = ok ? o : 0xffffffffu;
+    uint64_t m = __ballot(o < thr);
+    while (m != 0) {
+      const int e = __builtin_ctzll(m);
+      const uint32_t j = BY_LANE ? replay_lane((uint32_t)ji, e) : (uint32_t)(ji + e);
+      const uint32_t nhi = replay_lane(o, e);
+      const uint32_t nlo = (replay_lane(lo, K - 1) & ~0x3ffffffu) | j;
+      const uint32_t phi = replay_shr1(hi), plo = replay_shr1(lo);
+      const uint64_t nk = (uint64_t)nhi << 32 | nlo;
+      const bool gt = ((uint64_t)hi << 32 | lo) > nk, gtp = ((uint64_t)phi << 32 | plo) > nk;
+      hi = gtp ? phi : (gt ? nhi : hi);
+      lo = gtp ? plo : (gt ? nlo : lo);
+      thr = replay_lane(hi, K - 1);
+      m &= __ballot(o < thr) & ~((2ull << e) - 1ull);
+    }
+  }
+  // back to slot order: lane s takes slot s
+  __device__ __forceinline__ void end(int K, int lane) {
+    const int back = 4 * (lane < K ? (int)(63 - (lo >> 26)) : lane);
+    const uint32_t h = (uint32_t)__builtin_amdgcn_ds_permute(back, (int)hi);
+    v = h ? __uint_as_float(h - 1u) : __builtin_nanf("");
+    ix = __builtin_amdgcn_ds_permute(back, (int)lo) & 0x3ffffff;
+  }
+  // knn_sort_row's network with position p in lane p: an exchange of
+  // positions (a, a + stride) runs in both lanes, which agree on it.  Slots
+  // past `size` key as +inf with index pad_i.
+  template <int KC>
+  __device__ __forceinline__ void sort(int K, int size, int pad_i, int lane, float& d, int& x) const {
+    d = lane < size ? v : Lim<float>::inf();
+    x = lane < size ? ix : pad_i;
+    int va = lane < K ? 1 : 0;
+    auto cas = [&](int stride, bool up) {
+      const float pd = __shfl_xor(d, stride);
+      const int px = __shfl_xor(x, stride), pv = __shfl_xor(va, stride);
+      const bool lo = (lane & stride) == 0;
+      const float da = lo ? d : pd, db = lo ? pd : d;
+      const bool vA = (lo ? va : pv) != 0, vB = (lo ? pv : va) != 0;
+      const bool lt = !knn_isnan(da) && (knn_isnan(db) || da < db);
+      const bool sw = ((lt && vA) || !vB) == up;
+      if ((lane | stride) < KC && sw) {
+        d = pd;
+        x = px;
+        va = pv;
+      }
+    };
+    // loops, as everywhere here: a row runs this once, and code that is not in
+    // the instruction cache costs more than the steps themselves
+#pragma unroll 1
+    for (int sz = 2; sz <= 32; sz *= 2)
+#pragma unroll 1
+      for (int stride = sz / 2; stride > 0; stride /= 2) cas(stride, sz < 32 && (lane & sz) != 0);
+  }
+};
+
+// Rows whose order the distances alone do not decide (equal distances, or
+// values that are not finite): a total count, the rows as n P1 + q in the
+// order of arrival, and per cloud a count and the query numbers.  Up to
+// REDO_LIMIT rows are replayed one a workgroup (launch_knn_redo); more go to
+// the lane-a-row kernel, cloud by cloud.
+constexpr int REDO_LIMIT = 2048;
+
+struct RedoList {
+  uint32_t* total;  // [1], then counts[N]
+  uint32_t* rows;   // [N P1]
+  int32_t* queries; // [N P1], cloud n's from n P1
+};
+__device__ __forceinline__ void redo_push(const RedoList& r, int n, int P1, int q) {
+  const uint32_t a = atomicAdd(r.total, 1u);
+  r.rows[a] = (uint32_t)n * (uint32_t)P1 + (uint32_t)q;
+  const uint32_t b = atomicAdd(r.total + 1 + n, 1u);
+  r.queries[(size_t)n * P1 + b] = q;
+}
+inline int64_t redo_bytes(int64_t N, int64_t P1) {
+  auto up = [](int64_t x) { return (x + 255) / 256 * 256; };
+  return up((N + 1) * 4) + 2 * up(N * P1 * 4);
+}
+inline RedoList redo_at(void* ws, int64_t N, int64_t P1) {
+  auto up = [](int64_t x) { return (x + 255) / 256 * 256; };
+  RedoList r;
+  r.total = (uint32_t*)ws;
+  r.rows = (uint32_t*)((char*)ws + up((N + 1) * 4));
+  r.queries = (int32_t*)((char*)r.rows + up(N * P1 * 4));
+  return r;
+}
+
+// knn_redo.hip: the listed rows' MinK process (float), a workgroup a row
+void launch_knn_redo(const void* p1, const void* p2, const int64_t* l1, const int64_t* l2, int N,
+                     int P1, int P2, int D, int K, int norm, int pad, bool sort, const RedoList& r,
+                     int64_t* idxs, void* dists, hipStream_t s);
+
+}  // namespace tpo
