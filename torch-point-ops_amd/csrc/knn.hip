@@ -46,6 +46,12 @@ int64_t knn_feat_workspace(int64_t N, int64_t P1, int64_t P2, int64_t D);
 RedoList launch_knn_feat(const void* p1, const void* p2, const int64_t* l1, const int64_t* l2,
                          int N, int P1, int P2, int D, int K, int pad, bool sort, int64_t* idxs,
                          void* dists, void* ws, hipStream_t s);
+// knn_near.hip
+bool knn_near_applies(int dtype, int64_t N, int64_t P1, int64_t P2, int64_t D, int64_t K);
+int64_t knn_near_workspace(int64_t N, int64_t P1, int64_t P2);
+RedoList launch_knn_near(const void* p1, const void* p2, const int64_t* l1, const int64_t* l2,
+                         int N, int P1, int P2, int K, int norm, int pad, bool sort,
+                         bool grid_redo, int64_t* idxs, void* dists, void* ws, hipStream_t s);
 // knn_grid.hip
 bool knn_grid_applies(int dtype, int64_t D, int64_t K, int64_t P2);
 int64_t knn_grid_workspace(int64_t N, int64_t P2);
@@ -509,7 +515,8 @@ extern "C" int64_t tpo_knn_workspace_size(int dtype, int64_t N, int64_t P1, int6
   const int64_t hd = S > 0 ? hd_workspace_bytes(N * P1, S, K) : 0;
   const int64_t feat =
       knn_feat_applies(dtype, N, P1, P2, D, K, norm) ? knn_feat_workspace(N, P1, P2, D) : 0;
-  return std::max(order, std::max(hd, feat));
+  const int64_t near = knn_near_applies(dtype, N, P1, P2, D, K) ? knn_near_workspace(N, P1, P2) : 0;
+  return std::max(std::max(order, near), std::max(hd, feat));
 }
 
 static int knn_fwd_impl(int dtype, const void* p1, const void* p2, const int64_t* lengths1,
@@ -557,6 +564,18 @@ static int knn_fwd_impl(int dtype, const void* p1, const void* p2, const int64_t
                     sort_rows, r, idxs, dists, s);
     launch_fwd<float>(p1, p2, lengths1, lengths2, r.queries, (int)N, (int)P1, (int)P2, (int)D,
                       (int)K, norm, pad, sorted2, r.total, idxs, dists, s);
+    return check_launch("tpo_knn_fwd");
+  }
+  // rows by distance, three dimensions: a cell grid
+  if ((sort_rows || K == 1) && !(sorted2 & 1) && workspace &&
+      knn_near_applies(dtype, N, P1, P2, D, K) && workspace_bytes >= knn_near_workspace(N, P1, P2)) {
+    const bool grid_redo = sort_rows && knn_grid_applies(dtype, D, K, P2);
+    const RedoList r =
+        launch_knn_near(p1, p2, lengths1, lengths2, (int)N, (int)P1, (int)P2, (int)K, norm, pad,
+                        sort_rows, grid_redo, idxs, dists, workspace, s);
+    if (!grid_redo)
+      launch_fwd<float>(p1, p2, lengths1, lengths2, r.queries, (int)N, (int)P1, (int)P2, (int)D,
+                        (int)K, norm, pad, sorted2, r.total, idxs, dists, s);
     return check_launch("tpo_knn_fwd");
   }
   {  // long reference clouds, few queries: references sliced over workgroups

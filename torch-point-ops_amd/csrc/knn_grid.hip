@@ -37,7 +37,8 @@
 //      non-finite bound, processes [A, lengths2) by brute force instead.
 #include <utility>
 
-#include "knn_common.hpp"
+#include "knn_cells.hpp"
+#include "knn_replay.hpp"
 
 namespace tpo {
 namespace {
@@ -52,25 +53,6 @@ constexpr int KG_RING = 3;                    // chunks of coordinates in flight
 template <typename F, int... C>
 __device__ __forceinline__ void kg_static_for(F&& f, std::integer_sequence<int, C...>) {
   (f(std::integral_constant<int, C>{}), ...);
-}
-
-// Grid cell along one axis: monotonic non-decreasing in x (a subtraction, a
-// product by gs >= 0, a clamp and a truncation of a non-negative value);
-// NaN lands in cell 0.
-__device__ __forceinline__ int kg_axis(float x, float lo, float gs) {
-  float f = (x - lo) * gs;
-  f = fminf(fmaxf(f, 0.f), (float)(KG_G - 1));
-  return (int)f;
-}
-
-
-// knn.cu:148-158 for D = 3
-template <int NORM>
-__device__ __forceinline__ float kg_dist(const float (&q)[3], float x, float y, float z) {
-  float a = NORM == 2 ? knn_acc2(0.f, q[0] - x, true) : knn_acc1(0.f, q[0] - x, true);
-  a = NORM == 2 ? knn_acc2(a, q[1] - y, false) : knn_acc1(a, q[1] - y, false);
-  a = NORM == 2 ? knn_acc2(a, q[2] - z, false) : knn_acc1(a, q[2] - z, false);
-  return a;
 }
 
 // Points [0, L) of one cloud binned into a 16^3 grid over the bounding box
@@ -160,10 +142,11 @@ __device__ void kg_bin(const float* __restrict__ P, int L, float* __restrict__ h
   if (hdr && tid < 3) {
     hdr[tid] = glo[tid];
     hdr[3 + tid] = gs[tid];
+    if (tid == 0) hdr[6] = __int_as_float(KG_G);
   }
   auto cell_of = [&](float x, float y, float z) -> int {
-    const int ci[3] = {kg_axis(x, glo[0], gs[0]), kg_axis(y, glo[1], gs[1]),
-                       kg_axis(z, glo[2], gs[2])};
+    const int ci[3] = {kg_axis(x, glo[0], gs[0], KG_G), kg_axis(y, glo[1], gs[1], KG_G),
+                       kg_axis(z, glo[2], gs[2], KG_G)};
     if constexpr (HILBERT) {
       return (int)hilbert3_16(ci[0], ci[1], ci[2]);
     } else {
@@ -257,7 +240,7 @@ __global__ __launch_bounds__(1024) void knn_grid_setup_kernel(
     const int n = blockIdx.x - N;
     const int64_t l2 = len2[n];
     const int L2 = (int)(l2 < 0 ? 0 : (l2 > P2 ? P2 : l2));
-    float* h = hdr + (size_t)n * 8;
+    float* h = hdr + (size_t)n * KG_HDR;
     int32_t* cs = cstart + (size_t)n * (KG_CELLS + 1);
     int32_t* ls = list + (size_t)n * P2;
     if (L2 <= 1024 * KG_PPT) kg_bin<false, KG_PPT>(p2 + (size_t)n * P2 * 3, L2, h, cs, ls, sm);
@@ -265,13 +248,18 @@ __global__ __launch_bounds__(1024) void knn_grid_setup_kernel(
   }
 }
 
-template <int NORM, int KC, bool SORT>
+// The grid is knn_grid_setup_kernel's (list), or knn_near_setup_kernel's
+// (REDO: records with the index in w, its own cells an axis); `order` then
+// holds a RedoList's queries, of which there must be over REDO_LIMIT in all.
+template <int NORM, int KC, bool SORT, bool REDO>
 __global__ __launch_bounds__(256) void knn_grid_kernel(
     const float* __restrict__ p1, const float* __restrict__ p2, const int64_t* __restrict__ len1,
     const int64_t* __restrict__ len2, const int32_t* __restrict__ order,
     const float* __restrict__ hdr, const int32_t* __restrict__ cstart,
-    const int32_t* __restrict__ list, int P1, int P2, int K, int A, int nqb, int words,
-    int pad_sentinel, int64_t* __restrict__ idxs, float* __restrict__ dists) {
+    const int32_t* __restrict__ list, int cells_max, const uint32_t* __restrict__ redo, int P1,
+    int P2, int K, int A, int nqb, int words, int pad_sentinel, int64_t* __restrict__ idxs,
+    float* __restrict__ dists) {
+  if (REDO && redo[0] <= REDO_LIMIT) return;
   // LDS per wave: `words` bitmask words, a window of KG_WIN candidate
   // indices, and the current chunk's distances ([entry][lane])
   extern __shared__ uint32_t kg_lds[];
@@ -288,7 +276,7 @@ __global__ __launch_bounds__(256) void knn_grid_kernel(
   const float* __restrict__ rp = p2 + (size_t)n * P2 * 3;
 
   const int i = (blockIdx.x - n * nqb) * 256 + threadIdx.x;  // position in processing order
-  const bool in_range = i < P1;
+  const bool in_range = i < (REDO ? (int)redo[1 + n] : P1);
   const int q = in_range ? order[(size_t)n * P1 + i] : 0;
   const size_t row = (size_t)n * P1 + q;
   int64_t* __restrict__ io = idxs + row * K;
@@ -396,25 +384,24 @@ __global__ __launch_bounds__(256) void knn_grid_kernel(
     run(K, Ae, [](int e) { return e; });
     if (L2 > Ae) {
       // the lane's box: every later insertion is within B of the query per axis
-      const float* __restrict__ h = hdr + (size_t)n * 8;
+      const float* __restrict__ h = hdr + (size_t)n * KG_HDR;
+      const int G = __float_as_int(h[6]);
       int blo[3], bhi[3];
       bool ok = true;
       if (act) {
-        float B;
-        if (NORM == 2) B = __builtin_sqrtf(thr + 0x1p-120f) * (1.f + 0x1p-18f) + 0x1p-60f;
-        else B = thr * (1.f + 0x1p-18f) + 0x1p-100f;
+        const float B = kg_reach<NORM>(thr);
         ok = B < Lim<float>::inf();
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-          const float Bc = B + (__builtin_fabsf(qr[c]) + B) * 0x1p-20f;
+          const float Bc = kg_widen(B, qr[c]);
           ok = ok && __builtin_fabsf(qr[c]) < Lim<float>::inf();
-          blo[c] = kg_axis(qr[c] - Bc, h[c], h[3 + c]);
-          bhi[c] = kg_axis(qr[c] + Bc, h[c], h[3 + c]);
+          blo[c] = kg_axis(qr[c] - Bc, h[c], h[3 + c], G);
+          bhi[c] = kg_axis(qr[c] + Bc, h[c], h[3 + c], G);
         }
       } else {
 #pragma unroll
         for (int c = 0; c < 3; ++c) {
-          blo[c] = KG_G;
+          blo[c] = G;
           bhi[c] = -1;
         }
       }
@@ -438,7 +425,7 @@ __global__ __launch_bounds__(256) void knn_grid_kernel(
         runs_pre[g + 1] = runs_pre[g] + __shfl(rruns, 16 * g, 64);
       }
       const int w0 = Ae >> 5, w1 = (L2 + 31) >> 5;
-      if (__ballot(!ok) != 0 || cells > KG_MAX_BOX) {
+      if (__ballot(!ok) != 0 || cells > KG_MAX_BOX * (REDO ? 8 : 1)) {
         // no useful box: every reference of [Ae, L2) is a candidate
         for (int t = w0 + lane; t < w1; t += 64) {
           const int b0 = max(Ae - 32 * t, 0), b1 = min(L2 - 32 * t, 32);
@@ -451,8 +438,8 @@ __global__ __launch_bounds__(256) void knn_grid_kernel(
         // are consecutive in the list, so each (cx, cy) line of a box is one
         // run; runs are flattened over the lanes, 4 loads a lane at once.
         for (int t = w0 + lane; t < w1; t += 64) bm[t] = 0u;
-        const int32_t* __restrict__ cs = cstart + (size_t)n * (KG_CELLS + 1);
-        const int32_t* __restrict__ ls = list + (size_t)n * P2;
+        const int32_t* __restrict__ cs = cstart + (size_t)n * (cells_max + 1);
+        const int32_t* __restrict__ ls = list + (size_t)n * P2 * (REDO ? 4 : 1) + (REDO ? 3 : 0);
         const int nruns = runs_pre[4];
         int32_t* __restrict__ r_off = cl;      // run offsets (window area as scratch)
         int32_t* __restrict__ r_st = cl + 64;  // run starts in the list
@@ -469,7 +456,7 @@ __global__ __launch_bounds__(256) void knn_grid_kernel(
           int st = 0, ln = 0;
           if (has) {
             const int rl = r - runs_pre[g];
-            const int base = ((gx0 + rl / gny) * KG_G + gy0 + rl % gny) * KG_G;
+            const int base = ((gx0 + rl / gny) * G + gy0 + rl % gny) * G;
             st = cs[base + gz0];
             ln = cs[base + gz1 + 1] - st;
           }
@@ -495,7 +482,7 @@ __global__ __launch_bounds__(256) void knn_grid_kernel(
 #pragma unroll
                 for (int step = 32; step >= 1; step >>= 1)
                   if (r_off[lo + step] <= pp) lo += step;
-                jv[u] = ls[r_st[lo] + pp - r_off[lo]];
+                jv[u] = ls[(size_t)(r_st[lo] + pp - r_off[lo]) * (REDO ? 4 : 1)];
               }
             }
 #pragma unroll
@@ -580,7 +567,7 @@ KgLayout kg_layout(int64_t N, int64_t P2) {
   auto up = [](int64_t x) { return (x + 255) / 256 * 256; };
   KgLayout L;
   L.hdr = 0;
-  L.cstart = up(N * 8 * 4);
+  L.cstart = up(N * KG_HDR * 4);
   L.list = L.cstart + up(N * (KG_CELLS + 1) * 4);
   L.total = L.list + up(N * P2 * 4);
   return L;
@@ -588,28 +575,37 @@ KgLayout kg_layout(int64_t N, int64_t P2) {
 
 int kg_words(int64_t P2) { return (int)(((P2 + 31) / 32 + 63) / 64 * 64); }
 
-template <int NORM, int KC, bool SORT>
-void kg_launch(const void* p1, const void* p2, const int64_t* l1, const int64_t* l2,
-               const int32_t* order, const float* hdr, const int32_t* cs, const int32_t* ls,
-               int N, int P1, int P2, int K, int A, int pad, int64_t* idxs, void* dists,
-               hipStream_t s) {
-  const int nqb = (P1 + 255) / 256;
-  const int words = kg_words(P2);
+struct KgArgs {
+  const void *p1, *p2;
+  const int64_t *l1, *l2;
+  const int32_t* order;
+  const float* hdr;
+  const int32_t *cs, *ls;
+  int cells_max;
+  const uint32_t* redo;
+  int N, P1, P2, K, A, pad;
+  int64_t* idxs;
+  void* dists;
+  hipStream_t s;
+};
+
+template <int NORM, int KC, bool SORT, bool REDO>
+void kg_launch(const KgArgs& a) {
+  const int nqb = (a.P1 + 255) / 256;
+  const int words = kg_words(a.P2);
   const size_t lds = (size_t)KG_WAVES * (words + KG_WIN + KNN_CHUNK * 64) * 4;
-  hipLaunchKernelGGL((knn_grid_kernel<NORM, KC, SORT>), dim3(N * nqb), dim3(256), lds, s,
-                     (const float*)p1, (const float*)p2, l1, l2, order, hdr, cs, ls, P1, P2, K, A,
-                     nqb, words, pad, idxs, (float*)dists);
+  hipLaunchKernelGGL((knn_grid_kernel<NORM, KC, SORT, REDO>), dim3(a.N * nqb), dim3(256), lds, a.s,
+                     (const float*)a.p1, (const float*)a.p2, a.l1, a.l2, a.order, a.hdr, a.cs, a.ls,
+                     a.cells_max, a.redo, a.P1, a.P2, a.K, a.A, nqb, words, a.pad, a.idxs,
+                     (float*)a.dists);
 }
 
-template <int NORM, bool SORT>
-void kg_launch_k(const void* p1, const void* p2, const int64_t* l1, const int64_t* l2,
-                 const int32_t* order, const float* hdr, const int32_t* cs, const int32_t* ls,
-                 int N, int P1, int P2, int K, int A, int pad, int64_t* idxs, void* dists,
-                 hipStream_t s) {
-  if (K <= 4) kg_launch<NORM, 4, SORT>(p1, p2, l1, l2, order, hdr, cs, ls, N, P1, P2, K, A, pad, idxs, dists, s);
-  else if (K <= 8) kg_launch<NORM, 8, SORT>(p1, p2, l1, l2, order, hdr, cs, ls, N, P1, P2, K, A, pad, idxs, dists, s);
-  else if (K <= 16) kg_launch<NORM, 16, SORT>(p1, p2, l1, l2, order, hdr, cs, ls, N, P1, P2, K, A, pad, idxs, dists, s);
-  else kg_launch<NORM, 32, SORT>(p1, p2, l1, l2, order, hdr, cs, ls, N, P1, P2, K, A, pad, idxs, dists, s);
+template <int NORM, bool SORT, bool REDO>
+void kg_launch_k(const KgArgs& a) {
+  if (a.K <= 4) kg_launch<NORM, 4, SORT, REDO>(a);
+  else if (a.K <= 8) kg_launch<NORM, 8, SORT, REDO>(a);
+  else if (a.K <= 16) kg_launch<NORM, 16, SORT, REDO>(a);
+  else kg_launch<NORM, 32, SORT, REDO>(a);
 }
 
 }  // namespace
@@ -623,6 +619,11 @@ bool knn_grid_applies(int dtype, int64_t D, int64_t K, int64_t P2) {
   return dtype == TPO_F32 && D == 3 && K >= 1 && K <= 32 && P2 >= KG_MIN_P2 && P2 <= KG_MAX_P2;
 }
 
+static int kg_prefix(int K, int P2) {
+  const int A = (int)std::sqrt(4.0 * K * (double)P2);
+  return std::max(std::max(KG_PREFIX_MIN, std::min(KG_PREFIX_MAX, A)), K);
+}
+
 int64_t knn_grid_workspace(int64_t N, int64_t P2) { return kg_layout(N, P2).total; }
 
 void launch_knn_grid(const void* p1, const void* p2, const int64_t* l1, const int64_t* l2,
@@ -634,16 +635,25 @@ void launch_knn_grid(const void* p1, const void* p2, const int64_t* l1, const in
   int32_t* ls = (int32_t*)((char*)ws + L.list);
   hipLaunchKernelGGL(knn_grid_setup_kernel, dim3(2 * N), dim3(1024), 0, s, (const float*)p1, l1,
                      P1, order, (const float*)p2, l2, P2, N, hdr, cs, ls);
-  int A = (int)std::sqrt(4.0 * K * (double)P2);
-  A = std::max(KG_PREFIX_MIN, std::min(KG_PREFIX_MAX, A));
-  A = std::max(A, K);
+  KgArgs a{p1, p2, l1, l2, order, hdr, cs, ls, KG_CELLS, nullptr, N, P1, P2, K,
+           kg_prefix(K, P2), pad, idxs, dists, s};
   if (norm == 1) {
-    if (sort) kg_launch_k<1, true>(p1, p2, l1, l2, order, hdr, cs, ls, N, P1, P2, K, A, pad, idxs, dists, s);
-    else kg_launch_k<1, false>(p1, p2, l1, l2, order, hdr, cs, ls, N, P1, P2, K, A, pad, idxs, dists, s);
+    if (sort) kg_launch_k<1, true, false>(a);
+    else kg_launch_k<1, false, false>(a);
   } else {
-    if (sort) kg_launch_k<2, true>(p1, p2, l1, l2, order, hdr, cs, ls, N, P1, P2, K, A, pad, idxs, dists, s);
-    else kg_launch_k<2, false>(p1, p2, l1, l2, order, hdr, cs, ls, N, P1, P2, K, A, pad, idxs, dists, s);
+    if (sort) kg_launch_k<2, true, false>(a);
+    else kg_launch_k<2, false, false>(a);
   }
+}
+
+void launch_knn_grid_redo(const void* p1, const void* p2, const int64_t* l1, const int64_t* l2,
+                          int N, int P1, int P2, int K, int norm, int pad, const float* hdr,
+                          const int32_t* cs, int cells_max, const float* records, const RedoList& r,
+                          int64_t* idxs, void* dists, hipStream_t s) {
+  KgArgs a{p1, p2, l1, l2, r.queries, hdr, cs, (const int32_t*)records, cells_max, r.total, N, P1,
+           P2, K, kg_prefix(K, P2), pad, idxs, dists, s};
+  if (norm == 1) kg_launch_k<1, true, true>(a);
+  else kg_launch_k<2, true, true>(a);
 }
 
 }  // namespace tpo
