@@ -44,6 +44,26 @@ def test_fps_degenerate_and_ties(tpo, O, dev):
     assert (np_(tpo.furthest_point_sampling(cases[0].to(dev), 8)) == 0).all()
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("N", [2, 511, 512, 513, 1024, 1025, 2047, 2048, 2049, 3072, 3073, 4096, 6144,
+                               6145, 8191, 8192, 8193])
+def test_fps_held_sizes_vs_oracle(tpo, O, dev, dtype, N):
+    """Both sides of each register count of the kernel that holds a cloud, and
+    of its limit: a random cloud, one with many equal distances, one with
+    points that do not take part and values that are not finite."""
+    g = torch.Generator().manual_seed(N)
+    a = torch.randn(1, N, 3, generator=g)
+    b = torch.randint(-3, 4, (1, N, 3), generator=g).float() * 0.5
+    c = torch.randn(1, N, 3, generator=g)
+    c[0, N // 3:2 * N // 3] *= 1e-3
+    c[0, N // 2, 1] = float("nan")
+    c[0, N // 4, 2] = float("inf")
+    pts = torch.cat([a, b, c]).to(dtype)
+    m = min(N, 150)
+    got = tpo.furthest_point_sampling(pts.to(dev), m)
+    assert np.array_equal(np_(got), O.fps(np_(pts), m))
+
+
 def test_fps_large_n_bucket_path(tpo, O, dev):
     """N > 65536 uses buckets of more than 64 points."""
     g = torch.Generator().manual_seed(4)

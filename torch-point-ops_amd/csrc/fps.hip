@@ -213,6 +213,22 @@ __device__ __forceinline__ half_t bcast(half_t v, int lane) {
 }
 
 
+// out[1, m): rank -> point index, rank = bitrev(k mod BS) * per + k / BS
+// (-1: no point took part, index 0)
+__device__ __forceinline__ void fps_decode(int64_t* __restrict__ out, int m, int tid, int threads,
+                                           int bs, int bs_bits, int per) {
+  for (int j = 1 + tid; j < m; j += threads) {
+    const int64_t r = out[j];
+    int64_t k = 0;
+    if (r >= 0) {
+      const uint32_t q = (uint32_t)r / (uint32_t)per, rem = (uint32_t)r - q * (uint32_t)per;
+      const uint32_t tq = bs_bits ? (__builtin_bitreverse32(q) >> (32 - bs_bits)) : 0u;
+      k = (int64_t)tq + (int64_t)rem * bs;
+    }
+    out[j] = k;
+  }
+}
+
 template <typename T>
 __global__ __launch_bounds__(FPS_THREADS) void fps_kernel(const T* __restrict__ pts, int N, int m,
                                                           int bs, int bs_bits, int per,
@@ -540,18 +556,127 @@ __global__ __launch_bounds__(FPS_THREADS) void fps_kernel(const T* __restrict__ 
       }
     }
   }
-  // rank -> point index: rank = bitrev(k mod BS) * per + k / BS
   __syncthreads();
-  for (int j = 1 + tid; j < m; j += FPS_THREADS) {
-    const int64_t r = out[j];
-    int64_t k = 0;
-    if (r >= 0) {
-      const uint32_t q = (uint32_t)r / (uint32_t)per, rem = (uint32_t)r - q * (uint32_t)per;
-      const uint32_t tq = bs_bits ? (__builtin_bitreverse32(q) >> (32 - bs_bits)) : 0u;
-      k = (int64_t)tq + (int64_t)rem * bs;
-    }
-    out[j] = k;
+  fps_decode(out, m, tid, FPS_THREADS, bs, bs_bits, per);
+}
+
+// min(d, t) as fps.cu:146 takes it for a t that is never NaN: a NaN d leaves t
+__device__ __forceinline__ float fps_min(float d, float t) { return fminf(d, t); }
+__device__ __forceinline__ half_t fps_min(half_t d, half_t t) { return __builtin_fminf16(d, t); }
+
+// Clouds of at most 64 W PPT points, float or half: the whole cloud in the
+// registers of one workgroup, every point updated for every sample (no sort,
+// no buckets, no workspace).  A sample is a chain: PPT distances a lane, the
+// wave's best value by DPP and the lowest rank at it, one LDS atomicMax, one
+// barrier, and the winner's coordinates from an LDS table by rank.  The chain
+// alone takes about 0.43 us a sample (PPT = 2), a point a lane and wave adds
+// 0.02-0.04 us.  W: 16 clouds of 2048 points take 0.46 us a sample with 8
+// waves, 0.52 with 4, 0.51 with 16 (the bucket kernel 1.08); of 1024 0.44 with
+// 4, 0.48 with 8; of 8192 0.80 with 8, 1.13 with 4 (the bucket kernel 1.05).
+template <typename T, int W, int PPT>
+__global__ __launch_bounds__(64 * W) void fps_held_kernel(const T* __restrict__ pts, int N, int m,
+                                                          int bs, int bs_bits, int per,
+                                                          int64_t* __restrict__ idx_out) {
+  constexpr int TH = 64 * W;
+  __shared__ float4 s_at[TH * PPT + 512];  // coordinates by rank (ranks below N + 511)
+  __shared__ unsigned long long s_best[3];
+  const int b = blockIdx.x, tid = threadIdx.x, lane = lane_id(), w = wave_id();
+  const T* __restrict__ P = pts + (size_t)b * N * 3;
+  int64_t* __restrict__ out = idx_out + (size_t)b * m;
+  const T thr = FpsConst<T>::thr(), init = FpsConst<T>::init();
+  const T p0x = P[0], p0y = P[1], p0z = P[2];
+  T x[PPT], y[PPT], z[PPT], t[PPT];
+  uint32_t key[PPT];
+#pragma unroll
+  for (int u = 0; u < PPT; ++u) {
+    const int k = tid + TH * u, kc = min(k, N - 1);
+    x[u] = P[3 * kc];
+    y[u] = P[3 * kc + 1];
+    z[u] = P[3 * kc + 2];
   }
+#pragma unroll
+  for (int u = 0; u < PPT; ++u) {
+    const int k = tid + TH * u;
+    const bool valid = k < N && sq3(x[u], y[u], z[u]) > thr;  // fps.cu:142-143
+    const uint32_t tb = (uint32_t)(k & (bs - 1));
+    const uint32_t rev = bs_bits ? (__builtin_bitreverse32(tb) >> (32 - bs_bits)) : 0u;
+    const uint32_t rank = rev * (uint32_t)per + (uint32_t)(k >> bs_bits);
+    key[u] = valid ? ~rank : 0u;
+    if (k < N) s_at[rank] = make_float4((float)x[u], (float)y[u], (float)z[u], 0.f);
+    // the first sample (index 0)
+    const T d = sq3((T)(x[u] - p0x), (T)(y[u] - p0y), (T)(z[u] - p0z));  // fps.cu:145
+    t[u] = valid ? (d < init ? d : init) : (T)0;                         // fps.cu:146
+  }
+  if (tid < 3) s_best[tid] = 0;
+  if (tid == 0) out[0] = 0;
+  __syncthreads();
+  int rk = 0;  // wave 0: lane j mod 64 holds the rank of sample j
+  for (int j = 1; j < m; ++j) {
+    // running minima are >= +0 (a NaN distance never replaces one), so their
+    // float bits order like them
+    float mv = (float)t[0];
+#pragma unroll
+    for (int u = 1; u < PPT; ++u) mv = fmaxf(mv, (float)t[u]);
+    const uint32_t mh = wave_umax(__float_as_uint(mv));
+    uint32_t lk = 0;
+#pragma unroll
+    for (int u = 0; u < PPT; ++u) {
+      const uint32_t c = __float_as_uint((float)t[u]) == mh ? key[u] : 0u;
+      lk = c > lk ? c : lk;
+    }
+    const uint64_t has = __ballot(lk != 0u);
+    uint32_t bk;
+    if (__builtin_popcountll(has) <= 1)
+      bk = (uint32_t)__builtin_amdgcn_readlane((int)lk, has ? __builtin_ctzll(has) : 0);
+    else
+      bk = wave_umax(lk);
+    // three slots in turn: the next one is cleared before this barrier, after
+    // its last readers (before the previous one)
+    if (tid == 0) s_best[(j + 1) % 3] = 0;
+    if (lane == 0 && bk != 0u)
+      atomicMax(&s_best[j % 3], (unsigned long long)mh << 32 | (unsigned long long)bk);
+    __syncthreads();
+    const uint32_t g = (uint32_t)s_best[j % 3];
+    // nothing takes part: index 0 (rank -1 here)
+    const float4 at = s_at[g ? ~g : 0u];
+    const int r = g ? (int)~g : -1;
+    const T ox = g ? (T)at.x : p0x, oy = g ? (T)at.y : p0y, oz = g ? (T)at.z : p0z;
+    if (w == 0) {
+      rk = lane == (j & 63) ? r : rk;
+      if ((j & 63) == 63 || j == m - 1) {
+        const int jj = (j & ~63) + lane;
+        if (jj >= 1 && jj <= j) out[jj] = (int64_t)rk;
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < PPT; ++u) {
+      const T d = sq3((T)(x[u] - ox), (T)(y[u] - oy), (T)(z[u] - oz));
+      t[u] = fps_min(d, t[u]);
+    }
+  }
+  __syncthreads();
+  fps_decode(out, m, tid, TH, bs, bs_bits, per);
+}
+
+// The held kernel's limit: the coordinate table's LDS (139 KB at 8192).
+constexpr int FPS_HELD_MAX = 8192;
+
+template <typename T>
+bool launch_held(const void* points, int64_t B, int N, int m, int bs, int bits, int per,
+                 int64_t* idx, hipStream_t s) {
+  if (N > FPS_HELD_MAX) return false;
+#define FPS_HELD(W, PPT)                                                                        \
+  hipLaunchKernelGGL((fps_held_kernel<T, W, PPT>), dim3((unsigned)B), dim3(64 * W), 0, s,       \
+                     (const T*)points, N, m, bs, bits, per, idx)
+  if (N <= 512) FPS_HELD(4, 2);
+  else if (N <= 1024) FPS_HELD(4, 4);
+  else if (N <= 2048) FPS_HELD(8, 4);
+  else if (N <= 3072) FPS_HELD(8, 6);
+  else if (N <= 4096) FPS_HELD(8, 8);
+  else if (N <= 6144) FPS_HELD(8, 12);
+  else FPS_HELD(8, 16);
+#undef FPS_HELD
+  return true;
 }
 
 }  // namespace
@@ -590,6 +715,9 @@ extern "C" int tpo_fps_fwd(int dtype, const void* points, int64_t B, int64_t N, 
   }
   const int per = (int)((N + bs - 1) / bs);
   hipStream_t s = (hipStream_t)stream;
+  if ((dtype == TPO_F32 && launch_held<float>(points, B, (int)N, (int)nsamples, bs, bits, per, idx, s)) ||
+      (dtype == TPO_F16 && launch_held<half_t>(points, B, (int)N, (int)nsamples, bs, bits, per, idx, s)))
+    return check_launch("tpo_fps_fwd");
   switch (dtype) {
     case TPO_F32:
       hipLaunchKernelGGL(fps_kernel<float>, dim3((unsigned)B), dim3(FPS_THREADS), 0, s,
