@@ -198,6 +198,15 @@ int tpo_knn_fwd_sorted(int dtype, const void* p1, const void* p2,
                        void* stream);
 
 /*
+ * Bytes of workspace with which tpo_knn_fwd_sorted, and tpo_knn_fwd with
+ * K = 1, select rows by distance (float: cell grid for D = 3, matrix cores for
+ * D = 4 .. 128 with norm 2).  At least tpo_knn_workspace_size, with which the
+ * same rows come from the insertion-order kernels.
+ */
+int64_t tpo_knn_rows_workspace_size(int dtype, int64_t N, int64_t P1, int64_t P2, int64_t D,
+                                    int64_t K, int norm);
+
+/*
  * knn_gather forward.  Replaces the expand + gather + mask of
  * knn_gather (torch_point_ops/knn/__init__.py:136-183), which the reference
  * runs as torch ops.

@@ -513,10 +513,17 @@ extern "C" int64_t tpo_knn_workspace_size(int dtype, int64_t N, int64_t P1, int6
   if (knn_grid_applies(dtype, D, K, P2)) order += knn_grid_workspace(N, P2);
   const int S = hd_slices(dtype, N, P1, P2, D, K);
   const int64_t hd = S > 0 ? hd_workspace_bytes(N * P1, S, K) : 0;
-  const int64_t feat =
-      knn_feat_applies(dtype, N, P1, P2, D, K, norm) ? knn_feat_workspace(N, P1, P2, D) : 0;
+  return order > hd ? order : hd;
+}
+
+extern "C" int64_t tpo_knn_rows_workspace_size(int dtype, int64_t N, int64_t P1, int64_t P2,
+                                               int64_t D, int64_t K, int norm) {
+  const int64_t base = tpo_knn_workspace_size(dtype, N, P1, P2, D, K, norm);
+  if (base < 0) return base;
+  const int64_t feat = D != 3 && knn_feat_applies(dtype, N, P1, P2, D, K, norm)
+                           ? knn_feat_workspace(N, P1, P2, D) : 0;
   const int64_t near = knn_near_applies(dtype, N, P1, P2, D, K) ? knn_near_workspace(N, P1, P2) : 0;
-  return std::max(std::max(order, near), std::max(hd, feat));
+  return std::max(base, std::max(near, feat));
 }
 
 static int knn_fwd_impl(int dtype, const void* p1, const void* p2, const int64_t* lengths1,

@@ -271,7 +271,8 @@ std::tuple<at::Tensor, at::Tensor> knn_forward_hip(const at::Tensor& p1_in,
   }
   const at::Tensor p1 = p1_in.contiguous(), p2 = p2_in.contiguous();
   const int dt = dtype_code(p1, "knn_forward");
-  const int64_t ws = tpo_knn_workspace_size(dt, N, P1, P2, D, K, (int)norm);
+  const int64_t ws = K == 1 ? tpo_knn_rows_workspace_size(dt, N, P1, P2, D, K, (int)norm)
+                            : tpo_knn_workspace_size(dt, N, P1, P2, D, K, (int)norm);
   at::Tensor work = at::empty({ws > 0 ? ws : 1}, p1.options().dtype(at::kByte));
   check_rc(tpo_knn_fwd(dt, p1.data_ptr(), p2.data_ptr(), l1.data_ptr<int64_t>(),
                        l2.data_ptr<int64_t>(), N, P1, P2, D, K, (int)norm, (int)version,
@@ -313,7 +314,7 @@ std::tuple<at::Tensor, at::Tensor> knn_forward_sorted_hip(const at::Tensor& p1_i
   const at::Tensor l1 = lengths1_in.contiguous(), l2 = lengths2_in.contiguous();
   const at::Tensor p1 = p1_in.contiguous(), p2 = p2_in.contiguous();
   const int dt = dtype_code(p1, "knn_forward_sorted");
-  const int64_t ws = tpo_knn_workspace_size(dt, N, P1, P2, D, K, (int)norm);
+  const int64_t ws = tpo_knn_rows_workspace_size(dt, N, P1, P2, D, K, (int)norm);
   at::Tensor work = at::empty({ws > 0 ? ws : 1}, p1.options().dtype(at::kByte));
   check_rc(tpo_knn_fwd_sorted(dt, p1.data_ptr(), p2.data_ptr(), l1.data_ptr<int64_t>(),
                               l2.data_ptr<int64_t>(), N, P1, P2, D, K, (int)norm, (int)version,
