@@ -446,6 +446,92 @@ std::tuple<at::Tensor, at::Tensor> knn_backward_hip(const at::Tensor& p1_in,
   return {g1, g2};
 }
 
+// Autograd of the KNN operators in C++, as the Chamfer loss's: a step's forward
+// and backward run no Python.  Gradients of outputs that a loss leaves out are
+// not materialised; the index outputs carry none (knn/__init__.py:6-28).
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+template <typename Op>
+auto typed_op(const char* name) {
+  return c10::Dispatcher::singleton().findSchemaOrThrow(name, "").typed<Op>();
+}
+
+template <bool SORTED>
+class KnnFunction : public torch::autograd::Function<KnnFunction<SORTED>> {
+ public:
+  static variable_list forward(AutogradContext* ctx, const at::Tensor& p1, const at::Tensor& p2,
+                               const at::Tensor& lengths1, const at::Tensor& lengths2,
+                               int64_t norm, int64_t K, int64_t version) {
+    static auto op = typed_op<std::tuple<at::Tensor, at::Tensor>(
+        const at::Tensor&, const at::Tensor&, const at::Tensor&, const at::Tensor&, int64_t,
+        int64_t, int64_t)>(SORTED ? "torch_point_ops_knn::knn_forward_sorted"
+                                  : "torch_point_ops_knn::knn_forward");
+    at::Tensor idxs, dists;
+    {
+      at::AutoDispatchBelowADInplaceOrView below;
+      std::tie(idxs, dists) = op.call(p1, p2, lengths1, lengths2, norm, K, version);
+    }
+    ctx->save_for_backward({p1, p2, lengths1, lengths2, idxs});
+    ctx->saved_data["norm"] = norm;
+    ctx->mark_non_differentiable({idxs});
+    ctx->set_materialize_grads(false);
+    return {idxs, dists};
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    static auto op = typed_op<std::tuple<at::Tensor, at::Tensor>(
+        const at::Tensor&, const at::Tensor&, const at::Tensor&, const at::Tensor&,
+        const at::Tensor&, int64_t, const at::Tensor&)>("torch_point_ops_knn::knn_backward");
+    at::Tensor g1, g2, none;
+    if (grads[1].defined()) {
+      const auto s = ctx->get_saved_variables();
+      std::tie(g1, g2) =
+          op.call(s[0], s[1], s[2], s[3], s[4], ctx->saved_data["norm"].toInt(), grads[1]);
+    }
+    return {g1, g2, none, none, none, none, none};
+  }
+};
+
+template <bool SORTED>
+std::tuple<at::Tensor, at::Tensor> knn_forward_autograd(
+    const at::Tensor& p1, const at::Tensor& p2, const at::Tensor& lengths1,
+    const at::Tensor& lengths2, int64_t norm, int64_t K, int64_t version) {
+  auto out = KnnFunction<SORTED>::apply(p1, p2, lengths1, lengths2, norm, K, version);
+  return {out[0], out[1]};
+}
+
+class KnnGatherFunction : public torch::autograd::Function<KnnGatherFunction> {
+ public:
+  static at::Tensor forward(AutogradContext* ctx, const at::Tensor& x, const at::Tensor& idx,
+                            const at::Tensor& lengths) {
+    static auto op = typed_op<at::Tensor(const at::Tensor&, const at::Tensor&, const at::Tensor&)>(
+        "torch_point_ops_knn::knn_gather");
+    ctx->save_for_backward({idx, lengths});
+    ctx->saved_data["M"] = x.sym_size(1).guard_int(__FILE__, __LINE__);
+    ctx->set_materialize_grads(false);
+    at::AutoDispatchBelowADInplaceOrView below;
+    return op.call(x, idx, lengths);
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    static auto op =
+        typed_op<at::Tensor(const at::Tensor&, const at::Tensor&, const at::Tensor&, int64_t)>(
+            "torch_point_ops_knn::knn_gather_backward");
+    if (!grads[0].defined()) return {at::Tensor(), at::Tensor(), at::Tensor()};
+    const auto s = ctx->get_saved_variables();
+    const int64_t M = ctx->saved_data["M"].toInt();
+    if (at::GradMode::is_enabled())  // its own gradient is the gather (knn/__init__.py)
+      return {op.call(grads[0], s[0], s[1], M), at::Tensor(), at::Tensor()};
+    at::AutoDispatchBelowADInplaceOrView below;
+    return {op.call(grads[0], s[0], s[1], M), at::Tensor(), at::Tensor()};
+  }
+};
+
+at::Tensor knn_gather_autograd(const at::Tensor& x, const at::Tensor& idx,
+                               const at::Tensor& lengths) {
+  TORCH_CHECK(x.dim() == 3, "knn_gather expects (N,M,U) and (N,L,K)");
+  return KnnGatherFunction::apply(x, idx, lengths);
+}
+
 // ---------------------------------------------------------------------- fps
 at::Tensor fps_forward_hip(const at::Tensor& points_in, int64_t nsamples) {
   check_hip(points_in, "points");
@@ -522,6 +608,32 @@ at::Tensor gather_points_backward_hip(const at::Tensor& grad_in, const at::Tenso
                           work.data_ptr(), ws, stream_of(go)),
            "gather_points_backward");
   return out;
+}
+
+// gather_points' autograd (fps/__init__.py:8-30) in C++
+class GatherPointsFunction : public torch::autograd::Function<GatherPointsFunction> {
+ public:
+  static at::Tensor forward(AutogradContext* ctx, const at::Tensor& points, const at::Tensor& idx) {
+    static auto op = typed_op<at::Tensor(const at::Tensor&, const at::Tensor&)>(
+        "torch_point_ops_fps::gather_points_forward");
+    ctx->save_for_backward({idx});
+    ctx->saved_data["n"] = points.sym_size(2).guard_int(__FILE__, __LINE__);
+    ctx->set_materialize_grads(false);
+    at::AutoDispatchBelowADInplaceOrView below;
+    return op.call(points, idx);
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    static auto op = typed_op<at::Tensor(const at::Tensor&, const at::Tensor&, int64_t)>(
+        "torch_point_ops_fps::gather_points_backward");
+    if (!grads[0].defined()) return {at::Tensor(), at::Tensor()};
+    const auto s = ctx->get_saved_variables();
+    return {op.call(grads[0], s[0], ctx->saved_data["n"].toInt()), at::Tensor()};
+  }
+};
+
+at::Tensor gather_points_autograd(const at::Tensor& points, const at::Tensor& idx) {
+  TORCH_CHECK(points.dim() == 3, "gather_points expects (N,C,P), (N,M)");
+  return GatherPointsFunction::apply(points, idx);
 }
 
 // ---------------------------------------------------------------------- emd
@@ -640,6 +752,12 @@ TORCH_LIBRARY_IMPL(torch_point_ops_knn, CUDA, m) {
   m.impl("knn_backward", &knn_backward_hip);
 }
 
+TORCH_LIBRARY_IMPL(torch_point_ops_knn, Autograd, m) {
+  m.impl("knn_forward", &knn_forward_autograd<false>);
+  m.impl("knn_forward_sorted", &knn_forward_autograd<true>);
+  m.impl("knn_gather", &knn_gather_autograd);
+}
+
 TORCH_LIBRARY(torch_point_ops_fps, m) {
   m.def("fps_forward(Tensor points, int nsamples) -> Tensor");
   m.def("gather_points_forward(Tensor points, Tensor idx) -> Tensor");
@@ -649,6 +767,10 @@ TORCH_LIBRARY_IMPL(torch_point_ops_fps, CUDA, m) {
   m.impl("fps_forward", &fps_forward_hip);
   m.impl("gather_points_forward", &gather_points_forward_hip);
   m.impl("gather_points_backward", &gather_points_backward_hip);
+}
+
+TORCH_LIBRARY_IMPL(torch_point_ops_fps, Autograd, m) {
+  m.impl("gather_points_forward", &gather_points_autograd);
 }
 
 TORCH_LIBRARY(torch_point_ops_quick_fps, m) {

@@ -12,25 +12,7 @@ import torch
 from .. import _C  # noqa: F401
 
 
-def _gather_points_backward(ctx, grad_output):
-    (idx,) = ctx.saved_tensors
-    grad_points = torch.ops.torch_point_ops_fps.gather_points_backward(
-        grad_output, idx, ctx.n_points
-    )
-    return grad_points, None
-
-
-def _gather_points_setup_context(ctx, inputs, output):
-    points, idx = inputs
-    ctx.save_for_backward(idx)
-    ctx.n_points = points.shape[2]
-
-
-torch.library.register_autograd(
-    "torch_point_ops_fps::gather_points_forward",
-    _gather_points_backward,
-    setup_context=_gather_points_setup_context,
-)
+# gather_points_forward's autograd is registered in C++ (torch_ops.cpp).
 
 
 @torch.library.register_fake("torch_point_ops_fps::fps_forward")

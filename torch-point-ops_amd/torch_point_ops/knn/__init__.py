@@ -9,32 +9,9 @@ import torch
 from .. import _C  # noqa: F401
 
 
-def _knn_backward(ctx, grad_idxs, grad_dists):
-    p1, p2, lengths1, lengths2, idxs = ctx.saved_tensors
-    if grad_dists is None:  # gradients are not materialised: the index output has none
-        return None, None, None, None, None, None, None
-    grad_p1, grad_p2 = torch.ops.torch_point_ops_knn.knn_backward(
-        p1, p2, lengths1, lengths2, idxs, ctx.norm, grad_dists
-    )
-    # no gradient for lengths1, lengths2, norm, K, version
-    return grad_p1, grad_p2, None, None, None, None, None
-
-
-def _knn_setup_context(ctx, inputs, output):
-    p1, p2, lengths1, lengths2, norm, _K, _version = inputs
-    idxs, _dists = output
-    ctx.save_for_backward(p1, p2, lengths1, lengths2, idxs)
-    ctx.norm = norm
-    ctx.set_materialize_grads(False)  # no zero tensor for the index output
-
-
-torch.library.register_autograd(
-    "torch_point_ops_knn::knn_forward", _knn_backward, setup_context=_knn_setup_context
-)
-# the sorted forward's rows are a permutation of knn_forward's: same gradient
-torch.library.register_autograd(
-    "torch_point_ops_knn::knn_forward_sorted", _knn_backward, setup_context=_knn_setup_context
-)
+# The autograd of knn_forward, knn_forward_sorted (its rows are a permutation
+# of knn_forward's: same gradient) and knn_gather is registered in C++
+# (torch_ops.cpp): a training step runs no Python for them.
 
 
 @torch.library.register_fake("torch_point_ops_knn::knn_forward")
@@ -53,26 +30,6 @@ def _knn_forward_sorted_fake(p1, p2, lengths1, lengths2, norm, K, version):
 
 # dtypes whose sorted rows come straight from the kernel (2 <= K <= 32)
 _SORTED_IN_KERNEL = (torch.float32, torch.float64, torch.float16)
-
-
-def _knn_gather_backward(ctx, grad_out):
-    # gather's gradient: the rows added back (the masked slots carry none)
-    idx, lengths = ctx.saved_tensors
-    if grad_out is None or not ctx.needs_input_grad[0]:
-        return None, None, None
-    return torch.ops.torch_point_ops_knn.knn_gather_backward(grad_out, idx, lengths, ctx.M), None, None
-
-
-def _knn_gather_setup_context(ctx, inputs, output):
-    x, idx, lengths = inputs
-    ctx.save_for_backward(idx, lengths)
-    ctx.M = x.shape[1]
-
-
-torch.library.register_autograd(
-    "torch_point_ops_knn::knn_gather", _knn_gather_backward,
-    setup_context=_knn_gather_setup_context,
-)
 
 
 def _knn_gather_backward_backward(ctx, grad_grad_x):
