@@ -198,6 +198,13 @@ int tpo_knn_fwd_sorted(int dtype, const void* p1, const void* p2,
                        void* stream);
 
 /*
+ * Sorts the rows (N,P1,K) of a BF16 tpo_knn_fwd in place, K <= 32, as
+ * tpo_knn_fwd_sorted sorts the other types' rows.
+ */
+int tpo_knn_sort_rows(int dtype, const int64_t* lengths2, int64_t N, int64_t P1, int64_t K,
+                      int64_t* idxs, void* dists, void* stream);
+
+/*
  * Bytes of workspace with which tpo_knn_fwd_sorted, and tpo_knn_fwd with
  * K = 1, select rows by distance (float: cell grid for D = 3, matrix cores for
  * D = 4 .. 128 with norm 2).  At least tpo_knn_workspace_size, with which the

@@ -903,3 +903,21 @@ def test_bf16_knn_points_and_fallbacks(tpo, dev):
     tpo.knn_points(a, b, K=4)[1].float().sum().backward()
     assert a.grad.dtype == torch.bfloat16 and torch.isfinite(a.grad.float()).all()
     assert torch.isfinite(b.grad.float()).all()
+
+
+@pytest.mark.parametrize("K", [2, 3, 8, 17, 32])
+@pytest.mark.parametrize("D,P2", [(64, 300), (128, 5000), (35, 200), (3, 400)])
+def test_bf16_rows_sorted_in_kernel_match_torch_sort(tpo, dev, K, D, P2):
+    """Distances rounded to bfloat16 tie often: rows must come out as torch's
+    sort of the forward's rows leaves them, padding included (widths of the
+    matrix-core kernel and of the widened float kernels)."""
+    g = torch.Generator().manual_seed(K + D)
+    p1 = torch.randn(3, 77, D, generator=g).to(dev, torch.bfloat16)
+    p2 = torch.randn(3, P2, D, generator=g).to(dev, torch.bfloat16)
+    l1 = torch.tensor([77, 20, 77], device=dev)
+    l2 = torch.tensor([P2, P2 - 3, max(1, K - 1)], device=dev)
+    for version in (-1, 0):
+        si, sd = tpo.knn_points(p1, p2, l1, l2, K=K, version=version)
+        ri, rd = torch.ops.torch_point_ops_knn.knn_forward(p1, p2, l1, l2, 2, K, version)
+        ei, ed = _module_sort(ri, rd, l2, K)
+        assert torch.equal(si, ei) and torch.equal(sd, ed)

@@ -200,7 +200,53 @@ __global__ __launch_bounds__(KR_THREADS) void knn_redo_kernel(
   }
 }
 
+// bfloat16 rows of K <= 32 slots as the module's sort leaves them
+// (knn/__init__.py:111-131: slots past lengths2 key as +inf and read 0
+// afterwards), in place: the 32-wide network of knn_sort_row with position p in
+// lane p, two rows a wave.
+__global__ __launch_bounds__(256) void knn_sort_rows_kernel(const int64_t* __restrict__ len2,
+                                                            int64_t rows, int P1, int K,
+                                                            int64_t* __restrict__ idxs,
+                                                            __bf16* __restrict__ dists) {
+  const int l = threadIdx.x & 31;
+  const int64_t row = (int64_t)blockIdx.x * 8 + (threadIdx.x >> 5);
+  const bool live = row < rows;
+  const int64_t r = live ? row : rows - 1;
+  const int64_t l2 = len2[r / P1];
+  const int size = (int)(l2 < 0 ? 0 : (l2 < K ? l2 : K));
+  const bool slot = l < K;
+  float d = slot && l < size ? (float)dists[r * K + (slot ? l : 0)] : Lim<float>::inf();
+  int x = slot ? (int)idxs[r * K + l] : 0, va = slot ? 1 : 0;
+#pragma unroll 1
+  for (int sz = 2; sz <= 32; sz *= 2)
+#pragma unroll 1
+    for (int stride = sz / 2; stride > 0; stride /= 2) {
+      const float pd = __shfl_xor(d, stride);
+      const int px = __shfl_xor(x, stride), pv = __shfl_xor(va, stride);
+      const bool up = sz < 32 && (l & sz) != 0, lo = (l & stride) == 0;
+      const float da = lo ? d : pd, db = lo ? pd : d;
+      const bool vA = (lo ? va : pv) != 0, vB = (lo ? pv : va) != 0;
+      const bool lt = !knn_isnan(da) && (knn_isnan(db) || da < db);
+      const bool sw = ((lt && vA) || !vB) == up;
+      d = sw ? pd : d;
+      x = sw ? px : x;
+      va = sw ? pv : va;
+    }
+  if (live && slot) {
+    idxs[row * K + l] = (int64_t)x;
+    dists[row * K + l] = l < size ? (__bf16)d : (__bf16)0.f;
+  }
+}
+
 }  // namespace
+
+static void launch_knn_sort_rows(const int64_t* l2, int64_t N, int P1, int K, int64_t* idxs,
+                                 void* dists, hipStream_t s) {
+  const int64_t rows = N * P1;
+  if (rows > 0)
+    hipLaunchKernelGGL(knn_sort_rows_kernel, dim3((unsigned)((rows + 7) / 8)), dim3(256), 0, s, l2,
+                       rows, P1, K, idxs, (__bf16*)dists);
+}
 
 void launch_knn_redo(const void* p1, const void* p2, const int64_t* l1, const int64_t* l2, int N,
                      int P1, int P2, int D, int K, int norm, int pad, bool sort, const RedoList& r,
@@ -223,3 +269,16 @@ void launch_knn_redo(const void* p1, const void* p2, const int64_t* l1, const in
 }
 
 }  // namespace tpo
+
+using namespace tpo;
+
+extern "C" int tpo_knn_sort_rows(int dtype, const int64_t* lengths2, int64_t N, int64_t P1,
+                                 int64_t K, int64_t* idxs, void* dists, void* stream) {
+  if (dtype != TPO_BF16)
+    return set_error(TPO_ERR_DTYPE, "tpo_knn_sort_rows: unsupported dtype %d", dtype);
+  if (N < 0 || P1 < 0 || K < 1 || K > 32 || N >= (1 << 20) || P1 >= (1 << 30) ||
+      N * P1 > (int64_t)8 * 0x7fffffff)
+    return set_error(TPO_ERR_ARG, "tpo_knn_sort_rows: bad sizes");
+  launch_knn_sort_rows(lengths2, N, (int)P1, (int)K, idxs, dists, (hipStream_t)stream);
+  return check_launch("tpo_knn_sort_rows");
+}

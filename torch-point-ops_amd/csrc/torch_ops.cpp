@@ -284,7 +284,7 @@ std::tuple<at::Tensor, at::Tensor> knn_forward_hip(const at::Tensor& p1_in,
 
 // knn_points(return_sorted=True) in one launch: the forward with each row
 // sorted as the module's torch sort leaves it (knn/__init__.py:111-131).
-// float/double/half with 2 <= K <= 32; the module keeps its own sort otherwise.
+// 2 <= K <= 32; the module keeps its own sort otherwise.
 std::tuple<at::Tensor, at::Tensor> knn_forward_sorted_hip(const at::Tensor& p1_in,
                                                           const at::Tensor& p2_in,
                                                           const at::Tensor& lengths1_in,
@@ -312,6 +312,13 @@ std::tuple<at::Tensor, at::Tensor> knn_forward_sorted_hip(const at::Tensor& p1_i
   TORCH_CHECK(lengths1_in.scalar_type() == at::kLong && lengths2_in.scalar_type() == at::kLong,
               "lengths must be int64");
   const at::Tensor l1 = lengths1_in.contiguous(), l2 = lengths2_in.contiguous();
+  if (p1_in.scalar_type() == at::kBFloat16) {  // the forward's rows, then the sort in place
+    std::tie(idxs, dists) = knn_forward_hip(p1_in, p2_in, lengths1_in, lengths2_in, norm, K, version);
+    check_rc(tpo_knn_sort_rows(TPO_BF16, l2.data_ptr<int64_t>(), N, P1, K,
+                               idxs.data_ptr<int64_t>(), dists.data_ptr(), stream_of(p1_in)),
+             "knn_forward_sorted");
+    return {idxs, dists};
+  }
   const at::Tensor p1 = p1_in.contiguous(), p2 = p2_in.contiguous();
   const int dt = dtype_code(p1, "knn_forward_sorted");
   const int64_t ws = tpo_knn_rows_workspace_size(dt, N, P1, P2, D, K, (int)norm);
@@ -457,20 +464,39 @@ auto typed_op(const char* name) {
   return c10::Dispatcher::singleton().findSchemaOrThrow(name, "").typed<Op>();
 }
 
+// Whether autograd has to follow the call.  Without it the operator runs as it
+// is, also under transforms that a C++ autograd function refuses.
+bool followed(const at::Tensor& a) { return at::GradMode::is_enabled() && a.requires_grad(); }
+
+template <bool SORTED>
+auto knn_op() {
+  static auto op = typed_op<std::tuple<at::Tensor, at::Tensor>(
+      const at::Tensor&, const at::Tensor&, const at::Tensor&, const at::Tensor&, int64_t, int64_t,
+      int64_t)>(SORTED ? "torch_point_ops_knn::knn_forward_sorted"
+                       : "torch_point_ops_knn::knn_forward");
+  return op;
+}
+auto knn_gather_op() {
+  static auto op = typed_op<at::Tensor(const at::Tensor&, const at::Tensor&, const at::Tensor&)>(
+      "torch_point_ops_knn::knn_gather");
+  return op;
+}
+auto gather_points_op() {
+  static auto op = typed_op<at::Tensor(const at::Tensor&, const at::Tensor&)>(
+      "torch_point_ops_fps::gather_points_forward");
+  return op;
+}
+
 template <bool SORTED>
 class KnnFunction : public torch::autograd::Function<KnnFunction<SORTED>> {
  public:
   static variable_list forward(AutogradContext* ctx, const at::Tensor& p1, const at::Tensor& p2,
                                const at::Tensor& lengths1, const at::Tensor& lengths2,
                                int64_t norm, int64_t K, int64_t version) {
-    static auto op = typed_op<std::tuple<at::Tensor, at::Tensor>(
-        const at::Tensor&, const at::Tensor&, const at::Tensor&, const at::Tensor&, int64_t,
-        int64_t, int64_t)>(SORTED ? "torch_point_ops_knn::knn_forward_sorted"
-                                  : "torch_point_ops_knn::knn_forward");
     at::Tensor idxs, dists;
     {
       at::AutoDispatchBelowADInplaceOrView below;
-      std::tie(idxs, dists) = op.call(p1, p2, lengths1, lengths2, norm, K, version);
+      std::tie(idxs, dists) = knn_op<SORTED>().call(p1, p2, lengths1, lengths2, norm, K, version);
     }
     ctx->save_for_backward({p1, p2, lengths1, lengths2, idxs});
     ctx->saved_data["norm"] = norm;
@@ -496,6 +522,10 @@ template <bool SORTED>
 std::tuple<at::Tensor, at::Tensor> knn_forward_autograd(
     const at::Tensor& p1, const at::Tensor& p2, const at::Tensor& lengths1,
     const at::Tensor& lengths2, int64_t norm, int64_t K, int64_t version) {
+  if (!followed(p1) && !followed(p2)) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    return knn_op<SORTED>().call(p1, p2, lengths1, lengths2, norm, K, version);
+  }
   auto out = KnnFunction<SORTED>::apply(p1, p2, lengths1, lengths2, norm, K, version);
   return {out[0], out[1]};
 }
@@ -504,19 +534,15 @@ class KnnGatherFunction : public torch::autograd::Function<KnnGatherFunction> {
  public:
   static at::Tensor forward(AutogradContext* ctx, const at::Tensor& x, const at::Tensor& idx,
                             const at::Tensor& lengths) {
-    static auto op = typed_op<at::Tensor(const at::Tensor&, const at::Tensor&, const at::Tensor&)>(
-        "torch_point_ops_knn::knn_gather");
     ctx->save_for_backward({idx, lengths});
     ctx->saved_data["M"] = x.sym_size(1).guard_int(__FILE__, __LINE__);
-    ctx->set_materialize_grads(false);
     at::AutoDispatchBelowADInplaceOrView below;
-    return op.call(x, idx, lengths);
+    return knn_gather_op().call(x, idx, lengths);
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     static auto op =
         typed_op<at::Tensor(const at::Tensor&, const at::Tensor&, const at::Tensor&, int64_t)>(
             "torch_point_ops_knn::knn_gather_backward");
-    if (!grads[0].defined()) return {at::Tensor(), at::Tensor(), at::Tensor()};
     const auto s = ctx->get_saved_variables();
     const int64_t M = ctx->saved_data["M"].toInt();
     if (at::GradMode::is_enabled())  // its own gradient is the gather (knn/__init__.py)
@@ -529,6 +555,10 @@ class KnnGatherFunction : public torch::autograd::Function<KnnGatherFunction> {
 at::Tensor knn_gather_autograd(const at::Tensor& x, const at::Tensor& idx,
                                const at::Tensor& lengths) {
   TORCH_CHECK(x.dim() == 3, "knn_gather expects (N,M,U) and (N,L,K)");
+  if (!followed(x)) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    return knn_gather_op().call(x, idx, lengths);
+  }
   return KnnGatherFunction::apply(x, idx, lengths);
 }
 
@@ -614,18 +644,14 @@ at::Tensor gather_points_backward_hip(const at::Tensor& grad_in, const at::Tenso
 class GatherPointsFunction : public torch::autograd::Function<GatherPointsFunction> {
  public:
   static at::Tensor forward(AutogradContext* ctx, const at::Tensor& points, const at::Tensor& idx) {
-    static auto op = typed_op<at::Tensor(const at::Tensor&, const at::Tensor&)>(
-        "torch_point_ops_fps::gather_points_forward");
     ctx->save_for_backward({idx});
     ctx->saved_data["n"] = points.sym_size(2).guard_int(__FILE__, __LINE__);
-    ctx->set_materialize_grads(false);
     at::AutoDispatchBelowADInplaceOrView below;
-    return op.call(points, idx);
+    return gather_points_op().call(points, idx);
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     static auto op = typed_op<at::Tensor(const at::Tensor&, const at::Tensor&, int64_t)>(
         "torch_point_ops_fps::gather_points_backward");
-    if (!grads[0].defined()) return {at::Tensor(), at::Tensor()};
     const auto s = ctx->get_saved_variables();
     return {op.call(grads[0], s[0], ctx->saved_data["n"].toInt()), at::Tensor()};
   }
@@ -633,6 +659,10 @@ class GatherPointsFunction : public torch::autograd::Function<GatherPointsFuncti
 
 at::Tensor gather_points_autograd(const at::Tensor& points, const at::Tensor& idx) {
   TORCH_CHECK(points.dim() == 3, "gather_points expects (N,C,P), (N,M)");
+  if (!followed(points)) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    return gather_points_op().call(points, idx);
+  }
   return GatherPointsFunction::apply(points, idx);
 }
 

@@ -28,8 +28,8 @@ def _knn_forward_sorted_fake(p1, p2, lengths1, lengths2, norm, K, version):
     return _knn_forward_fake(p1, p2, lengths1, lengths2, norm, K, version)
 
 
-# dtypes whose sorted rows come straight from the kernel (2 <= K <= 32)
-_SORTED_IN_KERNEL = (torch.float32, torch.float64, torch.float16)
+# dtypes whose sorted rows come straight from the kernels (2 <= K <= 32)
+_SORTED_IN_KERNEL = (torch.float32, torch.float64, torch.float16, torch.bfloat16)
 
 
 def _knn_gather_backward_backward(ctx, grad_grad_x):
