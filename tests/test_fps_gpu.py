@@ -64,6 +64,32 @@ def test_fps_held_sizes_vs_oracle(tpo, O, dev, dtype, N):
     assert np.array_equal(np_(got), O.fps(np_(pts), m))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
+@pytest.mark.parametrize("N,m", [(8193, 2000), (9000, 9000), (20000, 700), (65535, 300)])
+@pytest.mark.parametrize("kind", ["random", "lattice", "clusters", "sparse"])
+def test_fps_rounds_vs_oracle(tpo, O, dev, dtype, N, m, kind):
+    """Several samples a round: random clouds, lattices (every value tied),
+    clusters with copies (values fall to 0 long before the last sample) and
+    clouds of which few points take part, also with every point sampled."""
+    if m > 3000 and kind == "random" and dtype == torch.float16:
+        m = 3000
+    g = torch.Generator().manual_seed(N + m)
+    p = torch.randn(2, N, 3, generator=g)
+    if kind == "lattice":
+        p = torch.randint(-6, 7, (2, N, 3), generator=g).float() * 0.25
+    elif kind == "clusters":
+        c = torch.randn(2, 40, 3, generator=g)
+        p = c[:, torch.randint(0, 40, (N,), generator=g)] + 1e-2 * p.round(decimals=1)
+    elif kind == "sparse":
+        p[:, 50:] *= 1e-3
+        p[0] *= 1e-3
+        p[1, 7, 0] = float("inf")
+        p[1, 9, 0] = float("nan")
+    pts = p.to(dtype)
+    got = tpo.furthest_point_sampling(pts.to(dev), m)
+    assert np.array_equal(np_(got), O.fps(np_(pts), m))
+
+
 def test_fps_large_n_bucket_path(tpo, O, dev):
     """N > 65536 uses buckets of more than 64 points."""
     g = torch.Generator().manual_seed(4)

@@ -32,6 +32,23 @@
 //   sample, while the result is bit-identical to the full sweep.  The first
 //   sample (index 0) touches every point; its update is made in the set-up
 //   pass that initialises the running minima, with the same arithmetic.
+//
+// Several samples a round (float and half, buckets of 64).  A sample's chain
+// (box test, L2 loads, reductions, barrier) is mostly latency, so a round
+// chooses every sample that is already certain: each wave publishes its two
+// best buckets' candidates and a bound on all its other points (the third
+// best bucket, and each published bucket's second best point).  In key order
+// the candidates are the next samples as long as each lies above every
+// wave's bound and no earlier one lowers its running minimum (tested with the
+// kernel's own distance, a lane a pair); the rest of the round's order is
+// unknown and waits.  All of a round's samples are then applied to each
+// bucket they touch in one visit.  At 65536 points a round chooses 7.9
+// samples on average (4.2 with one candidate a wave): 16 x 65536 -> 4096
+// takes 2.62 ms against 4.49 ms a sample at a time, 16 x 16384 -> 1024 0.70
+// against 1.08 ms.  Bound: VALU issue, about 1000 instructions a sample over
+// the 16 waves (box tests 250, visits 400, the rest per round).
+//
+// Small clouds: fps_held_kernel.
 #include "tpo_common.hpp"
 
 #pragma clang fp contract(off)
@@ -229,7 +246,9 @@ __device__ __forceinline__ void fps_decode(int64_t* __restrict__ out, int m, int
   }
 }
 
-template <typename T>
+// ROUNDS (float and half, buckets of 64 points): several samples a round, see
+// the file header.
+template <typename T, bool ROUNDS>
 __global__ __launch_bounds__(FPS_THREADS) void fps_kernel(const T* __restrict__ pts, int N, int m,
                                                           int bs, int bs_bits, int per,
                                                           char* __restrict__ ws,
@@ -244,6 +263,9 @@ __global__ __launch_bounds__(FPS_THREADS) void fps_kernel(const T* __restrict__ 
   };
   __shared__ WaveBest s_wb[2][FPS_WAVES];
   __shared__ unsigned long long s_gkey[3];
+  __shared__ uint32_t s_tau[ROUNDS ? 3 : 1];
+  __shared__ uint64_t s_ck[ROUNDS ? 2 : 1][2 * FPS_WAVES];  // a round's candidates
+  __shared__ float4 s_cp[ROUNDS ? 2 : 1][2 * FPS_WAVES];
 
   const int b = blockIdx.x;
   const int tid = threadIdx.x, lane = lane_id(), w = wave_id();
@@ -284,6 +306,7 @@ __global__ __launch_bounds__(FPS_THREADS) void fps_kernel(const T* __restrict__ 
   }
   for (int c = tid; c < FPS_CELLS; c += FPS_THREADS) s_cnt[c] = 0;
   if (tid < 3) s_gkey[tid] = 0;
+  if (ROUNDS && tid < 3) s_tau[tid] = 0;
   __syncthreads();
   float glo[3], gscale[3];
 #pragma unroll
@@ -371,6 +394,7 @@ __global__ __launch_bounds__(FPS_THREADS) void fps_kernel(const T* __restrict__ 
   V blo[3], bhi[3];
   C bbest = cand_none(ctag);
   T bx = (T)0, by = (T)0, bz = (T)0;
+  V bsec = (V)0;  // ROUNDS: no other point of the bucket has a larger running minimum
 #pragma unroll
   for (int c = 0; c < 3; ++c) {
     blo[c] = (V)__builtin_inf();
@@ -397,10 +421,13 @@ __global__ __launch_bounds__(FPS_THREADS) void fps_kernel(const T* __restrict__ 
       const T d0 = sq3((T)(x - p0x), (T)(y - p0y), (T)(z - p0z));
       const C cand = cand_make((V)(d0 < init ? d0 : init), mt, ctag);
       if (cand_gt(cand, bbest)) {
+        bsec = cand_valid(bbest) ? (V)cand_val(bbest) : (V)0;
         bbest = cand;
         bx = x;
         by = y;
         bz = z;
+      } else {
+        bsec = vmax(bsec, (V)cand_val(cand));
       }
     }
     }
@@ -423,6 +450,167 @@ __global__ __launch_bounds__(FPS_THREADS) void fps_kernel(const T* __restrict__ 
   const V tiny = (V)FpsConst<T>::tiny();
   auto reach_of = [&](C c) -> V { return cand_valid(c) ? vmax((V)cand_val(c) * grow, tiny) : (V)-1; };
   V reach = reach_of(bbest);
+  if constexpr (ROUNDS) {
+    // Candidate i of the round: the better (i even) or second (odd) bucket
+    // best of wave i / 2; lanes i and i + 32 of every wave hold it.
+    uint64_t ck = 0;
+    float cx = 0.f, cy = 0.f, cz = 0.f;
+    uint32_t pm = 0;  // the candidates that are the last round's samples
+    int done = 1;     // samples chosen so far
+    int l1 = wlane, l2 = 0;
+    C w2 = cand_none(ctag);
+    uint32_t third = 0;
+    bool changed = true;
+    for (int rd = 0;; ++rd) {
+      if (pm != 0) {
+        // buckets within reach of a sample, a bit a sample
+        uint32_t hm = 0;
+        for (uint32_t mk = pm; mk != 0; mk &= mk - 1) {
+          const int i = __builtin_ctz(mk);
+          const float o3[3] = {bcast(cx, i), bcast(cy, i), bcast(cz, i)};
+          V e[3];
+#pragma unroll
+          for (int c = 0; c < 3; ++c) e[c] = vmax(vmax(blo[c] - o3[c], o3[c] - bhi[c]), (V)0);
+          const V lb2 = vfma(e[2], e[2], vfma(e[1], e[1], e[0] * e[0]));
+          hm |= lb2 <= reach ? 1u << i : 0u;
+        }
+        uint64_t tm = __ballot(hm != 0);
+        auto visit = [&](auto nbc) {  // as below, each bucket for all its samples
+          constexpr int NB = decltype(nbc)::value;
+          int bu[NB], pos[NB];
+          FpsRec<T> rc[NB];
+          T t[NB], t2[NB];
+#pragma unroll
+          for (int u = 0; u < NB; ++u) {
+            bu[u] = __builtin_ctzll(tm);
+            tm &= tm - 1;
+            pos[u] = (bu[u] * FPS_WAVES + w) * 64 + lane;
+            rc[u] = recs[pos[u]];
+            t[u] = ts[pos[u]];
+          }
+#pragma unroll
+          for (int u = 0; u < NB; ++u) {
+            t2[u] = t[u];
+            uint32_t mk = (uint32_t)__builtin_amdgcn_readlane((int)hm, bu[u]);
+            do {
+              const int i = __builtin_ctz(mk);
+              mk &= mk - 1;
+              const T ox = (T)bcast(cx, i), oy = (T)bcast(cy, i), oz = (T)bcast(cz, i);
+              const T d = sq3((T)(rc[u].x - ox), (T)(rc[u].y - oy), (T)(rc[u].z - oz));  // fps.cu:145
+              t2[u] = d < t2[u] ? d : t2[u];                                              // fps.cu:146
+            } while (mk != 0);
+          }
+#pragma unroll
+          for (int u = 0; u < NB; ++u) {
+            // re-reduced only when its best point's own running minimum dropped
+            const uint32_t bkey = (uint32_t)__builtin_amdgcn_readlane((int)cand_keyword(bbest), bu[u]);
+            if (__ballot(rc[u].key == bkey && t2[u] != t[u]) == 0) continue;
+            int wl;
+            const C cand = cand_make((V)t2[u], rc[u].key, ctag);
+            const C best = wave_best_at(cand, wl);
+            const uint32_t second = wave_umax(lane == wl ? 0u : __float_as_uint((float)t2[u]));
+            const T nx = bcast(rc[u].x, wl), ny = bcast(rc[u].y, wl), nz = bcast(rc[u].z, wl);
+            if (lane == bu[u]) {
+              bbest = best;
+              bsec = (V)__uint_as_float(second);
+              bx = nx;
+              by = ny;
+              bz = nz;
+            }
+            changed = true;
+          }
+#pragma unroll
+          for (int u = 0; u < NB; ++u)
+            if (t2[u] != t[u]) ts[pos[u]] = t2[u];
+        };
+        while (tm) {
+          const int nt = __builtin_popcountll(tm);
+          if (nt == 1) visit(std::integral_constant<int, 1>{});
+          else if (nt == 2) visit(std::integral_constant<int, 2>{});
+          else if (nt == 3) visit(std::integral_constant<int, 3>{});
+          else if (nt <= 5) visit(std::integral_constant<int, 4>{});
+          else visit(std::integral_constant<int, 6>{});
+        }
+        reach = reach_of(bbest);
+      }
+      if (changed) {  // the wave's two best buckets, and a bound on everything else in it
+        changed = false;
+        (void)wave_best_at(bbest, l1);
+        const C rest = lane == l1 ? cand_none(ctag) : bbest;
+        w2 = wave_best_at(rest, l2);
+        const bool pub = lane == l1 || (lane == l2 && cand_valid(w2));
+        third = wave_umax(__float_as_uint(pub ? (float)bsec : (float)cand_val(bbest)));
+      }
+      const int par = rd & 1;
+      if (lane == l1) {
+        s_ck[par][2 * w] = bbest.k;
+        s_cp[par][2 * w] = make_float4((float)bx, (float)by, (float)bz, 0.f);
+      }
+      // (a wave without a second bucket publishes no candidate there)
+      if (lane == (cand_valid(w2) ? l2 : (l1 ^ 1))) {
+        s_ck[par][2 * w + 1] = cand_valid(w2) ? bbest.k : 0ull;
+        s_cp[par][2 * w + 1] = make_float4((float)bx, (float)by, (float)bz, 0.f);
+      }
+      // three slots in turn: the next round's are cleared here, after their
+      // last readers (before the first barrier of this round)
+      if (lane == 0) atomicMax(&s_tau[rd % 3], third);
+      if (tid == 0) {
+        s_tau[(rd + 1) % 3] = 0;
+        s_gkey[(rd + 1) % 3] = 0;
+      }
+      __syncthreads();
+      // candidate j is out of order when one with a larger key lowers its
+      // running minimum, or would not lower its own (infinite coordinates:
+      // it is chosen again and again): wave w tests its two, a lane a pair
+      {
+        const int j = 2 * w + (lane >> 5);
+        ck = s_ck[par][lane & 31];
+        const float4 ci = s_cp[par][lane & 31];
+        const uint64_t kj = s_ck[par][j];
+        const float4 cj = s_cp[par][j];
+        cx = ci.x;
+        cy = ci.y;
+        cz = ci.z;
+        const T d = sq3((T)((T)cj.x - (T)ci.x), (T)((T)cj.y - (T)ci.y), (T)((T)cj.z - (T)ci.z));
+        const bool stays = !((ci.x - ci.x) + (ci.y - ci.y) + (ci.z - ci.z) == 0.f);
+        const uint64_t hit = __ballot(
+            ck > kj && kj != 0 && (stays || (float)d < __uint_as_float((uint32_t)(kj >> 32))));
+        if ((lane & 31) == 0 && (uint32_t)(hit >> lane) != 0)
+          atomicMax(&s_gkey[rd % 3], (unsigned long long)kj);
+      }
+      __syncthreads();
+      // this round's samples: the candidates above every such one, and above
+      // every other point's value
+      const uint64_t out_of = s_gkey[rd % 3];
+      const uint64_t others = (uint64_t)s_tau[rd % 3] << 32 | 0xffffffffull;
+      const uint64_t floor_key = out_of > others ? out_of : others;
+      pm = (uint32_t)__ballot(ck > floor_key);
+      if (pm == 0) {  // only the largest is certain
+        int gl;
+        const C g = wave_best_at(C{ck}, gl);
+        if (!cand_valid(g)) {  // nothing takes part: index 0 from here on (rank -1)
+          for (int j = done + tid; j < m; j += FPS_THREADS) out[j] = -1;
+          break;
+        }
+        pm = 1u << gl;
+      }
+      if (w == 0) {  // in key order
+        int at = done;
+        for (uint32_t mk = pm; mk != 0; mk &= mk - 1) {
+          const int i = __builtin_ctz(mk);
+          const uint64_t k = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(ck >> 32), i) << 32 |
+                             (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)ck, i);
+          at += k > ck ? 1 : 0;
+        }
+        if (lane < 32 && (pm >> lane) & 1 && at < m) out[at] = (int64_t)(0xffffffffu - (uint32_t)ck);
+      }
+      done += __builtin_popcount(pm);
+      if (done >= m) break;
+    }
+    __syncthreads();
+    fps_decode(out, m, tid, FPS_THREADS, bs, bs_bits, per);
+    return;
+  }
   for (int j = 1; j < m; ++j) {
     const V o3[3] = {(V)ox, (V)oy, (V)oz};
     V e[3];
@@ -572,7 +760,7 @@ __device__ __forceinline__ half_t fps_min(half_t d, half_t t) { return __builtin
 // alone takes about 0.43 us a sample (PPT = 2), a point a lane and wave adds
 // 0.02-0.04 us.  W: 16 clouds of 2048 points take 0.46 us a sample with 8
 // waves, 0.52 with 4, 0.51 with 16 (the bucket kernel 1.08); of 1024 0.44 with
-// 4, 0.48 with 8; of 8192 0.80 with 8, 1.13 with 4 (the bucket kernel 1.05).
+// 4, 0.48 with 8.
 template <typename T, int W, int PPT>
 __global__ __launch_bounds__(64 * W) void fps_held_kernel(const T* __restrict__ pts, int N, int m,
                                                           int bs, int bs_bits, int per,
@@ -658,8 +846,9 @@ __global__ __launch_bounds__(64 * W) void fps_held_kernel(const T* __restrict__ 
   fps_decode(out, m, tid, TH, bs, bs_bits, per);
 }
 
-// The held kernel's limit: the coordinate table's LDS (139 KB at 8192).
-constexpr int FPS_HELD_MAX = 8192;
+// The held kernel's limit: at 8192 points it takes 0.80 us a sample, the bucket
+// kernel 0.75 (at 6144, 0.68).
+constexpr int FPS_HELD_MAX = 6144;
 
 template <typename T>
 bool launch_held(const void* points, int64_t B, int N, int m, int bs, int bits, int per,
@@ -673,8 +862,7 @@ bool launch_held(const void* points, int64_t B, int N, int m, int bs, int bits, 
   else if (N <= 2048) FPS_HELD(8, 4);
   else if (N <= 3072) FPS_HELD(8, 6);
   else if (N <= 4096) FPS_HELD(8, 8);
-  else if (N <= 6144) FPS_HELD(8, 12);
-  else FPS_HELD(8, 16);
+  else FPS_HELD(8, 12);
 #undef FPS_HELD
   return true;
 }
@@ -720,15 +908,15 @@ extern "C" int tpo_fps_fwd(int dtype, const void* points, int64_t B, int64_t N, 
     return check_launch("tpo_fps_fwd");
   switch (dtype) {
     case TPO_F32:
-      hipLaunchKernelGGL(fps_kernel<float>, dim3((unsigned)B), dim3(FPS_THREADS), 0, s,
+      hipLaunchKernelGGL((N <= 65536 ? fps_kernel<float, true> : fps_kernel<float, false>), dim3((unsigned)B), dim3(FPS_THREADS), 0, s,
                          (const float*)points, (int)N, (int)nsamples, bs, bits, per, (char*)workspace, idx);
       break;
     case TPO_F64:
-      hipLaunchKernelGGL(fps_kernel<double>, dim3((unsigned)B), dim3(FPS_THREADS), 0, s,
+      hipLaunchKernelGGL((fps_kernel<double, false>), dim3((unsigned)B), dim3(FPS_THREADS), 0, s,
                          (const double*)points, (int)N, (int)nsamples, bs, bits, per, (char*)workspace, idx);
       break;
     case TPO_F16:
-      hipLaunchKernelGGL(fps_kernel<half_t>, dim3((unsigned)B), dim3(FPS_THREADS), 0, s,
+      hipLaunchKernelGGL((N <= 65536 ? fps_kernel<half_t, true> : fps_kernel<half_t, false>), dim3((unsigned)B), dim3(FPS_THREADS), 0, s,
                          (const half_t*)points, (int)N, (int)nsamples, bs, bits, per, (char*)workspace, idx);
       break;
     default: return set_error(TPO_ERR_DTYPE, "tpo_fps_fwd: unsupported dtype %d", dtype);
