@@ -203,6 +203,60 @@ std::tuple<at::Tensor, at::Tensor, at::Tensor> chamfer_loss_forward_autograd(
   return {out[0], out[1], out[2]};
 }
 
+// Whether autograd has to follow the call.  Without it the operator runs as it
+// is, also under transforms that a C++ autograd function refuses.
+bool followed(const at::Tensor& a) { return at::GradMode::is_enabled() && a.requires_grad(); }
+
+// chamfer_forward's autograd (chamfer/__init__.py:6-28) in C++: an unused
+// distance output's gradient arrives undefined and counts as zeros.
+class ChamferFunction : public torch::autograd::Function<ChamferFunction> {
+ public:
+  typedef std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> Outputs;
+  static auto op() {
+    static auto h = c10::Dispatcher::singleton()
+                        .findSchemaOrThrow("torch_point_ops_chamfer::chamfer_forward", "")
+                        .typed<Outputs(const at::Tensor&, const at::Tensor&)>();
+    return h;
+  }
+  static torch::autograd::variable_list forward(torch::autograd::AutogradContext* ctx,
+                                                const at::Tensor& xyz1, const at::Tensor& xyz2) {
+    at::Tensor d1, d2, i1, i2;
+    {
+      at::AutoDispatchBelowADInplaceOrView below;
+      std::tie(d1, d2, i1, i2) = op().call(xyz1, xyz2);
+    }
+    ctx->save_for_backward({xyz1, xyz2, i1, i2});
+    ctx->mark_non_differentiable({i1, i2});
+    ctx->set_materialize_grads(false);
+    return {d1, d2, i1, i2};
+  }
+  static torch::autograd::variable_list backward(torch::autograd::AutogradContext* ctx,
+                                                 torch::autograd::variable_list grads) {
+    static auto bwd = c10::Dispatcher::singleton()
+                          .findSchemaOrThrow("torch_point_ops_chamfer::chamfer_backward", "")
+                          .typed<std::tuple<at::Tensor, at::Tensor>(
+                              const at::Tensor&, const at::Tensor&, const at::Tensor&,
+                              const at::Tensor&, const at::Tensor&, const at::Tensor&)>();
+    if (!grads[0].defined() && !grads[1].defined()) return {at::Tensor(), at::Tensor()};
+    const auto s = ctx->get_saved_variables();
+    const auto like = [&](const at::Tensor& g, const at::Tensor& idx) {
+      return g.defined() ? g : at::zeros_symint(idx.sym_sizes(), s[0].options());
+    };
+    at::Tensor g1, g2;
+    std::tie(g1, g2) = bwd.call(s[0], s[1], s[2], s[3], like(grads[0], s[2]), like(grads[1], s[3]));
+    return {g1, g2};
+  }
+};
+
+ChamferFunction::Outputs chamfer_forward_autograd(const at::Tensor& xyz1, const at::Tensor& xyz2) {
+  if (!followed(xyz1) && !followed(xyz2)) {
+    at::AutoDispatchBelowADInplaceOrView below;
+    return ChamferFunction::op().call(xyz1, xyz2);
+  }
+  auto out = ChamferFunction::apply(xyz1, xyz2);
+  return {out[0], out[1], out[2], out[3]};
+}
+
 // chamfer.cpp:21-31: the reference has no CPU kernel.
 std::tuple<at::Tensor, at::Tensor, at::Tensor, at::Tensor> chamfer_forward_cpu(
     const at::Tensor&, const at::Tensor&) {
@@ -463,10 +517,6 @@ template <typename Op>
 auto typed_op(const char* name) {
   return c10::Dispatcher::singleton().findSchemaOrThrow(name, "").typed<Op>();
 }
-
-// Whether autograd has to follow the call.  Without it the operator runs as it
-// is, also under transforms that a C++ autograd function refuses.
-bool followed(const at::Tensor& a) { return at::GradMode::is_enabled() && a.requires_grad(); }
 
 template <bool SORTED>
 auto knn_op() {
@@ -754,6 +804,7 @@ TORCH_LIBRARY_IMPL(torch_point_ops_chamfer, CPU, m) {
   m.impl("chamfer_loss_backward", &chamfer_loss_backward_cpu);
 }
 TORCH_LIBRARY_IMPL(torch_point_ops_chamfer, Autograd, m) {
+  m.impl("chamfer_forward", &chamfer_forward_autograd);
   m.impl("chamfer_loss_forward", &chamfer_loss_forward_autograd);
 }
 TORCH_LIBRARY_IMPL(torch_point_ops_chamfer, CUDA, m) {

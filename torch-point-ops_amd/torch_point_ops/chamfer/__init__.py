@@ -1,42 +1,12 @@
 """Chamfer distance (reference: torch_point_ops/chamfer/__init__.py:1-75).
 
 torch.ops.torch_point_ops_chamfer.chamfer_forward / chamfer_backward run the
-gfx950 kernels of libtpo_hip.so; this module adds the autograd formula and
-the FakeTensor kernels, as the reference does.
+gfx950 kernels of libtpo_hip.so; this module adds the FakeTensor kernels, as
+the reference does.
 """
 import torch
 
 from .. import _C  # noqa: F401
-
-
-def _chamfer_backward(ctx, grad_dist1, grad_dist2, grad_idx1, grad_idx2):
-    # index outputs carry no gradient (reference chamfer/__init__.py:6-11);
-    # gradients are not materialised, so an unused distance output arrives
-    # as None and counts as zeros
-    xyz1, xyz2, idx1, idx2 = ctx.saved_tensors
-    if grad_dist1 is None and grad_dist2 is None:
-        return None, None
-    if grad_dist1 is None:
-        grad_dist1 = torch.zeros(idx1.shape, dtype=xyz1.dtype, device=xyz1.device)
-    if grad_dist2 is None:
-        grad_dist2 = torch.zeros(idx2.shape, dtype=xyz2.dtype, device=xyz2.device)
-    return torch.ops.torch_point_ops_chamfer.chamfer_backward(
-        xyz1, xyz2, idx1, idx2, grad_dist1, grad_dist2
-    )
-
-
-def _chamfer_setup_context(ctx, inputs, output):
-    xyz1, xyz2 = inputs
-    _d1, _d2, idx1, idx2 = output
-    ctx.save_for_backward(xyz1, xyz2, idx1, idx2)
-    ctx.set_materialize_grads(False)  # no zero tensors for the index outputs
-
-
-torch.library.register_autograd(
-    "torch_point_ops_chamfer::chamfer_forward",
-    _chamfer_backward,
-    setup_context=_chamfer_setup_context,
-)
 
 
 @torch.library.register_fake("torch_point_ops_chamfer::chamfer_forward")
@@ -57,8 +27,8 @@ def _chamfer_backward_fake(xyz1, xyz2, idx1, idx2, grad_dist1, grad_dist2):
     return torch.empty_like(xyz1), torch.empty_like(xyz2)
 
 
-# chamfer_loss_forward's autograd is registered in C++ (torch_ops.cpp,
-# ChamferLossFunction): the training step's backward runs no Python.
+# The autograd of chamfer_forward and chamfer_loss_forward is registered in C++
+# (torch_ops.cpp): a training step runs no Python for them.
 
 
 @torch.library.register_fake("torch_point_ops_chamfer::chamfer_loss_forward")
