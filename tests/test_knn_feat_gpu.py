@@ -101,3 +101,62 @@ def test_single_nearest_takes_the_lower_index(tpo, O, dev, D, P2):
         i, d = tpo.knn_points(p1.to(dev), p2.to(dev), l1.to(dev), l2.to(dev), K=1, version=version)
         ei, ed = O.knn_fwd(p1.numpy(), p2.numpy(), l1.numpy(), l2.numpy(), K=1, version=version)
         assert np.array_equal(i.cpu().numpy(), ei) and np.array_equal(d.cpu().numpy(), ed)
+
+
+@pytest.mark.parametrize("D", [3, 9, 64])
+def test_rows_of_views_off_16_bytes(tpo, dev, D):
+    """Clouds that start 4 bytes past a 16-byte boundary."""
+    g = torch.Generator().manual_seed(D)
+    P1, P2, K = 70, 700, 9
+    a = torch.randn(2 * P1 * D + 1, generator=g).to(dev)[1:].view(2, P1, D)
+    b = torch.randn(2 * P2 * D + 1, generator=g).to(dev)[1:].view(2, P2, D)
+    b[:, 5] = b[:, 6]  # equal distances: replayed rows
+    l1, l2 = torch.tensor([P1, 33], device=dev), torch.tensor([P2, 500], device=dev)
+    ri, rd = torch.ops.torch_point_ops_knn.knn_forward(a, b, l1, l2, 2, K, 0)
+    ei, ed = _sorted_by_module(ri, rd, l2, K)
+    si, sd = tpo.knn_points(a, b, l1, l2, K=K, version=0)
+    assert torch.equal(si, ei) and torch.equal(sd, ed)
+
+
+def test_rows_captured_in_a_graph(tpo, dev):
+    """knn_points (both row paths, ties among the rows), sampling and the
+    gathers' gradients replayed from a graph on new inputs, with eager work
+    between the replays."""
+    g = torch.Generator().manual_seed(8)
+
+    def draw():
+        p = torch.randn(2, 900, 3, generator=g).round(decimals=1)
+        f = torch.randn(2, 300, 40, generator=g).round(decimals=0)
+        w = torch.randn(2, 900, 8, 3, generator=g)
+        return p.to(dev), f.to(dev), w.to(dev)
+
+    s_p, s_f, s_w = draw()
+    lens = torch.tensor([900, 700], device=dev)
+
+    def step(p, f, w):
+        q = p.detach().requires_grad_(True)
+        i, d = tpo.knn_points(p, p, lens, lens, K=8)
+        nn = tpo.knn_gather(q, i, lens)
+        (gq,) = torch.autograd.grad(nn, (q,), w)
+        fi, fd = tpo.knn_points(f, f, K=5)
+        s = tpo.furthest_point_sampling(p, 40)
+        return i, d, gq, fi, fd, s
+
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        for _ in range(2):
+            step(s_p, s_f, s_w)
+    torch.cuda.current_stream().wait_stream(side)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = step(s_p, s_f, s_w)
+    for _ in range(4):
+        p, f, w = draw()
+        want = [t.clone() for t in step(p, f, w)]
+        s_p.copy_(p), s_f.copy_(f), s_w.copy_(w)
+        torch.cuda.synchronize()
+        graph.replay()
+        torch.cuda.synchronize()
+        for a, b in zip(got, want):
+            assert torch.equal(a, b)

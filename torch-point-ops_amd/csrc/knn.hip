@@ -560,8 +560,15 @@ static int knn_fwd_impl(int dtype, const void* p1, const void* p2, const int64_t
   const int pad = v <= 1;
   const int sorted2 = (v == 3 && K == 2) | (sort_rows ? 2 : 0);  // the kernel's mode bits
   hipStream_t s = (hipStream_t)stream;
-  // rows by distance, many dimensions: candidates from the matrix cores
-  if ((sort_rows || K == 1) && !(sorted2 & 1) && D != 3 && workspace &&
+  // Rows by distance, where the caller gives the workspace for it (16-byte
+  // aligned): the sorted rows, and a single nearest, do not depend on the slot
+  // layout.  RegisterMinK<2> keeps its own order among equal distances.
+  const bool rows = (sort_rows || K == 1) && !(sorted2 & 1) && workspace &&
+                    ((uintptr_t)workspace & 15) == 0;
+  // many dimensions: candidates from the matrix cores (8 x 2048 x 2048, D =
+  // 64, K = 20: 58 us against 2500 with a query a lane over the whole cloud;
+  // 4 x 299 x 299, D = 9: 29 against 310)
+  if (rows && D != 3 &&
       knn_feat_applies(dtype, N, P1, P2, D, K, norm) &&
       workspace_bytes >= knn_feat_workspace(N, P1, P2, D)) {
     const RedoList r =
@@ -573,8 +580,10 @@ static int knn_fwd_impl(int dtype, const void* p1, const void* p2, const int64_t
                       (int)K, norm, pad, sorted2, r.total, idxs, dists, s);
     return check_launch("tpo_knn_fwd");
   }
-  // rows by distance, three dimensions: a cell grid
-  if ((sort_rows || K == 1) && !(sorted2 & 1) && workspace &&
+  // three dimensions: a cell grid (16 x 2048 x 2048, K = 16: 69 us a call
+  // against 210 with the prefix and box replay; 14 x 512 x 585, K = 8: 51
+  // against 70 brute force; 7 x 1915 x 358, K = 20: 50 against 147)
+  if (rows &&
       knn_near_applies(dtype, N, P1, P2, D, K) && workspace_bytes >= knn_near_workspace(N, P1, P2)) {
     const bool grid_redo = sort_rows && knn_grid_applies(dtype, D, K, P2);
     const RedoList r =
