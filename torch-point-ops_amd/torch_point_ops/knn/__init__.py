@@ -96,10 +96,13 @@ def knn_points(
         raise ValueError("p1 and p2 must have the same point dimension.")
     N, P1, _D = p1.shape
     P2 = p2.shape[1]
-    if lengths1 is None:
-        lengths1 = torch.full((N,), P1, dtype=torch.int64, device=p1.device)
+    # all points: one launch for both clouds where they are of one length
     if lengths2 is None:
         lengths2 = torch.full((N,), P2, dtype=torch.int64, device=p1.device)
+        if lengths1 is None and P1 == P2:
+            lengths1 = lengths2
+    if lengths1 is None:
+        lengths1 = torch.full((N,), P1, dtype=torch.int64, device=p1.device)
 
     if return_sorted and 2 <= K <= 32 and p1.dtype in _SORTED_IN_KERNEL and p1.is_cuda:
         # the kernel replays the sort below (torch's network, ties included)

@@ -4,6 +4,15 @@ import torch
 from . import knn_points
 
 
+def _whole(p1, p2, lengths1, lengths2):
+    """The default lengths made once for the search and the gather behind it."""
+    if lengths2 is None:
+        lengths2 = torch.full((p2.shape[0],), p2.shape[1], dtype=torch.int64, device=p2.device)
+        if lengths1 is None and p1.shape[:2] == p2.shape[:2]:
+            lengths1 = lengths2
+    return lengths1, lengths2
+
+
 class KNearestNeighbors(torch.nn.Module):
     """K nearest neighbours of p1's points in p2, optionally with the neighbours.
 
@@ -24,6 +33,8 @@ class KNearestNeighbors(torch.nn.Module):
         self.version = version
 
     def forward(self, p1, p2, lengths1=None, lengths2=None):
+        if self.return_nn:
+            lengths1, lengths2 = _whole(p1, p2, lengths1, lengths2)
         idxs, dists = knn_points(
             p1, p2, lengths1=lengths1, lengths2=lengths2, norm=self.norm, K=self.K,
             version=self.version, return_sorted=self.return_sorted,
@@ -40,6 +51,8 @@ class KNNFunction(torch.nn.Module):
 
     def forward(self, p1, p2, lengths1=None, lengths2=None, norm=2, K=1, version=-1,
                 return_nn=False, return_sorted=True):
+        if return_nn:
+            lengths1, lengths2 = _whole(p1, p2, lengths1, lengths2)
         idxs, dists = knn_points(
             p1, p2, lengths1=lengths1, lengths2=lengths2, norm=norm, K=K, version=version,
             return_sorted=return_sorted,
