@@ -620,9 +620,22 @@ KnLayout kn_layout(int64_t N, int64_t P1, int64_t P2) {
 
 }  // namespace
 
-// One workgroup bins a cloud: clouds of up to 2^18 points.
+// One workgroup bins a cloud: clouds of up to 2^18 points.  A search costs a
+// query about the same whatever the cloud, brute force (knn_fwd_kernel) about
+// in proportion to it, and less a query where many queries fill the GPU.
+// Measured, us with the grid / brute force, 131072 queries (8192 queries):
+//   P2 = 128: K = 3 76 / 51 (27 / 25), K = 8 101 / 65 (30 / 36), K = 32 165 / 150 (31 / 103)
+//   P2 = 256: K = 1 49 / 49, K = 8 90 / 75 (30 / 44), K = 16 105 / 114, K = 32 159 / 189
+//   P2 = 384: K = 8 97 / 82 (28 / 54);  P2 = 512: K = 3 66 / 69, K = 8 86 / 89, K = 16 117 / 142
+static bool kn_pays(int64_t rows, int64_t P2, int64_t K) {
+  if (P2 >= 512) return true;
+  const bool many = rows > 49152;  // 32768 queries still gain at P2 = 256 (43 / 48 at K = 8)
+  if (P2 >= 256) return !many || K == 1 || K >= 16;
+  return P2 >= 128 && K >= 16 && !many;
+}
+
 bool knn_near_applies(int dtype, int64_t N, int64_t P1, int64_t P2, int64_t D, int64_t K) {
-  return dtype == TPO_F32 && D == 3 && K >= 1 && K <= 32 && N >= 1 && P1 >= 1 && P2 >= 1 &&
+  return kn_pays(N * P1, P2, K) && dtype == TPO_F32 && D == 3 && K >= 1 && K <= 32 && N >= 1 && P1 >= 1 && P2 >= 1 &&
          P1 <= (1 << 18) && P2 <= (1 << 18) && N <= (1 << 16) && N * P1 <= 0x7fffffff;
 }
 
