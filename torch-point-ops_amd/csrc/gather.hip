@@ -209,15 +209,10 @@ __global__ __launch_bounds__(GATHER_ROWS_THREADS) void gather_bwd_rows_kernel(
           if (n >= ce) break;
           const bool hit = p[u] != 0xffff;
           const T* __restrict__ r = rows + (hit ? p[u] : 0);
-          // 0 + g, as the reference's atomicAdd into zeros gives (+0 for g = -0).
-          // Stored past the caches: nothing here reads the gradient again, and
-          // 268 MB of dirty lines would be written back under the next reads
-          // (a forward and backward of 16 x 64 x 65536, 4096 samples, new
-          // inputs each time: 122 -> 111 us; the backward alone the same).
+          // 0 + g, as the reference's atomicAdd into zeros gives (+0 for g = -0)
 #pragma unroll
           for (int c = 0; c < CB; ++c)
-            if (c < cn)
-              __builtin_nontemporal_store(hit ? (T)((T)0 + r[c * M]) : (T)0, dst + c * N + n);
+            if (c < cn) dst[c * N + n] = hit ? (T)((T)0 + r[c * M]) : (T)0;
         }
       }
       __syncthreads();  // the next chunk's fill waits for this chunk's map reads
