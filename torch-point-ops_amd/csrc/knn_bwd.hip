@@ -117,12 +117,12 @@ KbPlan kb_plan(int64_t N, int64_t P1, int64_t P2, int64_t D, int64_t K) {
 constexpr unsigned KB_NO_MIN = 0x7f800000u;
 
 // Counting sort of a workgroup's records (one a thread: reference row r with
-// terms t[0, D), or r < 0 for none) by bucket, into the workgroup's own
+// terms t[0, D), negated with NEG, or r < 0 for none) by bucket, into the workgroup's own
 // region; the table gets (count, start, largest |term|, smallest nonzero
 // |term|) per bucket, the last from s_min or `min_all` where none is kept.
 // s_cnt, s_max (and s_min) are zeroed (KB_NO_MIN) before the caller's last
 // barrier.
-template <typename T, typename A, int DC>
+template <typename T, typename A, int DC, bool NEG>
 __device__ __forceinline__ void kb_group_records(const T (&t)[DC], int r, int D, int n, int c,
                                                  int cpc, int R, int nb, unsigned min_all,
                                                  int* s_cnt, unsigned* s_max, unsigned* s_min,
@@ -130,6 +130,7 @@ __device__ __forceinline__ void kb_group_records(const T (&t)[DC], int r, int D,
                                                  int4* __restrict__ tab) {
   const int tid = threadIdx.x;
   const int bk = r >= 0 ? r / R : -1;
+  const auto term = [&](int d) { return NEG ? -t[d] : t[d]; };
   int rank = 0;
   if (bk >= 0) {
     rank = atomicAdd(&s_cnt[bk], 1);
@@ -171,9 +172,9 @@ __device__ __forceinline__ void kb_group_records(const T (&t)[DC], int r, int D,
     A* __restrict__ o = rec + ((int64_t)blockIdx.x * KB1_THREADS + s_cnt[bk] + rank) * rw;
     if constexpr (sizeof(A) == 4) {
       if (rw == 4) {
-        *reinterpret_cast<float4*>(o) =
-            make_float4(__int_as_float(r - bk * R), (float)t[0], D > 1 ? (float)t[DC > 1 ? 1 : 0] : 0.f,
-                        D > 2 ? (float)t[DC > 2 ? 2 : 0] : 0.f);
+        *reinterpret_cast<float4*>(o) = make_float4(__int_as_float(r - bk * R), (float)term(0),
+                                                    D > 1 ? (float)term(DC > 1 ? 1 : 0) : 0.f,
+                                                    D > 2 ? (float)term(DC > 2 ? 2 : 0) : 0.f);
         return;
       }
       o[0] = __int_as_float(r - bk * R);
@@ -182,7 +183,7 @@ __device__ __forceinline__ void kb_group_records(const T (&t)[DC], int r, int D,
     }
 #pragma unroll
     for (int d = 0; d < DC; ++d)
-      if (d < D) o[1 + d] = (A)t[d];
+      if (d < D) o[1 + d] = (A)term(d);
   }
 }
 
@@ -256,9 +257,7 @@ __global__ __launch_bounds__(KB1_THREADS) void knn_bwd_entry_kernel(
     gp1[((int64_t)n * P1 + q0) * D + e] = sum;
   }
   if constexpr (BUCKETED) {
-#pragma unroll
-    for (int d = 0; d < DC; ++d) diff[d] = (T)-diff[d];
-    kb_group_records<T, A, DC>(diff, r, D, n, c, cpc, R, nb, KB_NO_MIN, s_cnt, s_max, nullptr,
+    kb_group_records<T, A, DC, true>(diff, r, D, n, c, cpc, R, nb, KB_NO_MIN, s_cnt, s_max, nullptr,
                                s_part, rec, tab);
   }
 }
@@ -322,7 +321,8 @@ __device__ __forceinline__ void kb_for_records(const A* __restrict__ rec,
 // float terms within ~2^28 of the largest).  Integer sums are exact and
 // order-free, so grad_p2 is the same on every run; each row is converted
 // back once.
-template <typename T>
+// CHECKED: the table's smallest terms decide whether fixed point holds them.
+template <typename T, bool CHECKED>
 __global__ __launch_bounds__(KB2_THREADS) void knn_bwd_bucket_kernel(
     const typename BwdAcc<T>::type* __restrict__ rec, const int4* __restrict__ tab, int P2, int D,
     int cpc, int R, int nb, T* __restrict__ gp2) {
@@ -347,17 +347,17 @@ __global__ __launch_bounds__(KB2_THREADS) void knn_bwd_bucket_kernel(
     const int4 cs = t[c];
     tot += (unsigned)cs.x;
     m = max(m, (unsigned)cs.z);
-    if (cs.x) lo = min(lo, (unsigned)cs.w);
+    if (CHECKED && cs.x) lo = min(lo, (unsigned)cs.w);
   }
   for (int o = 32; o > 0; o >>= 1) {
     tot += (unsigned)__shfl_xor((int)tot, o, 64);
     m = max(m, (unsigned)__shfl_xor((int)m, o, 64));
-    lo = min(lo, (unsigned)__shfl_xor((int)lo, o, 64));
+    if constexpr (CHECKED) lo = min(lo, (unsigned)__shfl_xor((int)lo, o, 64));
   }
   if ((tid & 63) == 0 && tot) {
     atomicAdd(&s_total, tot);
     atomicMax(&s_max, m);
-    atomicMin(&s_min, lo);
+    if constexpr (CHECKED) atomicMin(&s_min, lo);
   }
   __syncthreads();
   const unsigned mb = s_max, total = s_total;
@@ -371,8 +371,8 @@ __global__ __launch_bounds__(KB2_THREADS) void knn_bwd_bucket_kernel(
   T* __restrict__ o = gp2 + ((int64_t)n * P2 + r0) * D;
   // with a smallest term given, fixed point only where it holds every term's
   // last bit (24 bits below the smallest term's exponent)
-  const int e1 = (int)((s_min >> 23) & 0xff) - 127;
-  if (mb < 0x7f800000u && (e1 < -126 ? -126 : e1) - 23 + S >= 0) {
+  const int e1 = CHECKED ? (int)((s_min >> 23) & 0xff) - 127 : 0;
+  if (mb < 0x7f800000u && (!CHECKED || (e1 < -126 ? -126 : e1) - 23 + S >= 0)) {
     if (mb != 0u) {
       const double scale = __builtin_ldexp(1.0, S);
       kb_for_records<A>(rec, t, n, cpc, D, [&](int row, const A (&v)[7]) {
@@ -446,7 +446,7 @@ __global__ __launch_bounds__(KB1_THREADS) void knn_gather_bwd_entry_kernel(
   __syncthreads();
   // double terms are summed in floating point: the fixed point holds 52 bits
   // below a bucket's largest term, a row of small ones would lose some
-  kb_group_records<T, A, DC>(t, r, U, n, c, cpc, R, nb, 1u, s_cnt, s_max,
+  kb_group_records<T, A, DC, false>(t, r, U, n, c, cpc, R, nb, 1u, s_cnt, s_max,
                              sizeof(A) == 4 ? s_min : nullptr, s_part, rec, tab);
 }
 
@@ -500,7 +500,7 @@ void launch_gather_bwd(const void* go, const int64_t* idx, const int64_t* length
     hipLaunchKernelGGL((knn_gather_bwd_entry_kernel<T, 7>), dim3((unsigned)p.w1),
                        dim3(KB1_THREADS), 0, s, (const T*)go, idx, lengths, (int)M, (int)LK,
                        (int)K, (int)U, p.cpc, p.R, p.nb, rec, tab);
-  hipLaunchKernelGGL(knn_bwd_bucket_kernel<T>, dim3((unsigned)(N * p.nb)), dim3(KB2_THREADS),
+  hipLaunchKernelGGL((knn_bwd_bucket_kernel<T, true>), dim3((unsigned)(N * p.nb)), dim3(KB2_THREADS),
                      (size_t)p.R * U * 8, s, (const A*)rec, (const int4*)tab, (int)M, (int)U,
                      p.cpc, p.R, p.nb, (T*)gx);
 }
@@ -540,7 +540,7 @@ void launch_bwd(const void* p1, const void* p2, const int64_t* l1, const int64_t
                          dim3(KB1_THREADS), 0, s, (const T*)p1, (const T*)p2, l1, idxs,
                          (const T*)gd, norm, (int)P1, (int)P2, (int)D, (int)K, p.rpw, p.cpc, p.R,
                          p.nb, (T*)gp1, (T*)gp2, rec, tab);
-    hipLaunchKernelGGL(knn_bwd_bucket_kernel<T>, dim3((unsigned)(N * p.nb)), dim3(KB2_THREADS),
+    hipLaunchKernelGGL((knn_bwd_bucket_kernel<T, false>), dim3((unsigned)(N * p.nb)), dim3(KB2_THREADS),
                        (size_t)p.R * D * 8, s, (const A*)rec, (const int4*)tab, (int)P2,
                        (int)D, p.cpc, p.R, p.nb, (T*)gp2);
     return;
