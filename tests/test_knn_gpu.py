@@ -368,6 +368,9 @@ def test_knn_gather_kernel_matches_torch_ops(tpo, dev, dtype, U, L):
     (2, 600, 300, 4, "infinite"),
     (3, 100, 60, 4, "zero"),
     (8, 300, 90, 6, "normal"),    # longer rows: torch's scatter
+    (3, 600, 300, 4, "2^-110"),   # double terms that a float holds, but not 52 bits below them
+    (3, 600, 300, 4, "2^-200"),   # double terms below the smallest float
+    (7, 50, 300, 4, "2^-200"),
 ])
 def test_knn_gather_backward_vs_float64(tpo, dev, dtype, U, M, L, K, terms):
     """Each row's gradient within the error of a float sum in any order,
@@ -382,6 +385,9 @@ def test_knn_gather_backward_vs_float64(tpo, dev, dtype, U, M, L, K, terms):
     if terms == "wide":
         span = 7 if dtype == torch.float16 else 60
         go = go * 2.0 ** torch.randint(-span, span + 1, go.shape, generator=g)
+    if terms.startswith("2^-"):  # and rows whose terms are all 2^-40 of the largest
+        go = go * 2.0 ** -int(terms[3:])
+        go[..., -1] *= 2.0 ** -40
     go = go.to(dtype)
     if terms == "infinite":
         go[0, 5, 1, 0] = float("inf")

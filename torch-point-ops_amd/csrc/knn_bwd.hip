@@ -119,15 +119,14 @@ constexpr unsigned KB_NO_MIN = 0x7f800000u;
 // Counting sort of a workgroup's records (one a thread: reference row r with
 // terms t[0, D), negated with NEG, or r < 0 for none) by bucket, into the workgroup's own
 // region; the table gets (count, start, largest |term|, smallest nonzero
-// |term|) per bucket, the last from s_min or `min_all` where none is kept.
+// |term|) per bucket, the last from s_min, KB_NO_MIN where none is kept.
 // s_cnt, s_max (and s_min) are zeroed (KB_NO_MIN) before the caller's last
 // barrier.
 template <typename T, typename A, int DC, bool NEG>
 __device__ __forceinline__ void kb_group_records(const T (&t)[DC], int r, int D, int n, int c,
-                                                 int cpc, int R, int nb, unsigned min_all,
-                                                 int* s_cnt, unsigned* s_max, unsigned* s_min,
-                                                 int* s_part, A* __restrict__ rec,
-                                                 int4* __restrict__ tab) {
+                                                 int cpc, int R, int nb, int* s_cnt,
+                                                 unsigned* s_max, unsigned* s_min, int* s_part,
+                                                 A* __restrict__ rec, int4* __restrict__ tab) {
   const int tid = threadIdx.x;
   const int bk = r >= 0 ? r / R : -1;
   const auto term = [&](int d) { return NEG ? -t[d] : t[d]; };
@@ -163,7 +162,7 @@ __device__ __forceinline__ void kb_group_records(const T (&t)[DC], int r, int D,
   // table [cloud][bucket][entry workgroup]: a bucket's entries are consecutive
   if (tid < nb)
     tab[((int64_t)n * nb + tid) * cpc + c] =
-        make_int4(cnt, start, (int)s_max[tid], (int)(s_min ? s_min[tid] : min_all));
+        make_int4(cnt, start, (int)s_max[tid], (int)(s_min ? s_min[tid] : KB_NO_MIN));
   __syncthreads();  // every count read before the starts overwrite them
   if (tid < nb) s_cnt[tid] = start;
   __syncthreads();
@@ -257,8 +256,8 @@ __global__ __launch_bounds__(KB1_THREADS) void knn_bwd_entry_kernel(
     gp1[((int64_t)n * P1 + q0) * D + e] = sum;
   }
   if constexpr (BUCKETED) {
-    kb_group_records<T, A, DC, true>(diff, r, D, n, c, cpc, R, nb, KB_NO_MIN, s_cnt, s_max, nullptr,
-                               s_part, rec, tab);
+    kb_group_records<T, A, DC, true>(diff, r, D, n, c, cpc, R, nb, s_cnt, s_max, nullptr, s_part,
+                                     rec, tab);
   }
 }
 
@@ -321,7 +320,10 @@ __device__ __forceinline__ void kb_for_records(const A* __restrict__ rec,
 // float terms within ~2^28 of the largest).  Integer sums are exact and
 // order-free, so grad_p2 is the same on every run; each row is converted
 // back once.
-// CHECKED: the table's smallest terms decide whether fixed point holds them.
+// CHECKED: the table's smallest terms decide whether fixed point holds them;
+// double terms are then always summed in floating point (the fixed point holds
+// 52 bits below a bucket's largest term, a row of small ones would lose some,
+// and the table's float bits do not reach down to a double's smallest terms).
 template <typename T, bool CHECKED>
 __global__ __launch_bounds__(KB2_THREADS) void knn_bwd_bucket_kernel(
     const typename BwdAcc<T>::type* __restrict__ rec, const int4* __restrict__ tab, int P2, int D,
@@ -372,7 +374,8 @@ __global__ __launch_bounds__(KB2_THREADS) void knn_bwd_bucket_kernel(
   // with a smallest term given, fixed point only where it holds every term's
   // last bit (24 bits below the smallest term's exponent)
   const int e1 = CHECKED ? (int)((s_min >> 23) & 0xff) - 127 : 0;
-  if (mb < 0x7f800000u && (!CHECKED || (e1 < -126 ? -126 : e1) - 23 + S >= 0)) {
+  const bool fixed = !CHECKED || (sizeof(A) == 4 && (e1 < -126 ? -126 : e1) - 23 + S >= 0);
+  if (mb < 0x7f800000u && fixed) {
     if (mb != 0u) {
       const double scale = __builtin_ldexp(1.0, S);
       kb_for_records<A>(rec, t, n, cpc, D, [&](int row, const A (&v)[7]) {
@@ -386,7 +389,7 @@ __global__ __launch_bounds__(KB2_THREADS) void knn_bwd_bucket_kernel(
     __syncthreads();
     const double inv = __builtin_ldexp(1.0, -S);
     for (int e = tid; e < ns * D; e += KB2_THREADS) o[e] = (T)((double)(long long)acc[e] * inv);
-  } else {  // infinite, NaN or wide-ranged terms: sums in floating point (order unspecified)
+  } else {  // infinite, NaN, wide-ranged or double terms: floating point (order unspecified)
     A* __restrict__ fa = reinterpret_cast<A*>(s_dyn);
     for (int e = tid; e < ns * D; e += KB2_THREADS) fa[e] = (A)0;
     __syncthreads();
@@ -444,10 +447,8 @@ __global__ __launch_bounds__(KB1_THREADS) void knn_gather_bwd_entry_kernel(
     if (any) r = (int)(j < 0 ? 0 : (j >= M ? M - 1 : j));
   }
   __syncthreads();
-  // double terms are summed in floating point: the fixed point holds 52 bits
-  // below a bucket's largest term, a row of small ones would lose some
-  kb_group_records<T, A, DC, false>(t, r, U, n, c, cpc, R, nb, 1u, s_cnt, s_max,
-                             sizeof(A) == 4 ? s_min : nullptr, s_part, rec, tab);
+  kb_group_records<T, A, DC, false>(t, r, U, n, c, cpc, R, nb, s_cnt, s_max,
+                                    sizeof(A) == 4 ? s_min : nullptr, s_part, rec, tab);
 }
 
 // Any D and K: one wave per query row, lanes over the coordinates (64 at a
