@@ -164,3 +164,32 @@ def test_fake_kernels(tpo):
         assert cost.shape == (2,) and match.shape == (2, 7, 5) and match.dtype == a.dtype
         g1, g2 = torch.ops.torch_point_ops_emd.emd_backward(cost, a, b, match)
         assert g1.shape == a.shape and g2.shape == b.shape
+
+
+class _Gather(torch.nn.Module):
+    """A learned layer in front of a gather: autograd follows the traced call."""
+
+    def __init__(self, op):
+        super().__init__()
+        self.layer, self.op = torch.nn.Linear(4, 4), op
+
+    def forward(self, x, idx):
+        return self.op(self.layer(x), idx)
+
+
+@pytest.mark.parametrize("strict", [True, False])
+@pytest.mark.parametrize("name", ["gather_points", "knn_gather"])
+def test_gathers_export_with_a_dynamic_number_of_points(tpo, name, strict):
+    from torch.export import Dim, export
+
+    if name == "gather_points":
+        m = _Gather(lambda x, idx: tpo.gather_points(x.transpose(1, 2).contiguous(), idx))
+        idx = torch.randint(0, 50, (2, 7))
+    else:
+        m = _Gather(lambda x, idx: torch.ops.torch_point_ops_knn.knn_gather(
+            x, idx, torch.full((2,), 9)))
+        idx = torch.randint(0, 50, (2, 7, 3))
+    e = export(m, (torch.randn(2, 50, 4), idx), dynamic_shapes=({1: Dim("n", min=8, max=4096)}, None),
+               strict=strict)
+    x = next(n for n in e.graph.nodes if n.name == "x").meta["val"]
+    assert not isinstance(x.shape[1], int)

@@ -585,16 +585,16 @@ class KnnGatherFunction : public torch::autograd::Function<KnnGatherFunction> {
   static at::Tensor forward(AutogradContext* ctx, const at::Tensor& x, const at::Tensor& idx,
                             const at::Tensor& lengths) {
     ctx->save_for_backward({idx, lengths});
-    ctx->saved_data["M"] = x.sym_size(1).guard_int(__FILE__, __LINE__);
+    ctx->saved_data["M"] = x.sym_size(1);  // symbolic while a program is traced
     at::AutoDispatchBelowADInplaceOrView below;
     return knn_gather_op().call(x, idx, lengths);
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
     static auto op =
-        typed_op<at::Tensor(const at::Tensor&, const at::Tensor&, const at::Tensor&, int64_t)>(
+        typed_op<at::Tensor(const at::Tensor&, const at::Tensor&, const at::Tensor&, c10::SymInt)>(
             "torch_point_ops_knn::knn_gather_backward");
     const auto s = ctx->get_saved_variables();
-    const int64_t M = ctx->saved_data["M"].toInt();
+    const c10::SymInt M = ctx->saved_data["M"].toSymInt();
     if (at::GradMode::is_enabled())  // its own gradient is the gather (knn/__init__.py)
       return {op.call(grads[0], s[0], s[1], M), at::Tensor(), at::Tensor()};
     at::AutoDispatchBelowADInplaceOrView below;
@@ -695,7 +695,7 @@ class GatherPointsFunction : public torch::autograd::Function<GatherPointsFuncti
  public:
   static at::Tensor forward(AutogradContext* ctx, const at::Tensor& points, const at::Tensor& idx) {
     ctx->save_for_backward({idx});
-    ctx->saved_data["n"] = points.sym_size(2).guard_int(__FILE__, __LINE__);
+    ctx->saved_data["n"] = points.sym_size(2);  // symbolic while a program is traced
     at::AutoDispatchBelowADInplaceOrView below;
     return gather_points_op().call(points, idx);
   }
@@ -703,7 +703,8 @@ class GatherPointsFunction : public torch::autograd::Function<GatherPointsFuncti
     static auto op = typed_op<at::Tensor(const at::Tensor&, const at::Tensor&, int64_t)>(
         "torch_point_ops_fps::gather_points_backward");
     const auto s = ctx->get_saved_variables();
-    return {op.call(grads[0], s[0], ctx->saved_data["n"].toInt()), at::Tensor()};
+    const int64_t n = ctx->saved_data["n"].toSymInt().guard_int(__FILE__, __LINE__);  // the schema's int
+    return {op.call(grads[0], s[0], n), at::Tensor()};
   }
 };
 
@@ -823,7 +824,7 @@ TORCH_LIBRARY(torch_point_ops_knn, m) {
   m.def("knn_forward_sorted(Tensor p1, Tensor p2, Tensor lengths1, Tensor lengths2, "
         "int norm, int K, int version) -> (Tensor, Tensor)");
   m.def("knn_gather(Tensor x, Tensor idx, Tensor lengths) -> Tensor");
-  m.def("knn_gather_backward(Tensor grad_out, Tensor idx, Tensor lengths, int M) -> Tensor");
+  m.def("knn_gather_backward(Tensor grad_out, Tensor idx, Tensor lengths, SymInt M) -> Tensor");
 }
 TORCH_LIBRARY_IMPL(torch_point_ops_knn, CUDA, m) {
   m.impl("knn_forward", &knn_forward_hip);
