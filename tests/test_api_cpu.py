@@ -193,3 +193,24 @@ def test_gathers_export_with_a_dynamic_number_of_points(tpo, name, strict):
                strict=strict)
     x = next(n for n in e.graph.nodes if n.name == "x").meta["val"]
     assert not isinstance(x.shape[1], int)
+
+
+@pytest.mark.parametrize("strict", [True, False])
+@pytest.mark.parametrize("module", [False, True])
+def test_knn_exports_with_two_dynamic_lengths_of_equal_examples(tpo, module, strict):
+    from torch.export import Dim, export
+
+    class M(torch.nn.Module):
+        def forward(self, a, b):
+            if module:
+                return tpo.KNearestNeighbors(K=1)(a, b)
+            return tpo.knn_points(a, b, K=1)
+
+    a, b = torch.randn(2, 50, 3), torch.randn(2, 50, 3)
+    e = export(M(), (a, b), dynamic_shapes=({1: Dim("n", min=8, max=4096)},
+                                            {1: Dim("m", min=8, max=4096)}), strict=strict)
+    for n, m in ((50, 50), (60, 31)):
+        a, b = torch.randn(2, n, 3), torch.randn(2, m, 3)
+        got = e.module()(a, b)
+        want = tpo.knn_points(a, b, K=1)
+        assert torch.equal(got[0], want[0]) and torch.equal(got[1], want[1])

@@ -67,6 +67,12 @@ def _knn_backward_fake(p1, p2, lengths1, lengths2, idxs, norm, grad_dists):
     return torch.empty_like(p1), torch.empty_like(p2)
 
 
+def _same_size(a, b):
+    """Whether two sizes are known to be equal.  Only plain numbers outside a traced
+    program are compared: there the comparison would tie two sizes that may differ."""
+    return not torch.compiler.is_compiling() and type(a) is int and type(b) is int and a == b
+
+
 def knn_points(
     p1: torch.Tensor,
     p2: torch.Tensor,
@@ -99,7 +105,7 @@ def knn_points(
     # all points: one launch for both clouds where they are of one length
     if lengths2 is None:
         lengths2 = torch.full((N,), P2, dtype=torch.int64, device=p1.device)
-        if lengths1 is None and P1 == P2:
+        if lengths1 is None and _same_size(P1, P2):
             lengths1 = lengths2
     if lengths1 is None:
         lengths1 = torch.full((N,), P1, dtype=torch.int64, device=p1.device)

@@ -1,14 +1,15 @@
 """KNN modules (reference: torch_point_ops/knn/knn.py:5-135)."""
 import torch
 
-from . import knn_points
+from . import _same_size, knn_points
 
 
 def _whole(p1, p2, lengths1, lengths2):
     """The default lengths made once for the search and the gather behind it."""
     if lengths2 is None:
         lengths2 = torch.full((p2.shape[0],), p2.shape[1], dtype=torch.int64, device=p2.device)
-        if lengths1 is None and p1.shape[:2] == p2.shape[:2]:
+        if (lengths1 is None and _same_size(p1.shape[0], p2.shape[0])
+                and _same_size(p1.shape[1], p2.shape[1])):
             lengths1 = lengths2
     return lengths1, lengths2
 
