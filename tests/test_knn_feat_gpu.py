@@ -53,7 +53,7 @@ def test_feature_rows_match_the_reference_order(tpo, dev, D, P1, P2, K, case):
 
 
 @pytest.mark.parametrize("case", ["few_ties", "all_ties", "runs", "nonfinite_query",
-                                  "nonfinite_cloud", "huge", "tiny", "short", "far_cloud"])
+                                  "nonfinite_cloud", "nan_of_ones", "huge", "tiny", "short", "far_cloud"])
 @pytest.mark.parametrize("D,K", [(64, 20), (9, 5)])
 def test_feature_rows_replayed_and_edge_values(tpo, dev, case, D, K):
     g = torch.Generator().manual_seed(len(case) + D)
@@ -79,6 +79,11 @@ def test_feature_rows_replayed_and_edge_values(tpo, dev, case, D, K):
         p2[0, 5, 1] = float("inf")
         p2[1, 7, 1] = float("nan")
         p2[2, 0, 0] = float("nan")
+    elif case == "nan_of_ones":  # every bit set, with either sign (a difference flips it)
+        for bits, at in ((-1, 0), (0x7FFFFFFF, 1)):
+            p2.view(torch.int32)[1, 40 + at:60:2] = bits
+            p2.view(torch.int32)[1, 3 + at, 1] = bits
+            p2.view(torch.int32)[1, 700 + at] = bits
     elif case == "huge":  # distances that overflow to infinity
         p2[0, ::3] *= 1e25
         p1[1] *= 1e30

@@ -95,10 +95,14 @@ def _hd_inputs(case, g, D):
     else:
         p1 = torch.randn(N, P1, D, generator=g)
         p2 = torch.randn(N, P2, D, generator=g)
-    if case == "descending":  # every reference closer than all before it: lists overflow
+    if case.startswith("descending"):  # every reference closer than all before it: lists overflow
         r = p2.norm(dim=-1)
         p2 = torch.gather(p2, 1, r.argsort(dim=1, descending=True)[..., None].expand(-1, -1, D))
         p1 = p1 * 1e-3
+    if case == "descending_nan":  # NaNs of all ones, either sign, among the recomputed references
+        p2.view(torch.int32)[0, 9000:9010] = -1
+        p2.view(torch.int32)[0, 9010:9020] = 0x7FFFFFFF
+        p2.view(torch.int32)[1, 4000:7000:100, 3] = 0x7FFFFFFF
     if case == "nonfinite":
         p2[0, 0, 5] = float("nan")       # fill slot 0: the threshold is NaN, nothing is inserted
         p2[1, 3, 0] = float("nan")       # another fill slot: never the maximum
@@ -122,7 +126,7 @@ def _hd_inputs(case, g, D):
 
 
 @pytest.mark.parametrize("case", ["random", "lattice", "descending", "short", "nonfinite",
-                                  "duplicates"])
+                                  "duplicates", "descending_nan"])
 @pytest.mark.parametrize("D,K,norm", [(128, 32, 2), (128, 9, 1), (64, 16, 2)])
 def test_high_d_sliced_forward_bit_exact(tpo, O, dev, case, D, K, norm):
     g = torch.Generator().manual_seed(D + K + norm + len(case))

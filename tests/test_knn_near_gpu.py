@@ -65,7 +65,7 @@ def test_near_rows_match_the_reference_order(tpo, dev, P1, P2, K, kind, norm):
         assert torch.equal(si, ei)
 
 
-@pytest.mark.parametrize("case", ["few_ties", "lattice", "nonfinite_query", "nonfinite_cloud",
+@pytest.mark.parametrize("case", ["few_ties", "lattice", "nonfinite_query", "nonfinite_cloud", "nan_of_ones",
                                   "huge", "short", "one_point"])
 @pytest.mark.parametrize("P2,K", [(1500, 16), (6000, 5)])
 def test_near_rows_replayed_and_edge_values(tpo, dev, case, P2, K):
@@ -86,6 +86,11 @@ def test_near_rows_replayed_and_edge_values(tpo, dev, case, P2, K):
         p2[0, 5, 1] = float("inf")
         p2[1, 7, 1] = float("nan")
         p2[2, 0, 0] = float("nan")
+    elif case == "nan_of_ones":  # every bit set, with either sign (a difference flips it)
+        for bits, at in ((-1, 0), (0x7FFFFFFF, 1)):
+            p2.view(torch.int32)[1, 40 + at:60:2] = bits
+            p2.view(torch.int32)[1, 3 + at, 1] = bits
+            p2.view(torch.int32)[1, 700 + at] = bits
     elif case == "huge":
         p2[0, ::3] *= 1e25
         p1[1] *= 1e30

@@ -21,8 +21,11 @@
 namespace tpo {
 
 // A distance (>= +0, +inf or NaN) as an unsigned that orders like it; list
-// entries put NaN (0) below every number, candidates above.
-__device__ __forceinline__ uint32_t replay_ord(float v) { return __float_as_uint(v) + 1u; }
+// entries put NaN (0) below every number, candidates above: any NaN, whatever
+// its bits (0xffffffff + 1 would be the smallest key).
+__device__ __forceinline__ uint32_t replay_ord(float v) {
+  return v != v ? 0xffffffffu : __float_as_uint(v) + 1u;
+}
 __device__ __forceinline__ uint32_t replay_shr1(uint32_t x) {  // lane i takes lane i-1 (lane 0: 0)
   return (uint32_t)__builtin_amdgcn_mov_dpp((int)x, 0x138, 0xF, 0xF, true);
 }
