@@ -558,6 +558,31 @@ def torch_reference_knn(p1, p2, K):
     return si[..., :K], sd[..., :K]
 
 
+@pytest.mark.parametrize("exponent", [-100, -140, -200, -400])
+def test_backward_of_small_double_distances(tpo, dev, exponent):
+    """Double coordinates far below the float range: scaling them by a power of
+    two scales the gradients by it, up to the order of the sums."""
+    g = torch.Generator().manual_seed(3)
+    N, P1, P2, K = 2, 300, 40, 5
+    p1 = torch.randn(N, P1, 3, generator=g, dtype=torch.float64)
+    p2 = torch.randn(N, P2, 3, generator=g, dtype=torch.float64)
+    idx = torch.randint(0, P2, (N, P1, K), generator=g)
+    gd = torch.randn(N, P1, K, generator=g, dtype=torch.float64)
+    l1, l2 = torch.full((N,), P1), torch.full((N,), P2)
+    scale = 2.0 ** exponent
+    g1, g2 = torch.ops.torch_point_ops_knn.knn_backward(
+        (p1 * scale).to(dev), (p2 * scale).to(dev), l1.to(dev), l2.to(dev), idx.to(dev), 2, gd.to(dev))
+    flat = idx.reshape(N, P1 * K, 1).expand(-1, -1, 3)
+    t = 2 * gd[..., None] * (p1[:, :, None] - torch.gather(p2, 1, flat).reshape(N, P1, K, 3))
+    want = torch.zeros_like(p2).scatter_add(1, flat, -t.reshape(N, P1 * K, 3))
+    mass = torch.zeros_like(p2).scatter_add(1, flat, t.abs().reshape(N, P1 * K, 3))
+    # a term's own roundings, and those of a sum of at most P1 K terms in any order
+    # (fixed point keeps 51 bits below the largest of all)
+    bound = (P1 * K + 4) * 2.0 ** -53 * mass + P1 * K * 2.0 ** -51 * t.abs().max()
+    assert ((g2.cpu() / scale - want).abs() <= bound).all()
+    assert ((g1.cpu() / scale - t.sum(2)).abs() <= (K + 4) * 2.0 ** -53 * t.abs().sum(2)).all()
+
+
 def test_reference_forward_and_known_values(tpo, dev):
     g = torch.Generator().manual_seed(0)
     p1 = torch.randn(2, 10, 3, generator=g).to(dev)

@@ -319,7 +319,8 @@ __device__ __forceinline__ void kb_for_records(const A* __restrict__ rec,
 // int64 range; each term is rounded to nearest on conversion (exact for
 // float terms within ~2^28 of the largest).  Integer sums are exact and
 // order-free, so grad_p2 is the same on every run; each row is converted
-// back once.
+// back once.  Double terms all below the smallest normal float, where the
+// table's float bits say little or nothing (0), are summed in floating point.
 // CHECKED: the table's smallest terms decide whether fixed point holds them;
 // double terms are then always summed in floating point (the fixed point holds
 // 52 bits below a bucket's largest term, a row of small ones would lose some,
@@ -374,7 +375,8 @@ __global__ __launch_bounds__(KB2_THREADS) void knn_bwd_bucket_kernel(
   // with a smallest term given, fixed point only where it holds every term's
   // last bit (24 bits below the smallest term's exponent)
   const int e1 = CHECKED ? (int)((s_min >> 23) & 0xff) - 127 : 0;
-  const bool fixed = !CHECKED || (sizeof(A) == 4 && (e1 < -126 ? -126 : e1) - 23 + S >= 0);
+  const bool fixed = CHECKED ? sizeof(A) == 4 && (e1 < -126 ? -126 : e1) - 23 + S >= 0
+                             : sizeof(A) == 4 || mb >= 0x00800000u;
   if (mb < 0x7f800000u && fixed) {
     if (mb != 0u) {
       const double scale = __builtin_ldexp(1.0, S);
