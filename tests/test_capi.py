@@ -146,3 +146,19 @@ def test_emd_sizes_and_errors(lib):
     assert lib.tpo_emd_bwd(0, None, None, None, None, 1, 4, 4, None, None, None, 0, None) == -4
     assert lib.tpo_emd_bwd(0, None, None, None, None, 1 << 31, 4, 4, None, None, None, 0,
                            None) == -1
+
+
+@pytest.mark.parametrize("K", [1, 4, 16, 32])
+def test_knn_rows_workspace_is_in_proportion_to_the_points(lib, K):
+    """Many short clouds do not take a fixed table each."""
+    I = ctypes.c_int64
+    for f in (lib.tpo_knn_rows_workspace_size, lib.tpo_knn_workspace_size):
+        f.argtypes = [ctypes.c_int, I, I, I, I, I, ctypes.c_int]
+        f.restype = I
+    for N, P1, P2 in ((1, 1, 512), (64, 1, 128), (32768, 1, 512), (65536, 1, 1024), (4096, 32, 2048),
+                      (16, 2048, 2048), (8, 16384, 16384), (1, 1 << 18, 1 << 18)):
+        rows = lib.tpo_knn_rows_workspace_size(0, N, P1, P2, 3, K, 2)
+        base = lib.tpo_knn_workspace_size(0, N, P1, P2, 3, K, 2)
+        # a record of 16 bytes a point, 8 bytes a query of rows left to replay, and
+        # the starts of at most eight cells a reference
+        assert base <= rows <= max(base, N * (P2 * (16 + 32) + P1 * 24 + 64) + 4096)

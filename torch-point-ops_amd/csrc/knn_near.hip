@@ -43,7 +43,14 @@ namespace tpo {
 namespace {
 
 constexpr int KN_GMAX = 32;
-constexpr int KN_CELLS = KN_GMAX * KN_GMAX * KN_GMAX;
+// Cells an axis at most for a cloud of P2 references: no more than eight cells a
+// reference, so that many short clouds do not take a whole table each (32
+// cells an axis are 131 KB).
+inline int kn_gmax(int64_t P2) {
+  int g = 8;
+  while (g < KN_GMAX && (int64_t)(g + 1) * (g + 1) * (g + 1) <= 8 * P2) ++g;
+  return g;
+}
 constexpr int KN_WAVES = 4;
 constexpr int KN_PPT = 16;  // clouds of up to 1024 KN_PPT points stay in registers in the setup
 
@@ -100,7 +107,7 @@ struct KnLds {
 // 1024 PPT points, loaded once, each placed by the rank its cell's counter
 // returned; otherwise streamed PPT points a thread at a time.
 template <bool QUERIES, bool HELD, int PPT>
-__device__ void kn_bin(const float* __restrict__ P, int L, int K, float* __restrict__ hdr,
+__device__ void kn_bin(const float* __restrict__ P, int L, int K, int gmax, float* __restrict__ hdr,
                        int32_t* __restrict__ cs, float4* __restrict__ out, KnLds& sm) {
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const float inf = Lim<float>::inf();
@@ -207,7 +214,7 @@ __device__ void kn_bin(const float* __restrict__ P, int L, int K, float* __restr
     const float want = fmaxf(2.f, 0.18f * (float)K);
     const float ratio = (float)L / ((float)max(o, 1) * want);
     G = (int)(16.f * __builtin_exp2f(__builtin_log2f(fmaxf(ratio, 1e-6f)) * (1.f / 2.3f)));
-    G = min(max(G, 2), KN_GMAX);
+    G = min(max(G, 2), gmax);
     scale(G, gs);
     if (tid < 3) {
       hdr[tid] = glo[tid];
@@ -288,7 +295,7 @@ __device__ void kn_bin(const float* __restrict__ P, int L, int K, float* __restr
 __global__ __launch_bounds__(1024) void knn_near_setup_kernel(
     const float* __restrict__ p1, const int64_t* __restrict__ len1, int P1,
     const float* __restrict__ p2, const int64_t* __restrict__ len2, int P2, int N, int K,
-    float* __restrict__ hdr, int32_t* __restrict__ cstart, float4* __restrict__ rrec,
+    int gmax, float* __restrict__ hdr, int32_t* __restrict__ cstart, float4* __restrict__ rrec,
     float4* __restrict__ qrec, uint32_t* __restrict__ redo_counts) {
   __shared__ KnLds sm;
   if (blockIdx.x == 0)
@@ -299,9 +306,9 @@ __global__ __launch_bounds__(1024) void knn_near_setup_kernel(
     const int L1 = (int)(l1 < 0 ? 0 : (l1 > P1 ? P1 : l1));
     float4* __restrict__ out = qrec + (size_t)n * P1;
     const float* p = p1 + (size_t)n * P1 * 3;
-    if (L1 <= 4096) kn_bin<true, true, 4>(p, L1, K, nullptr, nullptr, out, sm);
-    else if (L1 <= 1024 * KN_PPT) kn_bin<true, true, KN_PPT>(p, L1, K, nullptr, nullptr, out, sm);
-    else kn_bin<true, false, 4>(p, L1, K, nullptr, nullptr, out, sm);
+    if (L1 <= 4096) kn_bin<true, true, 4>(p, L1, K, gmax, nullptr, nullptr, out, sm);
+    else if (L1 <= 1024 * KN_PPT) kn_bin<true, true, KN_PPT>(p, L1, K, gmax, nullptr, nullptr, out, sm);
+    else kn_bin<true, false, 4>(p, L1, K, gmax, nullptr, nullptr, out, sm);
     for (int k = L1 + (int)threadIdx.x; k < P1; k += 1024)  // rows past lengths1 keep their place
       out[k] = make_float4(0.f, 0.f, 0.f, __int_as_float(k));
   } else {
@@ -310,11 +317,11 @@ __global__ __launch_bounds__(1024) void knn_near_setup_kernel(
     const int L2 = (int)(l2 < 0 ? 0 : (l2 > P2 ? P2 : l2));
     const float* p = p2 + (size_t)n * P2 * 3;
     float* h = hdr + (size_t)n * KG_HDR;
-    int32_t* cs = cstart + (size_t)n * (KN_CELLS + 1);
+    int32_t* cs = cstart + (size_t)n * (gmax * gmax * gmax + 1);
     float4* out = rrec + (size_t)n * P2;
-    if (L2 <= 4096) kn_bin<false, true, 4>(p, L2, K, h, cs, out, sm);
-    else if (L2 <= 1024 * KN_PPT) kn_bin<false, true, KN_PPT>(p, L2, K, h, cs, out, sm);
-    else kn_bin<false, false, 4>(p, L2, K, h, cs, out, sm);
+    if (L2 <= 4096) kn_bin<false, true, 4>(p, L2, K, gmax, h, cs, out, sm);
+    else if (L2 <= 1024 * KN_PPT) kn_bin<false, true, KN_PPT>(p, L2, K, gmax, h, cs, out, sm);
+    else kn_bin<false, false, 4>(p, L2, K, gmax, h, cs, out, sm);
   }
 }
 
@@ -398,8 +405,8 @@ __global__ __launch_bounds__(256) void knn_near_kernel(
     const int64_t* __restrict__ len1, const int64_t* __restrict__ len2,
     const float* __restrict__ hdr, const int32_t* __restrict__ cstart,
     const float4* __restrict__ rrec, const float* __restrict__ p1,
-    const float4* __restrict__ qrec, int P1, int P2, int K, int nqb, int pad_sentinel, RedoList redo, int64_t* __restrict__ idxs,
-    float* __restrict__ dists) {
+    const float4* __restrict__ qrec, int cells_max, int P1, int P2, int K, int nqb,
+    int pad_sentinel, RedoList redo, int64_t* __restrict__ idxs, float* __restrict__ dists) {
   __shared__ int32_t s_list[KN_WAVES * 4][KN_LIST];
   const int w = wave_id(), lane = lane_id(), l16 = lane & 15, g = lane >> 4;
   const int blk = xcd_logical_block(blockIdx.x, gridDim.x);  // a cloud's blocks share an XCD's L2
@@ -432,7 +439,7 @@ __global__ __launch_bounds__(256) void knn_near_kernel(
   if (__ballot(act) != 0 && L2 > 0) {
     const float* __restrict__ h = hdr + (size_t)n * KG_HDR;
     const int G = __float_as_int(h[6]);
-    const int32_t* __restrict__ cs = cstart + (size_t)n * (KN_CELLS + 1);
+    const int32_t* __restrict__ cs = cstart + (size_t)n * (cells_max + 1);
     const float4* __restrict__ rr = rrec + (size_t)n * P2;
     const bool fin = __float_as_int(h[7]) == 0 && __builtin_fabsf(qr[0]) < inf &&
                      __builtin_fabsf(qr[1]) < inf && __builtin_fabsf(qr[2]) < inf;
@@ -611,7 +618,8 @@ KnLayout kn_layout(int64_t N, int64_t P1, int64_t P2) {
   KnLayout L;
   L.hdr = 0;
   L.cstart = up(N * KG_HDR * 4);
-  L.rrec = L.cstart + up(N * (KN_CELLS + 1) * 4);
+  const int64_t g = kn_gmax(P2);
+  L.rrec = L.cstart + up(N * (g * g * g + 1) * 4);
   L.qrec = L.rrec + up(N * P2 * 16);
   L.redo = L.qrec + up(N * P1 * 16);
   L.total = L.redo + redo_bytes(N, P1);
@@ -664,12 +672,14 @@ RedoList launch_knn_near(const void* p1, const void* p2, const int64_t* l1, cons
   // references would hold the setup up (23 against 10 us at 8 x 16384 x 1024,
   // for 34 against 36 us).
   const bool order = P1 <= P2;
+  const int gmax = kn_gmax(P2), cells_max = gmax * gmax * gmax;
   hipLaunchKernelGGL(knn_near_setup_kernel, dim3(order ? 2 * N : N), dim3(1024), 0, s, (const float*)p1, l1, P1,
-                     (const float*)p2, l2, P2, N, K, hdr, cs, rrec, qrec, redo.total);
+                     (const float*)p2, l2, P2, N, K, gmax, hdr, cs, rrec, qrec, redo.total);
   const int nqb = (P1 + 4 * KN_WAVES - 1) / (4 * KN_WAVES);
 #define KNN_NEAR(NORM, R)                                                                        \
   hipLaunchKernelGGL((knn_near_kernel<NORM, R>), dim3(N * nqb), dim3(256), 0, s, l1, l2, hdr, cs, \
-                     rrec, (const float*)p1, order ? qrec : nullptr, P1, P2, K, nqb, pad, redo, idxs, (float*)dists)
+                     rrec, (const float*)p1, order ? qrec : nullptr, cells_max, P1, P2, K, nqb, pad, redo,    \
+                     idxs, (float*)dists)
 #define KNN_NEAR_K(NORM)                \
   do {                                  \
     if (!sort) KNN_NEAR(NORM, 0);       \
@@ -682,7 +692,7 @@ RedoList launch_knn_near(const void* p1, const void* p2, const int64_t* l1, cons
 #undef KNN_NEAR
   launch_knn_redo(p1, p2, l1, l2, N, P1, P2, 3, K, norm, pad, sort, redo, idxs, dists, s);
   if (grid_redo)
-    launch_knn_grid_redo(p1, p2, l1, l2, N, P1, P2, K, norm, pad, hdr, cs, KN_CELLS,
+    launch_knn_grid_redo(p1, p2, l1, l2, N, P1, P2, K, norm, pad, hdr, cs, cells_max,
                          (const float*)rrec, redo, idxs, dists, s);
   return redo;
 }
