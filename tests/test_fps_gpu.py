@@ -66,11 +66,12 @@ def test_fps_held_sizes_vs_oracle(tpo, O, dev, dtype, N):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16])
 @pytest.mark.parametrize("N,m", [(8193, 2000), (9000, 9000), (20000, 700), (65535, 300)])
-@pytest.mark.parametrize("kind", ["random", "lattice", "clusters", "sparse"])
+@pytest.mark.parametrize("kind", ["random", "lattice", "clusters", "sparse", "lattice_then_random"])
 def test_fps_rounds_vs_oracle(tpo, O, dev, dtype, N, m, kind):
     """Several samples a round: random clouds, lattices (every value tied),
     clusters with copies (values fall to 0 long before the last sample) and
-    clouds of which few points take part, also with every point sampled."""
+    clouds of which few points take part, also with every point sampled; a wide
+    lattice about a random part (samples one by one, then rounds again)."""
     if m > 3000 and kind == "random" and dtype == torch.float16:
         m = 3000
     g = torch.Generator().manual_seed(N + m)
@@ -80,6 +81,8 @@ def test_fps_rounds_vs_oracle(tpo, O, dev, dtype, N, m, kind):
     elif kind == "clusters":
         c = torch.randn(2, 40, 3, generator=g)
         p = c[:, torch.randint(0, 40, (N,), generator=g)] + 1e-2 * p.round(decimals=1)
+    elif kind == "lattice_then_random":
+        p[:, ::2] = torch.randint(-2, 3, p[:, ::2].shape, generator=g).float() * 8
     elif kind == "sparse":
         p[:, 50:] *= 1e-3
         p[0] *= 1e-3

@@ -44,9 +44,11 @@
 // unknown and waits.  All of a round's samples are then applied to each
 // bucket they touch in one visit.  At 65536 points a round chooses 7.9
 // samples on average (4.2 with one candidate a wave): 16 x 65536 -> 4096
-// takes 2.62 ms against 4.49 ms a sample at a time, 16 x 16384 -> 1024 0.70
+// takes 2.65 ms against 4.49 ms a sample at a time, 16 x 16384 -> 1024 0.70
 // against 1.08 ms.  Bound: VALU issue, about 1000 instructions a sample over
-// the 16 waves (box tests 250, visits 400, the rest per round).
+// the 16 waves (box tests 250, visits 400, the rest per round).  Where rounds
+// keep choosing one sample (equal running minima), stretches of samples are
+// taken one by one (FPS_WINDOW).
 //
 // Small clouds: fps_held_kernel.
 #include "tpo_common.hpp"
@@ -246,6 +248,25 @@ __device__ __forceinline__ void fps_decode(int64_t* __restrict__ out, int m, int
   }
 }
 
+// Rounds that choose few samples cost more than the samples one by one (a
+// second barrier and the candidates' test), where many running minima are
+// equal: lattices, repeated points, half values.  After a window of rounds
+// with under 1.5 samples a round on average the next `hold` samples are taken
+// one by one, twice as many after each further such window.  16 x 65536 -> 4096
+// points of a 16^3 lattice: 4.34 ms, all in rounds 7.53, one by one 4.47; drawn
+// from 32768 points 3.26 / 6.12 / 3.45; random 2.65 / 2.62 / 4.49.
+constexpr int FPS_WINDOW = 8, FPS_WINDOW_MIN = 12, FPS_HOLD = 32;
+
+__device__ __forceinline__ void fps_clear_slots(unsigned long long* s_gkey, uint32_t* s_tau,
+                                                int tid) {
+  __syncthreads();
+  if (tid < 3) {
+    s_gkey[tid] = 0;
+    s_tau[tid] = 0;
+  }
+  __syncthreads();
+}
+
 // ROUNDS (float and half, buckets of 64 points): several samples a round, see
 // the file header.
 template <typename T, bool ROUNDS>
@@ -270,7 +291,7 @@ __global__ __launch_bounds__(FPS_THREADS) void fps_kernel(const T* __restrict__ 
   const int b = blockIdx.x;
   const int tid = threadIdx.x, lane = lane_id(), w = wave_id();
   const FpsLayout L = fps_layout<T>(N);
-  const int s_sz = (int)(64 * ((N + 64 * FPS_THREADS - 1) / (64 * FPS_THREADS)));
+  const int s_sz = ROUNDS ? 64 : (int)(64 * ((N + 64 * FPS_THREADS - 1) / (64 * FPS_THREADS)));
   const int nb = (N + s_sz - 1) / s_sz;
   char* base = ws + (size_t)b * L.stride;
   FpsRec<T>* __restrict__ recs = (FpsRec<T>*)(base + L.off_r);
@@ -432,14 +453,9 @@ __global__ __launch_bounds__(FPS_THREADS) void fps_kernel(const T* __restrict__ 
     }
     }
   }
-  // the wave's best bucket (uniform)
-  int wlane;
-  C wbest = wave_best_at(bbest, wlane);
-
   // ---- 4. the sampling loop ----
   T ox = p0x, oy = p0y, oz = p0z;
   if (tid == 0) out[0] = 0;
-  int rk = 0;  // wave 0: lane j mod 64 holds the rank of sample j
   // A bucket is visited only when the squared distance from the new sample to
   // its box is at most reach = max(best * (1 + 2 margin), tiny); beyond it the
   // sample is provably farther from every point in the bucket than that
@@ -450,299 +466,325 @@ __global__ __launch_bounds__(FPS_THREADS) void fps_kernel(const T* __restrict__ 
   const V tiny = (V)FpsConst<T>::tiny();
   auto reach_of = [&](C c) -> V { return cand_valid(c) ? vmax((V)cand_val(c) * grow, tiny) : (V)-1; };
   V reach = reach_of(bbest);
-  if constexpr (ROUNDS) {
-    // Candidate i of the round: the better (i even) or second (odd) bucket
-    // best of wave i / 2; lanes i and i + 32 of every wave hold it.
-    uint64_t ck = 0;
-    float cx = 0.f, cy = 0.f, cz = 0.f;
-    uint32_t pm = 0;  // the candidates that are the last round's samples
-    int done = 1;     // samples chosen so far
-    int l1 = wlane, l2 = 0;
-    C w2 = cand_none(ctag);
-    uint32_t third = 0;
-    bool changed = true;
-    for (int rd = 0;; ++rd) {
-      if (pm != 0) {
-        // buckets within reach of a sample, a bit a sample
-        uint32_t hm = 0;
-        for (uint32_t mk = pm; mk != 0; mk &= mk - 1) {
-          const int i = __builtin_ctz(mk);
-          const float o3[3] = {bcast(cx, i), bcast(cy, i), bcast(cz, i)};
-          V e[3];
+  int done = 1;  // samples chosen so far
+  int hold = FPS_HOLD;
+  for (bool again = false;; again = true) {
+    int wlane;
+    if constexpr (ROUNDS) {
+      // Candidate i of the round: the better (i even) or second (odd) bucket
+      // best of wave i / 2; lanes i and i + 32 of every wave hold it.
+      uint64_t ck = 0;
+      float cx = (float)ox, cy = (float)oy, cz = (float)oz;
+      uint32_t pm = again ? 1u : 0u;  // the candidates that are the last round's samples
+      int l1 = 0, l2 = 0;
+      C w2 = cand_none(ctag);
+      uint32_t third = 0;
+      bool changed = true;
+      int window = 0, since = done;  // rounds of the present window, samples before it
+      if (again) fps_clear_slots(s_gkey, s_tau, tid);
+      for (int rd = 0;; ++rd) {
+        if (pm != 0) {
+          // buckets within reach of a sample, a bit a sample
+          uint32_t hm = 0;
+          for (uint32_t mk = pm; mk != 0; mk &= mk - 1) {
+            const int i = __builtin_ctz(mk);
+            const float o3[3] = {bcast(cx, i), bcast(cy, i), bcast(cz, i)};
+            V e[3];
 #pragma unroll
-          for (int c = 0; c < 3; ++c) e[c] = vmax(vmax(blo[c] - o3[c], o3[c] - bhi[c]), (V)0);
-          const V lb2 = vfma(e[2], e[2], vfma(e[1], e[1], e[0] * e[0]));
-          hm |= lb2 <= reach ? 1u << i : 0u;
+            for (int c = 0; c < 3; ++c) e[c] = vmax(vmax(blo[c] - o3[c], o3[c] - bhi[c]), (V)0);
+            const V lb2 = vfma(e[2], e[2], vfma(e[1], e[1], e[0] * e[0]));
+            hm |= lb2 <= reach ? 1u << i : 0u;
+          }
+          uint64_t tm = __ballot(hm != 0);
+          auto visit = [&](auto nbc) {  // as below, each bucket for all its samples
+            constexpr int NB = decltype(nbc)::value;
+            int bu[NB], pos[NB];
+            FpsRec<T> rc[NB];
+            T t[NB], t2[NB];
+#pragma unroll
+            for (int u = 0; u < NB; ++u) {
+              bu[u] = __builtin_ctzll(tm);
+              tm &= tm - 1;
+              pos[u] = (bu[u] * FPS_WAVES + w) * 64 + lane;
+              rc[u] = recs[pos[u]];
+              t[u] = ts[pos[u]];
+            }
+#pragma unroll
+            for (int u = 0; u < NB; ++u) {
+              t2[u] = t[u];
+              uint32_t mk = (uint32_t)__builtin_amdgcn_readlane((int)hm, bu[u]);
+              do {
+                const int i = __builtin_ctz(mk);
+                mk &= mk - 1;
+                const T ox = (T)bcast(cx, i), oy = (T)bcast(cy, i), oz = (T)bcast(cz, i);
+                const T d = sq3((T)(rc[u].x - ox), (T)(rc[u].y - oy), (T)(rc[u].z - oz));  // fps.cu:145
+                t2[u] = d < t2[u] ? d : t2[u];                                              // fps.cu:146
+              } while (mk != 0);
+            }
+#pragma unroll
+            for (int u = 0; u < NB; ++u) {
+              // re-reduced only when its best point's own running minimum dropped
+              const uint32_t bkey = (uint32_t)__builtin_amdgcn_readlane((int)cand_keyword(bbest), bu[u]);
+              if (__ballot(rc[u].key == bkey && t2[u] != t[u]) == 0) continue;
+              int wl;
+              const C cand = cand_make((V)t2[u], rc[u].key, ctag);
+              const C best = wave_best_at(cand, wl);
+              const uint32_t second = wave_umax(lane == wl ? 0u : __float_as_uint((float)t2[u]));
+              const T nx = bcast(rc[u].x, wl), ny = bcast(rc[u].y, wl), nz = bcast(rc[u].z, wl);
+              if (lane == bu[u]) {
+                bbest = best;
+                bsec = (V)__uint_as_float(second);
+                bx = nx;
+                by = ny;
+                bz = nz;
+              }
+              changed = true;
+            }
+#pragma unroll
+            for (int u = 0; u < NB; ++u)
+              if (t2[u] != t[u]) ts[pos[u]] = t2[u];
+          };
+          while (tm) {
+            const int nt = __builtin_popcountll(tm);
+            if (nt == 1) visit(std::integral_constant<int, 1>{});
+            else if (nt == 2) visit(std::integral_constant<int, 2>{});
+            else if (nt == 3) visit(std::integral_constant<int, 3>{});
+            else if (nt <= 5) visit(std::integral_constant<int, 4>{});
+            else visit(std::integral_constant<int, 6>{});
+          }
+          reach = reach_of(bbest);
         }
-        uint64_t tm = __ballot(hm != 0);
-        auto visit = [&](auto nbc) {  // as below, each bucket for all its samples
-          constexpr int NB = decltype(nbc)::value;
-          int bu[NB], pos[NB];
+        if (window == FPS_WINDOW) {
+          if (done - since < FPS_WINDOW_MIN) break;  // every chosen sample is applied here
+          window = 0;
+          since = done;
+          hold = FPS_HOLD;
+        }
+        ++window;
+        if (changed) {  // the wave's two best buckets, and a bound on everything else in it
+          changed = false;
+          (void)wave_best_at(bbest, l1);
+          const C rest = lane == l1 ? cand_none(ctag) : bbest;
+          w2 = wave_best_at(rest, l2);
+          const bool pub = lane == l1 || (lane == l2 && cand_valid(w2));
+          third = wave_umax(__float_as_uint(pub ? (float)bsec : (float)cand_val(bbest)));
+        }
+        const int par = rd & 1;
+        if (lane == l1) {
+          s_ck[par][2 * w] = bbest.k;
+          s_cp[par][2 * w] = make_float4((float)bx, (float)by, (float)bz, 0.f);
+        }
+        // (a wave without a second bucket publishes no candidate there)
+        if (lane == (cand_valid(w2) ? l2 : (l1 ^ 1))) {
+          s_ck[par][2 * w + 1] = cand_valid(w2) ? bbest.k : 0ull;
+          s_cp[par][2 * w + 1] = make_float4((float)bx, (float)by, (float)bz, 0.f);
+        }
+        // three slots in turn: the next round's are cleared here, after their
+        // last readers (before the first barrier of this round)
+        if (lane == 0) atomicMax(&s_tau[rd % 3], third);
+        if (tid == 0) {
+          s_tau[(rd + 1) % 3] = 0;
+          s_gkey[(rd + 1) % 3] = 0;
+        }
+        __syncthreads();
+        // candidate j is out of order when one with a larger key lowers its
+        // running minimum, or would not lower its own (infinite coordinates:
+        // it is chosen again and again): wave w tests its two, a lane a pair
+        {
+          const int j = 2 * w + (lane >> 5);
+          ck = s_ck[par][lane & 31];
+          const float4 ci = s_cp[par][lane & 31];
+          const uint64_t kj = s_ck[par][j];
+          const float4 cj = s_cp[par][j];
+          cx = ci.x;
+          cy = ci.y;
+          cz = ci.z;
+          const T d = sq3((T)((T)cj.x - (T)ci.x), (T)((T)cj.y - (T)ci.y), (T)((T)cj.z - (T)ci.z));
+          const bool stays = !((ci.x - ci.x) + (ci.y - ci.y) + (ci.z - ci.z) == 0.f);
+          const uint64_t hit = __ballot(
+              ck > kj && kj != 0 && (stays || (float)d < __uint_as_float((uint32_t)(kj >> 32))));
+          if ((lane & 31) == 0 && (uint32_t)(hit >> lane) != 0)
+            atomicMax(&s_gkey[rd % 3], (unsigned long long)kj);
+        }
+        __syncthreads();
+        // this round's samples: the candidates above every such one, and above
+        // every other point's value
+        const uint64_t out_of = s_gkey[rd % 3];
+        const uint64_t others = (uint64_t)s_tau[rd % 3] << 32 | 0xffffffffull;
+        const uint64_t floor_key = out_of > others ? out_of : others;
+        pm = (uint32_t)__ballot(ck > floor_key);
+        if (pm == 0) {  // only the largest is certain
+          int gl;
+          const C g = wave_best_at(C{ck}, gl);
+          if (!cand_valid(g)) {  // nothing takes part: index 0 from here on (rank -1)
+            for (int j = done + tid; j < m; j += FPS_THREADS) out[j] = -1;
+            done = m;
+            break;
+          }
+          pm = 1u << gl;
+        }
+        if (w == 0) {  // in key order
+          int at = done;
+          for (uint32_t mk = pm; mk != 0; mk &= mk - 1) {
+            const int i = __builtin_ctz(mk);
+            const uint64_t k = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(ck >> 32), i) << 32 |
+                               (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)ck, i);
+            at += k > ck ? 1 : 0;
+          }
+          if (lane < 32 && (pm >> lane) & 1 && at < m) out[at] = (int64_t)(0xffffffffu - (uint32_t)ck);
+        }
+        done += __builtin_popcount(pm);
+        if (done >= m) break;
+      }
+      if (done >= m) break;
+      fps_clear_slots(s_gkey, s_tau, tid);
+      ox = oy = oz = (T)0;  // (applied)
+    }
+    C wbest = wave_best_at(bbest, wlane);  // the wave's best bucket (uniform)
+    const int from = done, to = ROUNDS ? min(m, done + hold) : m;
+    int rk = 0;  // wave 0: lane j mod 64 holds the rank of sample j
+    for (int j = from; j < to; ++j) {
+      const V o3[3] = {(V)ox, (V)oy, (V)oz};
+      V e[3];
+#pragma unroll
+      for (int c = 0; c < 3; ++c) e[c] = vmax(vmax(blo[c] - o3[c], o3[c] - bhi[c]), (V)0);
+      const V lb2 = vfma(e[2], e[2], vfma(e[1], e[1], e[0] * e[0]));
+      // the first sample's updates were made while the cloud was set up (or by
+      // the round before)
+      uint64_t tm = j > from ? __ballot(lb2 <= reach) : 0;
+      bool rereduce = false;  // the best of the wave's best bucket changed
+      // Touched buckets are visited NB at a time: every slot's loads are issued
+      // first (the rounds below never leave a slot empty; an empty slot would
+      // re-read slot 0's bucket), the NB wave reductions are independent
+      // straight-line code, and the running-minimum stores come last, so no load
+      // or reduction of the batch waits for a store.
+      auto visit = [&](auto nbc) {
+        constexpr int NB = decltype(nbc)::value;
+        int bits[NB];
+#pragma unroll
+        for (int u = 0; u < NB; ++u) {
+          bits[u] = tm ? __builtin_ctzll(tm) : -1;
+          tm &= tm ? tm - 1 : 0;
+        }
+        for (int p0 = 0; p0 < s_sz; p0 += 64) {
+          int pos[NB];
           FpsRec<T> rc[NB];
-          T t[NB], t2[NB];
+          T t[NB];
 #pragma unroll
           for (int u = 0; u < NB; ++u) {
-            bu[u] = __builtin_ctzll(tm);
-            tm &= tm - 1;
-            pos[u] = (bu[u] * FPS_WAVES + w) * 64 + lane;
+            const int bu = bits[u] >= 0 ? bits[u] : bits[0];
+            pos[u] = (bu * FPS_WAVES + w) * s_sz + p0 + lane;
             rc[u] = recs[pos[u]];
             t[u] = ts[pos[u]];
           }
+          T t2[NB];
+          C cand[NB];
 #pragma unroll
           for (int u = 0; u < NB; ++u) {
-            t2[u] = t[u];
-            uint32_t mk = (uint32_t)__builtin_amdgcn_readlane((int)hm, bu[u]);
-            do {
-              const int i = __builtin_ctz(mk);
-              mk &= mk - 1;
-              const T ox = (T)bcast(cx, i), oy = (T)bcast(cy, i), oz = (T)bcast(cz, i);
-              const T d = sq3((T)(rc[u].x - ox), (T)(rc[u].y - oy), (T)(rc[u].z - oz));  // fps.cu:145
-              t2[u] = d < t2[u] ? d : t2[u];                                              // fps.cu:146
-            } while (mk != 0);
+            const T d = sq3((T)(rc[u].x - ox), (T)(rc[u].y - oy), (T)(rc[u].z - oz));  // fps.cu:145
+            t2[u] = d < t[u] ? d : t[u];                                                // fps.cu:146
+            cand[u] = cand_make((V)t2[u], rc[u].key, ctag);
+          }
+          // A bucket's best stays its best unless that point's own running
+          // minimum dropped (the others can only drop too), so the reduction
+          // runs only then (always for buckets larger than 64 points).
+          bool red[NB];
+#pragma unroll
+          for (int u = 0; u < NB; ++u) {
+            const int bu = bits[u] >= 0 ? bits[u] : bits[0];
+            const uint32_t bkey = (uint32_t)__builtin_amdgcn_readlane((int)cand_keyword(bbest), bu);
+            red[u] = bits[u] >= 0 && (s_sz > 64 || __ballot(rc[u].key == bkey && t2[u] != t[u]) != 0);
           }
 #pragma unroll
           for (int u = 0; u < NB; ++u) {
-            // re-reduced only when its best point's own running minimum dropped
-            const uint32_t bkey = (uint32_t)__builtin_amdgcn_readlane((int)cand_keyword(bbest), bu[u]);
-            if (__ballot(rc[u].key == bkey && t2[u] != t[u]) == 0) continue;
+            if (!red[u]) continue;
             int wl;
-            const C cand = cand_make((V)t2[u], rc[u].key, ctag);
-            const C best = wave_best_at(cand, wl);
-            const uint32_t second = wave_umax(lane == wl ? 0u : __float_as_uint((float)t2[u]));
-            const T nx = bcast(rc[u].x, wl), ny = bcast(rc[u].y, wl), nz = bcast(rc[u].z, wl);
-            if (lane == bu[u]) {
-              bbest = best;
-              bsec = (V)__uint_as_float(second);
-              bx = nx;
-              by = ny;
-              bz = nz;
+            const C best = wave_best_at(cand[u], wl);
+            const T cx = bcast(rc[u].x, wl), cy = bcast(rc[u].y, wl), cz = bcast(rc[u].z, wl);
+            if constexpr (ROUNDS) {  // the next rounds' bound
+              const uint32_t second = wave_umax(lane == wl ? 0u : __float_as_uint((float)t2[u]));
+              if (lane == bits[u]) bsec = (V)__uint_as_float(second);
             }
-            changed = true;
+            // passes after the first (buckets larger than 64) keep the max
+            if (lane == bits[u] && (p0 == 0 || cand_gt(best, bbest))) {
+              bbest = best;
+              bx = cx;
+              by = cy;
+              bz = cz;
+            }
+            rereduce |= bits[u] == wlane;
           }
 #pragma unroll
           for (int u = 0; u < NB; ++u)
-            if (t2[u] != t[u]) ts[pos[u]] = t2[u];
-        };
+            if (bits[u] >= 0 && t2[u] != t[u]) ts[pos[u]] = t2[u];
+        }
+      };
+      if (tm) {
+        // the visiting waves set the barrier's arrival: let them issue first
+        __builtin_amdgcn_s_setprio(3);
         while (tm) {
           const int nt = __builtin_popcountll(tm);
+          // rounds of exactly the touched count (an empty slot would cost a
+          // whole load and distance pass), 5 at a time beyond that (beside the
+          // rounds of several samples, 3: the shorter code is 3-5% faster)
           if (nt == 1) visit(std::integral_constant<int, 1>{});
           else if (nt == 2) visit(std::integral_constant<int, 2>{});
-          else if (nt == 3) visit(std::integral_constant<int, 3>{});
-          else if (nt <= 5) visit(std::integral_constant<int, 4>{});
-          else visit(std::integral_constant<int, 6>{});
+          else if (ROUNDS || nt == 3) visit(std::integral_constant<int, 3>{});
+          else if (nt == 4) visit(std::integral_constant<int, 4>{});
+          else visit(std::integral_constant<int, 5>{});
         }
         reach = reach_of(bbest);
+        __builtin_amdgcn_s_setprio(0);
       }
-      if (changed) {  // the wave's two best buckets, and a bound on everything else in it
-        changed = false;
-        (void)wave_best_at(bbest, l1);
-        const C rest = lane == l1 ? cand_none(ctag) : bbest;
-        w2 = wave_best_at(rest, l2);
-        const bool pub = lane == l1 || (lane == l2 && cand_valid(w2));
-        third = wave_umax(__float_as_uint(pub ? (float)bsec : (float)cand_val(bbest)));
+      if (rereduce) {  // the wave's best bucket changed; otherwise wbest stands
+        wbest = wave_best_at(bbest, wlane);
       }
-      const int par = rd & 1;
-      if (lane == l1) {
-        s_ck[par][2 * w] = bbest.k;
-        s_cp[par][2 * w] = make_float4((float)bx, (float)by, (float)bz, 0.f);
-      }
-      // (a wave without a second bucket publishes no candidate there)
-      if (lane == (cand_valid(w2) ? l2 : (l1 ^ 1))) {
-        s_ck[par][2 * w + 1] = cand_valid(w2) ? bbest.k : 0ull;
-        s_cp[par][2 * w + 1] = make_float4((float)bx, (float)by, (float)bz, 0.f);
-      }
-      // three slots in turn: the next round's are cleared here, after their
-      // last readers (before the first barrier of this round)
-      if (lane == 0) atomicMax(&s_tau[rd % 3], third);
-      if (tid == 0) {
-        s_tau[(rd + 1) % 3] = 0;
-        s_gkey[(rd + 1) % 3] = 0;
-      }
-      __syncthreads();
-      // candidate j is out of order when one with a larger key lowers its
-      // running minimum, or would not lower its own (infinite coordinates:
-      // it is chosen again and again): wave w tests its two, a lane a pair
-      {
-        const int j = 2 * w + (lane >> 5);
-        ck = s_ck[par][lane & 31];
-        const float4 ci = s_cp[par][lane & 31];
-        const uint64_t kj = s_ck[par][j];
-        const float4 cj = s_cp[par][j];
-        cx = ci.x;
-        cy = ci.y;
-        cz = ci.z;
-        const T d = sq3((T)((T)cj.x - (T)ci.x), (T)((T)cj.y - (T)ci.y), (T)((T)cj.z - (T)ci.z));
-        const bool stays = !((ci.x - ci.x) + (ci.y - ci.y) + (ci.z - ci.z) == 0.f);
-        const uint64_t hit = __ballot(
-            ck > kj && kj != 0 && (stays || (float)d < __uint_as_float((uint32_t)(kj >> 32))));
-        if ((lane & 31) == 0 && (uint32_t)(hit >> lane) != 0)
-          atomicMax(&s_gkey[rd % 3], (unsigned long long)kj);
-      }
-      __syncthreads();
-      // this round's samples: the candidates above every such one, and above
-      // every other point's value
-      const uint64_t out_of = s_gkey[rd % 3];
-      const uint64_t others = (uint64_t)s_tau[rd % 3] << 32 | 0xffffffffull;
-      const uint64_t floor_key = out_of > others ? out_of : others;
-      pm = (uint32_t)__ballot(ck > floor_key);
-      if (pm == 0) {  // only the largest is certain
-        int gl;
-        const C g = wave_best_at(C{ck}, gl);
-        if (!cand_valid(g)) {  // nothing takes part: index 0 from here on (rank -1)
-          for (int j = done + tid; j < m; j += FPS_THREADS) out[j] = -1;
-          break;
+      const int par = j & 1;
+      C g;
+      int gw;
+      WaveBest mine;
+      // the lane holding the wave's best publishes it from its own registers;
+      // every lane then reads wave (lane mod 16)'s entry
+      if constexpr (sizeof(C) == 8) {
+        // Packed keys: every wave folds its best into one LDS word with an
+        // atomic max; slots rotate over 3 iterations so the reset of the next
+        // slot (before this barrier) never races with its readers (before the
+        // previous barrier) or its writers (after this barrier).
+        if (tid == 0) s_gkey[(j + 1) % 3] = 0;
+        if (lane == wlane) {
+          atomicMax(&s_gkey[j % 3], (unsigned long long)bbest.k);
+          s_wb[par][w] = WaveBest{bbest, bx, by, bz};
         }
-        pm = 1u << gl;
+        __syncthreads();
+        mine = s_wb[par][lane & (FPS_WAVES - 1)];  // issued with the key read
+        g = C{s_gkey[j % 3]};
+        gw = lane_of(mine.c, g);
+      } else {
+        if (lane == wlane) s_wb[par][w] = WaveBest{bbest, bx, by, bz};
+        __syncthreads();
+        mine = s_wb[par][lane & (FPS_WAVES - 1)];
+        g = row0_best(mine.c);
+        gw = lane_of(mine.c, g);
       }
-      if (w == 0) {  // in key order
-        int at = done;
-        for (uint32_t mk = pm; mk != 0; mk &= mk - 1) {
-          const int i = __builtin_ctz(mk);
-          const uint64_t k = (uint64_t)(uint32_t)__builtin_amdgcn_readlane((int)(ck >> 32), i) << 32 |
-                             (uint32_t)__builtin_amdgcn_readlane((int)(uint32_t)ck, i);
-          at += k > ck ? 1 : 0;
+      // Nothing participates: the reference's index 0 (rank -1 here).  The
+      // rank is decoded to an index after the loop, off the critical path.
+      const bool gv = cand_valid(g);
+      ox = gv ? bcast(mine.x, gw) : p0x;
+      oy = gv ? bcast(mine.y, gw) : p0y;
+      oz = gv ? bcast(mine.z, gw) : p0z;
+      const int r = gv ? (int)cand_rank(g) : -1;
+      // wave 0 stores the ranks 64 at a time
+      if (w == 0) {
+        rk = lane == (j & 63) ? r : rk;
+        if ((j & 63) == 63 || j == to - 1) {
+          const int jj = (j & ~63) + lane;
+          if (jj >= from && jj <= j) out[jj] = (int64_t)rk;
         }
-        if (lane < 32 && (pm >> lane) & 1 && at < m) out[at] = (int64_t)(0xffffffffu - (uint32_t)ck);
-      }
-      done += __builtin_popcount(pm);
-      if (done >= m) break;
-    }
-    __syncthreads();
-    fps_decode(out, m, tid, FPS_THREADS, bs, bs_bits, per);
-    return;
-  }
-  for (int j = 1; j < m; ++j) {
-    const V o3[3] = {(V)ox, (V)oy, (V)oz};
-    V e[3];
-#pragma unroll
-    for (int c = 0; c < 3; ++c) e[c] = vmax(vmax(blo[c] - o3[c], o3[c] - bhi[c]), (V)0);
-    const V lb2 = vfma(e[2], e[2], vfma(e[1], e[1], e[0] * e[0]));
-    // the first sample's updates were made while the cloud was set up
-    uint64_t tm = j > 1 ? __ballot(lb2 <= reach) : 0;
-    bool rereduce = false;  // the best of the wave's best bucket changed
-    // Touched buckets are visited NB at a time: every slot's loads are issued
-    // first (the rounds below never leave a slot empty; an empty slot would
-    // re-read slot 0's bucket), the NB wave reductions are independent
-    // straight-line code, and the running-minimum stores come last, so no load
-    // or reduction of the batch waits for a store.
-    auto visit = [&](auto nbc) {
-      constexpr int NB = decltype(nbc)::value;
-      int bits[NB];
-#pragma unroll
-      for (int u = 0; u < NB; ++u) {
-        bits[u] = tm ? __builtin_ctzll(tm) : -1;
-        tm &= tm ? tm - 1 : 0;
-      }
-      for (int p0 = 0; p0 < s_sz; p0 += 64) {
-        int pos[NB];
-        FpsRec<T> rc[NB];
-        T t[NB];
-#pragma unroll
-        for (int u = 0; u < NB; ++u) {
-          const int bu = bits[u] >= 0 ? bits[u] : bits[0];
-          pos[u] = (bu * FPS_WAVES + w) * s_sz + p0 + lane;
-          rc[u] = recs[pos[u]];
-          t[u] = ts[pos[u]];
-        }
-        T t2[NB];
-        C cand[NB];
-#pragma unroll
-        for (int u = 0; u < NB; ++u) {
-          const T d = sq3((T)(rc[u].x - ox), (T)(rc[u].y - oy), (T)(rc[u].z - oz));  // fps.cu:145
-          t2[u] = d < t[u] ? d : t[u];                                                // fps.cu:146
-          cand[u] = cand_make((V)t2[u], rc[u].key, ctag);
-        }
-        // A bucket's best stays its best unless that point's own running
-        // minimum dropped (the others can only drop too), so the reduction
-        // runs only then (always for buckets larger than 64 points).
-        bool red[NB];
-#pragma unroll
-        for (int u = 0; u < NB; ++u) {
-          const int bu = bits[u] >= 0 ? bits[u] : bits[0];
-          const uint32_t bkey = (uint32_t)__builtin_amdgcn_readlane((int)cand_keyword(bbest), bu);
-          red[u] = bits[u] >= 0 && (s_sz > 64 || __ballot(rc[u].key == bkey && t2[u] != t[u]) != 0);
-        }
-#pragma unroll
-        for (int u = 0; u < NB; ++u) {
-          if (!red[u]) continue;
-          int wl;
-          const C best = wave_best_at(cand[u], wl);
-          const T cx = bcast(rc[u].x, wl), cy = bcast(rc[u].y, wl), cz = bcast(rc[u].z, wl);
-          // passes after the first (buckets larger than 64) keep the max
-          if (lane == bits[u] && (p0 == 0 || cand_gt(best, bbest))) {
-            bbest = best;
-            bx = cx;
-            by = cy;
-            bz = cz;
-          }
-          rereduce |= bits[u] == wlane;
-        }
-#pragma unroll
-        for (int u = 0; u < NB; ++u)
-          if (bits[u] >= 0 && t2[u] != t[u]) ts[pos[u]] = t2[u];
-      }
-    };
-    if (tm) {
-      // the visiting waves set the barrier's arrival: let them issue first
-      __builtin_amdgcn_s_setprio(3);
-      while (tm) {
-        const int nt = __builtin_popcountll(tm);
-        // rounds of exactly the touched count (an empty slot would cost a
-        // whole load and distance pass), 5 at a time beyond that
-        if (nt == 1) visit(std::integral_constant<int, 1>{});
-        else if (nt == 2) visit(std::integral_constant<int, 2>{});
-        else if (nt == 3) visit(std::integral_constant<int, 3>{});
-        else if (nt == 4) visit(std::integral_constant<int, 4>{});
-        else visit(std::integral_constant<int, 5>{});
-      }
-      reach = reach_of(bbest);
-      __builtin_amdgcn_s_setprio(0);
-    }
-    if (rereduce) {  // the wave's best bucket changed; otherwise wbest stands
-      wbest = wave_best_at(bbest, wlane);
-    }
-    const int par = j & 1;
-    C g;
-    int gw;
-    WaveBest mine;
-    // the lane holding the wave's best publishes it from its own registers;
-    // every lane then reads wave (lane mod 16)'s entry
-    if constexpr (sizeof(C) == 8) {
-      // Packed keys: every wave folds its best into one LDS word with an
-      // atomic max; slots rotate over 3 iterations so the reset of the next
-      // slot (before this barrier) never races with its readers (before the
-      // previous barrier) or its writers (after this barrier).
-      if (tid == 0) s_gkey[(j + 1) % 3] = 0;
-      if (lane == wlane) {
-        atomicMax(&s_gkey[j % 3], (unsigned long long)bbest.k);
-        s_wb[par][w] = WaveBest{bbest, bx, by, bz};
-      }
-      __syncthreads();
-      mine = s_wb[par][lane & (FPS_WAVES - 1)];  // issued with the key read
-      g = C{s_gkey[j % 3]};
-      gw = lane_of(mine.c, g);
-    } else {
-      if (lane == wlane) s_wb[par][w] = WaveBest{bbest, bx, by, bz};
-      __syncthreads();
-      mine = s_wb[par][lane & (FPS_WAVES - 1)];
-      g = row0_best(mine.c);
-      gw = lane_of(mine.c, g);
-    }
-    // Nothing participates: the reference's index 0 (rank -1 here).  The
-    // rank is decoded to an index after the loop, off the critical path.
-    const bool gv = cand_valid(g);
-    ox = gv ? bcast(mine.x, gw) : p0x;
-    oy = gv ? bcast(mine.y, gw) : p0y;
-    oz = gv ? bcast(mine.z, gw) : p0z;
-    const int r = gv ? (int)cand_rank(g) : -1;
-    // wave 0 stores the ranks 64 at a time
-    if (w == 0) {
-      rk = lane == (j & 63) ? r : rk;
-      if ((j & 63) == 63 || j == m - 1) {
-        const int jj = (j & ~63) + lane;
-        if (jj >= 1 && jj <= j) out[jj] = (int64_t)rk;
       }
     }
+    done = to;
+    if (!ROUNDS || done >= m) break;
+    hold *= 2;
   }
   __syncthreads();
   fps_decode(out, m, tid, FPS_THREADS, bs, bs_bits, per);
