@@ -162,3 +162,18 @@ def test_knn_rows_workspace_is_in_proportion_to_the_points(lib, K):
         # a record of 16 bytes a point, 8 bytes a query of rows left to replay, and
         # the starts of at most eight cells a reference
         assert base <= rows <= max(base, N * (P2 * (16 + 32) + P1 * 24 + 64) + 4096)
+
+
+@pytest.mark.parametrize("sizes,rows", [
+    # 3-D: long clouds, and short ones of which there are not too many
+    ((16, 2048, 2048, 3, 16), True), ((8, 16384, 1024, 3, 3), True), ((16, 32, 512, 3, 4), True),
+    ((4096, 32, 512, 3, 4), False), ((4096, 32, 512, 3, 32), True), ((1024, 1, 2048, 3, 4), True),
+    ((64, 2048, 512, 3, 8), False), ((64, 2048, 512, 3, 16), True), ((1, 100, 127, 3, 32), False),
+])
+def test_which_knn_calls_select_rows_by_distance(lib, sizes, rows):
+    I = ctypes.c_int64
+    for f in (lib.tpo_knn_rows_workspace_size, lib.tpo_knn_workspace_size):
+        f.argtypes = [ctypes.c_int, I, I, I, I, I, ctypes.c_int]
+        f.restype = I
+    more = lib.tpo_knn_rows_workspace_size(0, *sizes, 2) > lib.tpo_knn_workspace_size(0, *sizes, 2)
+    assert more == rows

@@ -631,20 +631,44 @@ KnLayout kn_layout(int64_t N, int64_t P1, int64_t P2) {
 // One workgroup bins a cloud: clouds of up to 2^18 points.  A search costs a
 // query about the same whatever the cloud, brute force (knn_fwd_kernel) about
 // in proportion to it, and less a query where many queries fill the GPU.
-// Measured, us with the grid / brute force, 131072 queries (8192 queries):
+// Measured, us with the grid / brute force, 8 clouds of 16384 queries (8192
+// queries):
 //   P2 = 128: K = 3 76 / 51 (27 / 25), K = 8 101 / 65 (30 / 36), K = 32 165 / 150 (31 / 103)
 //   P2 = 256: K = 1 49 / 49, K = 8 90 / 75 (30 / 44), K = 16 105 / 114, K = 32 159 / 189
 //   P2 = 384: K = 8 97 / 82 (28 / 54);  P2 = 512: K = 3 66 / 69, K = 8 86 / 89, K = 16 117 / 142
-static bool kn_pays(int64_t rows, int64_t P2, int64_t K) {
-  if (P2 >= 512) return true;
+// Shorter clouds of queries are put in order sooner for brute force, which then
+// gains more; 64 (128) clouds of 2048 queries:
+//   P2 = 512: K = 1 54 / 48 (80 / 68), K = 3 72 / 56 (114 / 80), K = 12 101 / 123 (181 / 188)
+//   P2 = 768: K = 3 71 / 68 (115 / 97), K = 8 92 / 95 (159 / 137)
+//   P2 = 1024: K = 8 94 / 107 (165 / 158)
+// And a set-up workgroup fills a CU: beyond 256 of them they run one after
+// another, 7 us a round (4096 / 1024 / 512 clouds of 32 queries):
+//   P2 = 512: K = 4 295 / 145, 96 / 56, 58 / 52, K = 16 326 / 324, 112 / 114, K = 32 404 / 630
+//   P2 = 1024: K = 4 318 / 193, 102 / 76, 66 / 66, K = 16 363 / 427, K = 32 458 / 858
+// Clouds of 2048 references and more have a grid in the slot-order path too.
+static bool kn_pays(int64_t N, int64_t P1, int64_t P2, int64_t K) {
+  if (P2 >= 2048) return true;
+  const int64_t rows = N * P1, setups = P1 <= P2 ? 2 * N : N;
+  if (setups > 256) {
+    const int64_t least = K < 8 ? setups : K < 16 ? (setups > 1024 ? setups : setups / 2)
+                                  : K < 24 ? setups / 4 : setups / 32;
+    if (P2 < least) return false;
+  }
   const bool many = rows > 49152;  // 32768 queries still gain at P2 = 256 (43 / 48 at K = 8)
+  if (many && N >= 32) {
+    if (K >= 12) return P2 >= (K < 24 || (rows > 98304 && N >= 512) ? 512 : 256);
+    if (N >= 128) return P2 >= (rows > 98304 ? 1024 : 768);
+    return P2 >= (rows > 98304 ? 768 : 512);
+  }
+  if (P2 >= 512) return true;
   if (P2 >= 256) return !many || K == 1 || K >= 16;
   return P2 >= 128 && K >= 16 && !many;
 }
 
 bool knn_near_applies(int dtype, int64_t N, int64_t P1, int64_t P2, int64_t D, int64_t K) {
-  return kn_pays(N * P1, P2, K) && dtype == TPO_F32 && D == 3 && K >= 1 && K <= 32 && N >= 1 && P1 >= 1 && P2 >= 1 &&
-         P1 <= (1 << 18) && P2 <= (1 << 18) && N <= (1 << 16) && N * P1 <= 0x7fffffff;
+  return dtype == TPO_F32 && D == 3 && K >= 1 && K <= 32 && N >= 1 && P1 >= 1 && P2 >= 1 &&
+         P1 <= (1 << 18) && P2 <= (1 << 18) && N <= (1 << 16) && N * P1 <= 0x7fffffff &&
+         kn_pays(N, P1, P2, K);
 }
 
 int64_t knn_near_workspace(int64_t N, int64_t P1, int64_t P2) { return kn_layout(N, P1, P2).total; }
