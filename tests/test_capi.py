@@ -169,6 +169,9 @@ def test_knn_rows_workspace_is_in_proportion_to_the_points(lib, K):
     ((16, 2048, 2048, 3, 16), True), ((8, 16384, 1024, 3, 3), True), ((16, 32, 512, 3, 4), True),
     ((4096, 32, 512, 3, 4), False), ((4096, 32, 512, 3, 32), True), ((1024, 1, 2048, 3, 4), True),
     ((64, 2048, 512, 3, 8), False), ((64, 2048, 512, 3, 16), True), ((1, 100, 127, 3, 32), False),
+    # features: not the shortest clouds under few or many queries
+    ((8, 2048, 2048, 64, 20), True), ((1, 16, 8, 9, 5), False), ((128, 1024, 128, 4, 8), False),
+    ((1, 1024, 128, 4, 8), True), ((65536, 1, 16, 16, 8), False), ((1, 1, 100000, 4, 1), True),
 ])
 def test_which_knn_calls_select_rows_by_distance(lib, sizes, rows):
     I = ctypes.c_int64

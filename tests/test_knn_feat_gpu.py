@@ -28,12 +28,13 @@ def _check(tpo, dev, p1, p2, l1, l2, K):
 
 # widths at the edges of the 16-wide k-steps with six more entries for the
 # norms, and not multiples of 4; reference counts at the edges of the tiles
-# (32), of the all-candidates lists (192), of the fine groups (31 tiles) and of
-# several tiles a group (over 128 tiles a wave)
+# (32), of the fine groups (up to 32 tiles, made odd: 992 and 993 references)
+# and of several tiles a group (over 128 tiles: 4064 and 4096)
 @pytest.mark.parametrize("D,P1,P2,K", [
     (4, 70, 1, 3), (9, 64, 31, 5), (10, 65, 33, 20), (11, 130, 192, 32), (26, 63, 193, 32),
     (27, 200, 255, 16), (35, 333, 992, 20), (42, 1, 993, 2), (58, 128, 1024, 10),
-    (64, 500, 2048, 20), (74, 96, 3000, 32), (90, 33, 5000, 5), (106, 40, 700, 8),
+    (64, 500, 2048, 20), (9, 70, 4064, 32), (20, 70, 4096, 31), (74, 96, 3000, 32),
+    (90, 33, 5000, 5), (106, 40, 700, 8),
     (122, 64, 4128, 31), (128, 257, 9001, 16), (64, 30, 33000, 32), (16, 700, 4095, 12),
 ])
 @pytest.mark.parametrize("case", ["normal", "offset", "self"])
@@ -49,6 +50,22 @@ def test_feature_rows_match_the_reference_order(tpo, dev, D, P1, P2, K, case):
         p1 = p2[:, torch.randint(0, P2, (P1,), generator=g)].contiguous()
     l1 = torch.tensor([P1, max(1, P1 - 5)])
     l2 = torch.tensor([P2, max(1, (2 * P2) // 3)])
+    _check(tpo, dev, p1, p2, l1, l2, K)
+
+
+# lengths at the edges of the clouds that are listed whole (32 + 2 K) and of a
+# row's list (128), alone and in the mostly empty tiles of a longer cloud, where
+# few more than K groups hold a reference
+@pytest.mark.parametrize("P2", [0, 352, 1056, 9001])
+@pytest.mark.parametrize("D,K", [(16, 5), (64, 16), (9, 31), (35, 32)])
+def test_feature_rows_of_short_lengths(tpo, dev, D, K, P2):
+    g = torch.Generator().manual_seed(D + P2)
+    l2 = torch.tensor([1, K - 1, K, K + 1, 31 + 2 * K, 32 + 2 * K, 33 + 2 * K, 127, 128, 129, 130, 0])
+    N, P1, P2 = len(l2), 70, P2 or 130
+    p1, p2 = torch.randn(N, P1, D, generator=g), torch.randn(N, P2, D, generator=g)
+    p2[:, 3] = p2[:, 9]
+    l1 = torch.full((N,), P1)
+    l1[2], l1[-2] = 64, 33
     _check(tpo, dev, p1, p2, l1, l2, K)
 
 

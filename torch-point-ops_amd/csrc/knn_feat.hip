@@ -70,6 +70,12 @@ __host__ __device__ inline int kf_ksteps(int64_t D) { return (int)((D + 6 + 15) 
 __host__ __device__ inline int kf_tiles2(int64_t P2) { return (int)((P2 + 31) / 32) | 1; }
 __host__ __device__ inline int kf_tiles1(int64_t P1) { return (int)((P1 + KF_Q - 1) / KF_Q) * 2; }
 
+// Clouds up to this length are listed whole: the K-th group minimum bounds
+// little there.  8 x 1024 queries, D = 16, us with the bound / listed whole:
+// 64 references 28 / 40 (K = 8), 96 32 / 63 (K = 16), 112 86 / 79 (K = 32), 128
+// 33 / 91 (K = 4), 82 / 100 (K = 32).
+__host__ __device__ inline int kf_list(int K) { return 32 + 2 * K; }
+
 struct KfLayout {
   int64_t qb, rb, qinfo, tinfo, redo, total;
 };
@@ -302,7 +308,7 @@ __global__ __launch_bounds__(KF_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
     // ones: groups of 16, over m tiles of the wave where there are more
     // than 16 of them.
     const bool fine = TE <= 4 * KF_WAVES;
-    if (L2 > KF_CAP) {
+    if (L2 > kf_list(K)) {
       const int m = ((TE + KF_WAVES - 1) / KF_WAVES + 15) / 16;
       float run[2] = {Lim<float>::inf(), Lim<float>::inf()};
       int i = 0, slot = 0;
@@ -367,7 +373,7 @@ __global__ __launch_bounds__(KF_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
       const float L = (far * far) * (1.f + 0x1p-20f) + E;
       const bool active = q0 + qi < L1;
       const bool fin = del < Lim<float>::inf() && len < Lim<float>::inf();
-      const bool all = L2 <= KF_CAP;
+      const bool all = L2 <= KF_CAP && !(L < 1.0e37f);
       const bool bad = all ? !fin : !(L < 1.0e37f);
       lim[b] = !active || bad ? -Lim<float>::inf() : (all ? 3.0e38f : L);
       if (w == 0 && h == 0) sm.bad[qi] = bad;
@@ -546,9 +552,27 @@ void kf_launch(const void* p1, const void* p2, const int64_t* l1, const int64_t*
 
 }  // namespace
 
+// Short clouds stay with a query a lane (knn_fwd_kernel).  Beyond what one launch
+// takes, that one costs about ref_ns a reference and 0.8 us a neighbour, more
+// where the queries are more than the GPU's lanes; this path 13 us and, in
+// blocks of 64, 0.6 + 0.006 D + 0.035 K ns a query.  Measured, us a query a lane
+// / here: D = 4, K = 4: 1024 queries 24 / 28 (P2 = 32), 37 / 28 (64); 32768
+// queries 37 / 40 (64), 49 / 40 (96); 131072 queries 79 / 123 (128), 139 / 135
+// (256); D = 9, K = 32, 131072 queries: 255 / 500 (128), 385 / 310 (256);
+// D = 128, K = 4, 32768 queries: 85 / 81 (32), 160 / 66 (64).
+static bool kf_pays(int64_t rows, int64_t P2, int64_t D, int64_t K) {
+  if (P2 >= 4096) return true;
+  const double ref_ns = D == 64 ? 500 : D == 128 ? 1000
+                        : D <= 12 ? 70 * D : (rows < 512 ? 85 : 120) * D;
+  const double full = rows > 83000 ? rows / 83000.0 : 1.0;
+  const double here = 13000 + rows * (0.6 + 0.006 * D + 0.035 * K);
+  return (P2 * ref_ns + 800 * K) * full >= (here > 18000 ? here : 18000);
+}
+
 bool knn_feat_applies(int dtype, int64_t N, int64_t P1, int64_t P2, int64_t D, int64_t K, int norm) {
   if (dtype != TPO_F32 || norm != 2 || D < 4 || D > KF_DMAX || K < 1 || K > 32) return false;
   if (N < 1 || P1 < 1 || P2 < 1 || P2 > (1 << 26) || N * P1 > 0x7fffffff) return false;
+  if (!kf_pays(N * kf_tiles1(P1) * 32, P2, D, K)) return false;
   // every tile is a workgroup of one launch
   return N * (kf_tiles1(P1) + (int64_t)kf_tiles2(P2)) <= 0x7fffffff;
 }
