@@ -69,6 +69,25 @@ def test_feature_rows_of_short_lengths(tpo, dev, D, K, P2):
     _check(tpo, dev, p1, p2, l1, l2, K)
 
 
+# every row tied or not finite, more of them than are replayed: left to the
+# lane-a-row kernel, and (64 and 128 dimensions, few queries, long clouds) to
+# the kernels that slice the references
+@pytest.mark.parametrize("N,P1,P2,D,K", [(3, 4003, 300, 9, 5), (2, 9000, 170, 4, 12), (1, 1500, 4000, 64, 8),
+                                         (2, 1100, 3000, 128, 20)])
+@pytest.mark.parametrize("case", ["lattice", "one_nan"])
+def test_feature_rows_too_many_to_replay(tpo, dev, N, P1, P2, D, K, case):
+    g = torch.Generator().manual_seed(P1 + D)
+    p1, p2 = torch.randn(N, P1, D, generator=g), torch.randn(N, P2, D, generator=g)
+    if case == "lattice":
+        p1, p2 = (p1 > 0.5).float(), (p2 > 0.5).float()
+    else:
+        p2[0, P2 - 2, 1] = float("nan")
+    l1, l2 = torch.full((N,), P1), torch.full((N,), P2)
+    l1[-1] = P1 - 3
+    l2[-1] = P2 - 1
+    _check(tpo, dev, p1, p2, l1, l2, K)
+
+
 @pytest.mark.parametrize("case", ["few_ties", "all_ties", "runs", "nonfinite_query",
                                   "nonfinite_cloud", "nan_of_ones", "huge", "tiny", "short", "far_cloud"])
 @pytest.mark.parametrize("D,K", [(64, 20), (9, 5)])

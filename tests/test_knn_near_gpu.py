@@ -26,9 +26,9 @@ def _cloud(kind, g, N, P):
     return x
 
 
-# query and reference counts at the edges of a row (16), a wave (64), a
-# workgroup (256), the register-held setups (4096, 16384) and above; K at the
-# edges of the slot counts (4, 8, 16, 32)
+# reference and query counts at the edges of the register-held setups (4096,
+# 16384) and above, and on both sides of the choice between the grid and brute
+# force; K at the edges of the slots' registers (16, 32)
 @pytest.mark.parametrize("P1,P2,K", [
     (1, 1, 1), (15, 2, 3), (17, 40, 4), (64, 33, 32), (65, 257, 5), (255, 1024, 8), (257, 500, 9),
     (1000, 2048, 16), (4096, 4097, 17), (4097, 4096, 3), (700, 16384, 16), (16390, 300, 12),
@@ -63,6 +63,72 @@ def test_near_rows_match_the_reference_order(tpo, dev, P1, P2, K, kind, norm):
         si, sd = tpo.knn_points(a, b, la, lb, K=K, norm=norm, version=0)
         assert torch.equal(sd, ed)
         assert torch.equal(si, ei)
+
+
+def _takes_rows(N, P1, P2, D, K):
+    """Whether knn_points selects rows by distance for these sizes."""
+    import ctypes
+
+    from torch_point_ops import _native
+
+    I = ctypes.c_int64
+    L = ctypes.CDLL(_native.HIP_LIB)
+    f = L.tpo_knn_rows_workspace_size, L.tpo_knn_workspace_size
+    for g in f:
+        g.argtypes, g.restype = [ctypes.c_int, I, I, I, I, I, ctypes.c_int], I
+    return f[0](0, N, P1, P2, D, K, 2) > f[1](0, N, P1, P2, D, K, 2)
+
+
+# a wave searches four queries and a workgroup 16; clouds shorter than a row's
+# K, empty ones, and queries in row order (more of them than references)
+@pytest.mark.parametrize("P1,P2,K", [(1, 512, 3), (3, 600, 16), (4, 512, 2), (5, 700, 8), (15, 513, 9),
+                                     (16, 512, 17), (17, 640, 32), (31, 900, 1), (2100, 1800, 12),
+                                     (700, 600, 5), (33, 2500, 24)])
+@pytest.mark.parametrize("kind", ["normal", "blobs"])
+def test_near_rows_of_few_queries_and_short_lengths(tpo, O, dev, P1, P2, K, kind):
+    g = torch.Generator().manual_seed(P1 + 7 * P2 + K)
+    N = 7
+    assert _takes_rows(N, P1, P2, 3, K)
+    p1, p2 = _cloud(kind, g, N, P1), _cloud(kind, g, N, P2)
+    l1 = torch.tensor([P1, P1, P1, max(1, P1 - 1), P1, P1, 0])
+    l2 = torch.tensor([P2, K + 1, K, max(0, K - 1), 1, 0, P2])
+    a, b, la, lb = p1.to(dev), p2.to(dev), l1.to(dev), l2.to(dev)
+    si, sd = tpo.knn_points(a, b, la, lb, K=K, version=0)
+    if K == 1:
+        ei, ed = O.knn_fwd(p1.numpy(), p2.numpy(), l1.numpy(), l2.numpy(), K=1, version=0)
+        assert np.array_equal(si.cpu().numpy(), ei) and np.array_equal(sd.cpu().numpy(), ed)
+        return
+    ri, rd = torch.ops.torch_point_ops_knn.knn_forward(a, b, la, lb, 2, K, 0)
+    ei, ed = _sorted_by_module(ri, rd, lb, K)
+    assert torch.equal(sd, ed) and torch.equal(si, ei)
+
+
+# rows with equal distances replayed one by one, and too many for that: lists in
+# the queries' order (P1 <= P2) and from row order, to the grid's lane-a-row
+# kernel (2048 references and more) and to brute force
+@pytest.mark.parametrize("N,P1,P2,K", [(2, 5000, 6000, 16), (3, 3001, 3001, 3), (2, 5001, 2500, 8),
+                                       (4, 1999, 700, 20), (3, 2600, 900, 5), (2, 8000, 1023, 32),
+                                       (40, 130, 520, 16), (1, 3000, 40000, 4)])
+@pytest.mark.parametrize("tied", [0.0, 0.02, 0.3, 1.0])
+def test_near_rows_of_clouds_with_repeated_points(tpo, dev, N, P1, P2, K, tied):
+    g = torch.Generator().manual_seed(P1 + P2 + K)
+    assert _takes_rows(N, P1, P2, 3, K)
+    p1, p2 = torch.randn(N, P1, 3, generator=g), torch.randn(N, P2, 3, generator=g)
+    m = int(P2 * tied)
+    p2[:, :m] = p2[:, torch.randint(0, max(1, m // 2), (m,), generator=g)]
+    p2 = p2[:, torch.randperm(P2, generator=g)].contiguous()
+    if tied == 1.0:  # a lattice as well
+        p1, p2 = (p1 * 4).round() / 4, (p2 * 4).round() / 4
+    l1 = torch.full((N,), P1)
+    l1[-1] = P1 - 7
+    l2 = torch.full((N,), P2)
+    l2[0] = P2 - P2 // 3
+    a, b, la, lb = p1.to(dev), p2.to(dev), l1.to(dev), l2.to(dev)
+    for norm in (2, 1):
+        si, sd = tpo.knn_points(a, b, la, lb, K=K, norm=norm, version=0)
+        ri, rd = torch.ops.torch_point_ops_knn.knn_forward(a, b, la, lb, norm, K, 0)
+        ei, ed = _sorted_by_module(ri, rd, lb, K)
+        assert torch.equal(sd, ed) and torch.equal(si, ei)
 
 
 @pytest.mark.parametrize("case", ["few_ties", "lattice", "nonfinite_query", "nonfinite_cloud", "nan_of_ones",

@@ -25,6 +25,7 @@
 //   reference's global-memory MinK.
 #include <utility>
 
+#include "knn_order.hpp"
 #include "knn_replay.hpp"
 
 namespace tpo {
@@ -39,13 +40,13 @@ int hd_slices(int dtype, int64_t N, int64_t P1, int64_t P2, int64_t D, int64_t K
 int64_t hd_workspace_bytes(int64_t rows, int64_t S, int64_t K);
 void launch_hd(const void* p1, const void* p2, const int64_t* l1, const int64_t* l2, int N, int P1,
                int P2, int D, int K, int norm, int S, int pad, bool sort, int64_t* idxs,
-               void* dists, void* ws, hipStream_t s);
+               void* dists, void* ws, const uint32_t* only, hipStream_t s);
 // knn_feat.hip
 bool knn_feat_applies(int dtype, int64_t N, int64_t P1, int64_t P2, int64_t D, int64_t K, int norm);
 int64_t knn_feat_workspace(int64_t N, int64_t P1, int64_t P2, int64_t D);
 RedoList launch_knn_feat(const void* p1, const void* p2, const int64_t* l1, const int64_t* l2,
-                         int N, int P1, int P2, int D, int K, int pad, bool sort, int64_t* idxs,
-                         void* dists, void* ws, hipStream_t s);
+                         int N, int P1, int P2, int D, int K, int pad, bool sort, bool sliced,
+                         int64_t* idxs, void* dists, void* ws, hipStream_t s);
 // knn_near.hip
 bool knn_near_applies(int dtype, int64_t N, int64_t P1, int64_t P2, int64_t D, int64_t K);
 int64_t knn_near_workspace(int64_t N, int64_t P1, int64_t P2);
@@ -65,117 +66,32 @@ void launch_knn_grid(const void* p1, const void* p2, const int64_t* l1, const in
 namespace tpo {
 namespace {
 
-// Per cloud, the valid queries (row < lengths1) in Morton order of a 16^3
-// grid over their bounding box.  The order only decides which queries share
-// a wave: neighbouring queries share their nearest references, so the MinK
-// insertions of a wave's lanes coincide and the candidate loop below runs
-// fewer iterations.  Results are bit-identical in any order.
-constexpr int KNN_GRID = 16;
-constexpr int KNN_CELLS = KNN_GRID * KNN_GRID * KNN_GRID;
-
+// Per cloud, the valid queries (row < lengths1) in spatial order.
 template <typename T>
 __global__ __launch_bounds__(1024) void knn_order_kernel(const T* __restrict__ p1,
                                                          const int64_t* __restrict__ len1, int P1,
                                                          int32_t* __restrict__ order) {
-  __shared__ uint32_t cnt[KNN_CELLS];
-  __shared__ float red[6][16];
-  __shared__ uint32_t part[16];
-  const int n = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-  int64_t l1 = len1[n];
+  __shared__ KnnOrderLds sm;
+  const int n = blockIdx.x;
+  const int64_t l1 = len1[n];
   const int L1 = (int)(l1 < 0 ? 0 : (l1 > P1 ? P1 : l1));
-  const T* __restrict__ P = p1 + (size_t)n * P1 * 3;
   int32_t* __restrict__ out = order + (size_t)n * P1;
-  float lo[3] = {__builtin_inff(), __builtin_inff(), __builtin_inff()};
-  float hi[3] = {-__builtin_inff(), -__builtin_inff(), -__builtin_inff()};
-  for (int k = tid; k < L1; k += 1024)
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      const float v = (float)P[3 * k + c];
-      lo[c] = fminf(lo[c], v);
-      hi[c] = fmaxf(hi[c], v);
-    }
-#pragma unroll
-  for (int c = 0; c < 3; ++c)
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) {
-      lo[c] = fminf(lo[c], __shfl_xor(lo[c], m, 64));
-      hi[c] = fmaxf(hi[c], __shfl_xor(hi[c], m, 64));
-    }
-  if (lane == 0)
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      red[c][w] = lo[c];
-      red[3 + c][w] = hi[c];
-    }
-  for (int c = tid; c < KNN_CELLS; c += 1024) cnt[c] = 0;
-  __syncthreads();
-  float glo[3], gs[3];
-#pragma unroll
-  for (int c = 0; c < 3; ++c) {
-    float a = __builtin_inff(), z = -__builtin_inff();
-    for (int v = 0; v < 16; ++v) {
-      a = fminf(a, red[c][v]);
-      z = fmaxf(z, red[3 + c][v]);
-    }
-    glo[c] = a;
-    const float ext = z - a;
-    gs[c] = (ext > 0.f && ext < __builtin_inff()) ? (float)KNN_GRID / ext : 0.f;
-  }
-  auto cell_of = [&](int k) -> uint32_t {
-    uint32_t code = 0;
-#pragma unroll
-    for (int c = 0; c < 3; ++c) {
-      const float f = ((float)P[3 * k + c] - glo[c]) * gs[c];
-      int i = (f == f) ? (int)f : 0;
-      i = i < 0 ? 0 : (i > KNN_GRID - 1 ? KNN_GRID - 1 : i);
-      uint32_t v = (uint32_t)i;
-      v = (v | (v << 4)) & 0x0c3;
-      v = (v | (v << 2)) & 0x249;
-      code |= v << c;
-    }
-    return code;
-  };
-  for (int k = tid; k < L1; k += 1024) atomicAdd(&cnt[cell_of(k)], 1u);
-  __syncthreads();
-  {  // exclusive scan, 4 cells per thread
-    uint32_t v[4], sum = 0;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      v[i] = cnt[tid * 4 + i];
-      sum += v[i];
-    }
-    uint32_t incl = sum;
-#pragma unroll
-    for (int d = 1; d < 64; d <<= 1) {
-      const uint32_t o = (uint32_t)__shfl_up((int)incl, d, 64);
-      if (lane >= d) incl += o;
-    }
-    if (lane == 63) part[w] = incl;
-    __syncthreads();
-    uint32_t run = incl - sum;
-    for (int v2 = 0; v2 < w; ++v2) run += part[v2];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      cnt[tid * 4 + i] = run;
-      run += v[i];
-    }
-  }
-  __syncthreads();
-  for (int k = tid; k < L1; k += 1024) out[atomicAdd(&cnt[cell_of(k)], 1u)] = k;
-  for (int k = L1 + tid; k < P1; k += 1024) out[k] = k;  // rows past lengths1 keep their place
+  knn_order_rows(p1 + (size_t)n * P1 * 3, L1, nullptr, sm, out);
+  for (int k = L1 + (int)threadIdx.x; k < P1; k += 1024) out[k] = k;  // rows past lengths1 keep their place
 }
 
 // mode bit 0: RegisterMinK<2> (version 3, K = 2); bit 1 (= SORT): rows
 // sorted as knn_points(return_sorted=True) returns them (knn_sort_row).
-// redo: the counts of a RedoList whose queries `order` holds, or null.  With
-// one, the listed rows alone are processed, when there are over REDO_LIMIT.
+// redo_counts: the counts of a RedoList whose queries `order` holds, which alone are
+// processed, or null.
 template <typename T, int DT, int NORM, int KC, bool SORT>
 __global__ __launch_bounds__(256) void knn_fwd_kernel(
     const T* __restrict__ p1, const T* __restrict__ p2, const int64_t* __restrict__ len1,
     const int64_t* __restrict__ len2, const int32_t* __restrict__ order, int P1, int P2, int D,
-    int K, int nqb, int pad_sentinel, int mode, const uint32_t* __restrict__ redo,
+    int K, int nqb, int pad_sentinel, int mode, const uint32_t* __restrict__ redo_counts,
     int64_t* __restrict__ idxs, T* __restrict__ dists) {
-  if (redo && redo[0] <= REDO_LIMIT) return;
+  // (float rows alone are listed: the other types' kernels stay free of it)
+  const uint32_t* const redo = sizeof(T) == 4 ? redo_counts : nullptr;
   const int sorted2 = mode & 1;
   // float D=3: reference points reach the lanes through a wave-private LDS
   // block (each lane stages one, every lane reads them back as broadcasts),
@@ -184,10 +100,13 @@ __global__ __launch_bounds__(256) void knn_fwd_kernel(
   constexpr bool STAGED = DT == 3 && sizeof(T) == 4;
   __shared__ float4 s_ref[STAGED ? 4 : 1][64];
   const int n = blockIdx.x / nqb;
-  const int i = (blockIdx.x - n * nqb) * 256 + threadIdx.x;  // position in processing order
-  const bool in_range = i < (redo ? (int)redo[1 + n] : P1);
+  const int i0 = (blockIdx.x - n * nqb) * 256, i = i0 + threadIdx.x;  // position in processing order
+  const int positions = redo ? (int)redo[n] : P1;
+  if (i0 >= positions) return;  // (usually nothing is listed)
+  const bool in_range = i < positions;
   if (!STAGED && !in_range) return;
-  const int q = in_range ? (order ? order[(size_t)n * P1 + i] : i) : 0;  // query row of this lane
+  const size_t places = redo ? (size_t)redo_stride(P1) : (size_t)P1;
+  const int q = in_range ? (order ? order[n * places + i] : i) : 0;  // query row of this lane
   int64_t l1 = len1[n], l2 = len2[n];
   l1 = l1 < 0 ? 0 : (l1 > P1 ? P1 : l1);
   l2 = l2 < 0 ? 0 : (l2 > P2 ? P2 : l2);
@@ -516,12 +435,19 @@ extern "C" int64_t tpo_knn_workspace_size(int dtype, int64_t N, int64_t P1, int6
   return order > hd ? order : hd;
 }
 
+// The row path of many dimensions: its own workspace, and behind it that of
+// the sliced kernels where these take the rows that are too many to replay.
+static int64_t feat_workspace(int dtype, int64_t N, int64_t P1, int64_t P2, int64_t D, int64_t K) {
+  const int S = hd_slices(dtype, N, P1, P2, D, K);
+  return knn_feat_workspace(N, P1, P2, D) + (S > 0 ? hd_workspace_bytes(N * P1, S, K) : 0);
+}
+
 extern "C" int64_t tpo_knn_rows_workspace_size(int dtype, int64_t N, int64_t P1, int64_t P2,
                                                int64_t D, int64_t K, int norm) {
   const int64_t base = tpo_knn_workspace_size(dtype, N, P1, P2, D, K, norm);
   if (base < 0) return base;
   const int64_t feat = D != 3 && knn_feat_applies(dtype, N, P1, P2, D, K, norm)
-                           ? knn_feat_workspace(N, P1, P2, D) : 0;
+                           ? feat_workspace(dtype, N, P1, P2, D, K) : 0;
   const int64_t near = knn_near_applies(dtype, N, P1, P2, D, K) ? knn_near_workspace(N, P1, P2) : 0;
   return std::max(base, std::max(near, feat));
 }
@@ -570,14 +496,20 @@ static int knn_fwd_impl(int dtype, const void* p1, const void* p2, const int64_t
   // 4 x 299 x 299, D = 9: 29 against 310)
   if (rows && D != 3 &&
       knn_feat_applies(dtype, N, P1, P2, D, K, norm) &&
-      workspace_bytes >= knn_feat_workspace(N, P1, P2, D)) {
+      workspace_bytes >= feat_workspace(dtype, N, P1, P2, D, K)) {
+    const int S = hd_slices(dtype, N, P1, P2, D, K);
     const RedoList r =
         launch_knn_feat(p1, p2, lengths1, lengths2, (int)N, (int)P1, (int)P2, (int)D, (int)K, pad,
-                        sort_rows, idxs, dists, workspace, s);
+                        sort_rows, S > 0, idxs, dists, workspace, s);
     launch_knn_redo(p1, p2, lengths1, lengths2, (int)N, (int)P1, (int)P2, (int)D, (int)K, norm, pad,
-                    sort_rows, r, idxs, dists, s);
-    launch_fwd<float>(p1, p2, lengths1, lengths2, r.queries, (int)N, (int)P1, (int)P2, (int)D,
-                      (int)K, norm, pad, sorted2, r.total, idxs, dists, s);
+                    sort_rows, r, REDO_ROWS, nullptr, idxs, dists, s);
+    if (S > 0)
+      launch_hd(p1, p2, lengths1, lengths2, (int)N, (int)P1, (int)P2, (int)D, (int)K, norm, S, pad,
+                sort_rows, idxs, dists, (char*)workspace + knn_feat_workspace(N, P1, P2, D),
+                r.counts, s);
+    else
+      launch_fwd<float>(p1, p2, lengths1, lengths2, r.queries, (int)N, (int)P1, (int)P2, (int)D,
+                        (int)K, norm, pad, sorted2, r.counts, idxs, dists, s);
     return check_launch("tpo_knn_fwd");
   }
   // three dimensions: a cell grid (16 x 2048 x 2048, K = 16: 69 us a call
@@ -591,14 +523,14 @@ static int knn_fwd_impl(int dtype, const void* p1, const void* p2, const int64_t
                         sort_rows, grid_redo, idxs, dists, workspace, s);
     if (!grid_redo)
       launch_fwd<float>(p1, p2, lengths1, lengths2, r.queries, (int)N, (int)P1, (int)P2, (int)D,
-                        (int)K, norm, pad, sorted2, r.total, idxs, dists, s);
+                        (int)K, norm, pad, sorted2, r.counts, idxs, dists, s);
     return check_launch("tpo_knn_fwd");
   }
   {  // long reference clouds, few queries: references sliced over workgroups
     const int S = hd_slices(dtype, N, P1, P2, D, K);
     if (S > 0 && workspace && workspace_bytes >= hd_workspace_bytes(N * P1, S, K) && v <= 1) {
       launch_hd(p1, p2, lengths1, lengths2, (int)N, (int)P1, (int)P2, (int)D, (int)K, norm, S,
-                pad, sort_rows, idxs, dists, workspace, s);
+                pad, sort_rows, idxs, dists, workspace, nullptr, s);
       return check_launch("tpo_knn_fwd");
     }
   }

@@ -97,7 +97,7 @@ __global__ __launch_bounds__(256) void knn_feat_prep_kernel(
     const float* __restrict__ p1, const float* __restrict__ p2, const int64_t* __restrict__ len1,
     const int64_t* __restrict__ len2, int N, int P1, int P2, int D, int T1, int T2, int KS,
     uint4* __restrict__ qb, uint4* __restrict__ rb, float2* __restrict__ qinfo,
-    float2* __restrict__ tinfo, uint32_t* __restrict__ redo_counts) {
+    float2* __restrict__ tinfo, RedoList redo) {
   __shared__ float s_c[KF_DMAX];
   __shared__ __align__(16) char s_rows[32 * (9 * 32 + 16)];  // rows of 16 KS bfloat16, 16 bytes apart
   __shared__ float s_max[2][4];
@@ -106,8 +106,7 @@ __global__ __launch_bounds__(256) void knn_feat_prep_kernel(
   const int blk = second ? (int)blockIdx.x - N * T1 : (int)blockIdx.x;
   const int T = second ? T2 : T1;
   const int n = blk / T, t = blk - n * T;
-  if (blockIdx.x == 0)
-    for (int i = tid; i <= N; i += 256) redo_counts[i] = 0u;
+  if (!second && t == 0) redo_clear(redo, n);
   int64_t l1 = len1[n], l2 = len2[n];
   const int L1 = (int)(l1 < 0 ? 0 : (l1 > P1 ? P1 : l1));
   const int L2 = (int)(l2 < 0 ? 0 : (l2 > P2 ? P2 : l2));
@@ -207,7 +206,8 @@ struct KfLds {
   float bound[KF_Q];
   int cnt[KF_Q], bad[KF_Q];
   float red[2][KF_WAVES];
-  float q[KF_Q * (KF_DMAX + 4)];
+  alignas(16) float q[KF_Q * (KF_DMAX + 4)];
+  bool many;
 };
 __host__ __device__ inline int kf_qstride(int D) { return (D + KF_DC - 1) / KF_DC * KF_DC + 4; }
 static_assert(sizeof(KfLds) <= 160 * 1024, "LDS of one CU");
@@ -230,7 +230,6 @@ __global__ __launch_bounds__(KF_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
   const int q0 = qblk * KF_Q;
   const int nq = min(KF_Q, P1 - q0);
   const int size = min(L2, K);
-  const int TE = min(T2, L2);  // tiles with references (reference i T2 + t in tile t)
   const int QS = kf_qstride(D);  // LDS row of a query's floats
   const int j32 = lane & 31, h = lane >> 5;
 
@@ -268,15 +267,19 @@ __global__ __launch_bounds__(KF_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
     for (int i = tid; i < KF_Q * KF_GS / 4; i += KF_THREADS)
       reinterpret_cast<float4*>(sm.gm)[i] = make_float4(inf, inf, inf, inf);
     if (tid < KF_Q) sm.cnt[tid] = 0;
+    if (tid == 0) sm.many = redo_many(redo, blockIdx.x >> 8);
     __syncthreads();
 #pragma unroll
     for (int v = 0; v < KF_WAVES; ++v) {
       dr = fmaxf(dr, sm.red[0][v]);
       lr = fmaxf(lr, sm.red[1][v]);
     }
+    // (rows that are listed unsearched: no tile is looked at)
+    const int TE = __builtin_amdgcn_readfirstlane(sm.many ? 0 : min(T2, L2));
 
     const uint4* __restrict__ rsrc = rb + (size_t)n * T2 * KS * 64 + lane;
-    // tile t's products: acc[b] = the 16 values of column block b of this lane
+    // the tiles with references (reference i T2 + t in tile t), t < TE; tile t's
+    // products: acc[b] = the 16 values of column block b of this lane
     // (rows 8 (v / 4) + 4 h + v % 4); the next tile's operands are loaded first
     auto sweep = [&](auto&& use) {
       fb8_t a[KS];
@@ -391,8 +394,12 @@ __global__ __launch_bounds__(KF_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
           mask &= mask - 1;
           const int qi = 32 * b + j32;
           const int pos = atomicAdd(&sm.cnt[qi], 1);
-          if (pos < KF_CAP)
+          if (pos < KF_CAP) {
             sm.c.key[qi * KF_CS + pos] = (uint32_t)((8 * (v >> 2) + 4 * h + (v & 3)) * T2 + t);
+          } else {  // the list has overflowed: no more of this row
+            lim[b] = -Lim<float>::inf();
+            mask = 0;
+          }
         }
       }
     });
@@ -404,7 +411,7 @@ __global__ __launch_bounds__(KF_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
     // 12k at D = 64), the next step's loads in flight
     {
       const int qi = tid >> 3;
-      const int c = min(sm.cnt[qi], KF_CAP);
+      const int c = sm.cnt[qi] > KF_CAP ? 0 : sm.cnt[qi];  // (an overflowed row is replayed)
       const float* __restrict__ qv = sm.q + qi * QS;
       const float* __restrict__ rbase = p2 + (size_t)n * P2 * D;
       float* __restrict__ st = sm.c.stage[w];
@@ -478,6 +485,8 @@ __global__ __launch_bounds__(KF_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
   // 4. ranks and rows, 8 lanes a query, KF_CE candidates a lane at once
   // against all of the query's
   const int qi = tid >> 3, sub = tid & 7;
+  if (q0 + qi >= L1 && q0 + qi < redo_stride(P1))
+    redo_mark<KF_WAVES>(redo, n, P1, q0 + qi, 0, sub == 0, false, false, 0);
   if (qi >= nq) return;
   const size_t row = (size_t)n * P1 + q0 + qi;
   int64_t* __restrict__ io = idxs + row * K;
@@ -489,7 +498,7 @@ __global__ __launch_bounds__(KF_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
     }
     return;
   }
-  const int c = min(sm.cnt[qi], KF_CAP);
+  const int c = sm.cnt[qi] > KF_CAP ? 0 : sm.cnt[qi];
   bool again = sm.cnt[qi] > KF_CAP || c < size || sm.bad[qi] != 0;
   const uint64_t* __restrict__ keys = sm.c.key + qi * KF_CS;
   for (int e0 = sub; e0 < c; e0 += 8 * KF_CE) {
@@ -528,16 +537,17 @@ __global__ __launch_bounds__(KF_THREADS) __attribute__((amdgpu_waves_per_eu(2)))
     io[s] = pad_sentinel ? -1 : 0;
     dout[s] = pad_d;
   }
-  if (((__ballot(again) >> (lane & 56)) & 0xff) != 0 && sub == 0) redo_push(redo, n, P1, q0 + qi);
+  redo_mark<KF_WAVES>(redo, n, P1, q0 + qi, q0 + qi, sub == 0,
+                      ((__ballot(again) >> (lane & 56)) & 0xff) != 0, w == 0, blockIdx.x >> 8);
 }
 
 template <int KS>
 void kf_launch(const void* p1, const void* p2, const int64_t* l1, const int64_t* l2, int N, int P1,
-               int P2, int D, int K, int pad, bool sort, const KfLayout& L, char* ws,
-               int64_t* idxs, void* dists, hipStream_t s) {
+               int P2, int D, int K, int pad, bool sort, const KfLayout& L, int64_t limit,
+               char* ws, int64_t* idxs, void* dists, hipStream_t s) {
   const int T1 = kf_tiles1(P1), T2 = kf_tiles2(P2);
   const int vec4 = D % 4 == 0 && (((uintptr_t)p2) & 15) == 0;
-  const RedoList redo = redo_at(ws + L.redo, N, P1);
+  const RedoList redo = redo_at(ws + L.redo, N, P1, limit);
   const dim3 g((unsigned)(N * (T1 / 2))), b(KF_THREADS);
 #define KNN_FEAT(SORT)                                                                           \
   hipLaunchKernelGGL((knn_feat_kernel<KS, SORT>), g, b, 0, s, (const float*)p1,                  \
@@ -551,6 +561,22 @@ void kf_launch(const void* p1, const void* p2, const int64_t* l1, const int64_t*
 }
 
 }  // namespace
+
+// Rows replayed one a workgroup at most: where that takes as long as the
+// kernels that take all of them (sliced: knn_hd_*_kernel; else a lane a row).
+// A replayed row takes about 25 + K / 2 ns and 5 + D / 5 ps a reference, the
+// lane-a-row kernel, up to 65536 rows, per reference 72 D ns (D <= 12), 115 D
+// ns, 0.6 us (D = 64) or 1.3 us (D = 128), the sliced kernels 0.33 D ns.
+// 8 x 2048 x 2048, K = 20, D = 64, every row tied: 1360 us against 2650; 4 x
+// 4096 x 16384, D = 9: 4800 against 10600; 8 x 4096 x 512, D = 4: 900 against
+// 380.
+static int64_t kf_redo_limit(int64_t P2, int64_t D, int64_t K, bool sliced) {
+  const double row = 25 + 0.5 * K + P2 * (5 + 0.2 * D) * 1e-3;
+  const double ref = sliced ? 0.33 * D : D == 64 ? 600 : D == 128 ? 1300
+                                       : D <= 12 ? 72.0 * D : 115.0 * D;
+  const double n = P2 * ref / row;
+  return n < 1024 ? 1024 : n > (1 << 20) ? 1 << 20 : (int64_t)n;
+}
 
 // Short clouds stay with a query a lane (knn_fwd_kernel).  Beyond what one launch
 // takes, that one costs about ref_ns a reference and 0.8 us a neighbour, more
@@ -582,27 +608,26 @@ int64_t knn_feat_workspace(int64_t N, int64_t P1, int64_t P2, int64_t D) {
 }
 
 RedoList launch_knn_feat(const void* p1, const void* p2, const int64_t* l1, const int64_t* l2,
-                         int N, int P1, int P2, int D, int K, int pad, bool sort, int64_t* idxs,
-                         void* dists, void* ws, hipStream_t s) {
+                         int N, int P1, int P2, int D, int K, int pad, bool sort, bool sliced,
+                         int64_t* idxs, void* dists, void* ws, hipStream_t s) {
   const KfLayout L = kf_layout(N, P1, P2, D);
+  const int64_t limit = kf_redo_limit(P2, D, K, sliced);
   char* w = (char*)ws;
   const int KS = kf_ksteps(D), T1 = kf_tiles1(P1), T2 = kf_tiles2(P2);
-  const RedoList redo = redo_at(w + L.redo, N, P1);
+  const RedoList redo = redo_at(w + L.redo, N, P1, limit);
   hipLaunchKernelGGL(knn_feat_prep_kernel, dim3((unsigned)(N * (T1 + T2))), dim3(256), 0, s,
                      (const float*)p1, (const float*)p2, l1, l2, N, P1, P2, D, T1, T2, KS,
                      (uint4*)(w + L.qb), (uint4*)(w + L.rb), (float2*)(w + L.qinfo),
-                     (float2*)(w + L.tinfo), redo.total);
+                     (float2*)(w + L.tinfo), redo);
+#define KF_CASE(KS)                                                                             \
+  case KS:                                                                                     \
+    kf_launch<KS>(p1, p2, l1, l2, N, P1, P2, D, K, pad, sort, L, limit, w, idxs, dists, s);     \
+    break
   switch (KS) {
-    case 1: kf_launch<1>(p1, p2, l1, l2, N, P1, P2, D, K, pad, sort, L, w, idxs, dists, s); break;
-    case 2: kf_launch<2>(p1, p2, l1, l2, N, P1, P2, D, K, pad, sort, L, w, idxs, dists, s); break;
-    case 3: kf_launch<3>(p1, p2, l1, l2, N, P1, P2, D, K, pad, sort, L, w, idxs, dists, s); break;
-    case 4: kf_launch<4>(p1, p2, l1, l2, N, P1, P2, D, K, pad, sort, L, w, idxs, dists, s); break;
-    case 5: kf_launch<5>(p1, p2, l1, l2, N, P1, P2, D, K, pad, sort, L, w, idxs, dists, s); break;
-    case 6: kf_launch<6>(p1, p2, l1, l2, N, P1, P2, D, K, pad, sort, L, w, idxs, dists, s); break;
-    case 7: kf_launch<7>(p1, p2, l1, l2, N, P1, P2, D, K, pad, sort, L, w, idxs, dists, s); break;
-    case 8: kf_launch<8>(p1, p2, l1, l2, N, P1, P2, D, K, pad, sort, L, w, idxs, dists, s); break;
-    default: kf_launch<9>(p1, p2, l1, l2, N, P1, P2, D, K, pad, sort, L, w, idxs, dists, s); break;
+    KF_CASE(1); KF_CASE(2); KF_CASE(3); KF_CASE(4); KF_CASE(5);
+    KF_CASE(6); KF_CASE(7); KF_CASE(8); KF_CASE(9);
   }
+#undef KF_CASE
   return redo;
 }
 

@@ -250,7 +250,7 @@ __global__ __launch_bounds__(1024) void knn_grid_setup_kernel(
 
 // The grid is knn_grid_setup_kernel's (list), or knn_near_setup_kernel's
 // (REDO: records with the index in w, its own cells an axis); `order` then
-// holds a RedoList's queries, of which there must be over REDO_LIMIT in all.
+// holds a RedoList's queries and `redo` their counts.
 template <int NORM, int KC, bool SORT, bool REDO>
 __global__ __launch_bounds__(256) void knn_grid_kernel(
     const float* __restrict__ p1, const float* __restrict__ p2, const int64_t* __restrict__ len1,
@@ -259,7 +259,6 @@ __global__ __launch_bounds__(256) void knn_grid_kernel(
     const int32_t* __restrict__ list, int cells_max, const uint32_t* __restrict__ redo, int P1,
     int P2, int K, int A, int nqb, int words, int pad_sentinel, int64_t* __restrict__ idxs,
     float* __restrict__ dists) {
-  if (REDO && redo[0] <= REDO_LIMIT) return;
   // LDS per wave: `words` bitmask words, a window of KG_WIN candidate
   // indices, and the current chunk's distances ([entry][lane])
   extern __shared__ uint32_t kg_lds[];
@@ -268,6 +267,9 @@ __global__ __launch_bounds__(256) void knn_grid_kernel(
   int32_t* __restrict__ cl = reinterpret_cast<int32_t*>(bm + words);
   float* __restrict__ dl = reinterpret_cast<float*>(cl + KG_WIN) + lane;
   const int n = blockIdx.x / nqb;
+  const int i0 = (blockIdx.x - n * nqb) * 256, i = i0 + threadIdx.x;  // position in processing order
+  const int positions = REDO ? (int)redo[n] : P1;
+  if (REDO && i0 >= positions) return;  // (usually nothing is listed)
   int64_t l1 = len1[n], l2 = len2[n];
   l1 = l1 < 0 ? 0 : (l1 > P1 ? P1 : l1);
   l2 = l2 < 0 ? 0 : (l2 > P2 ? P2 : l2);
@@ -275,9 +277,8 @@ __global__ __launch_bounds__(256) void knn_grid_kernel(
   const int Ae = min(A, L2);
   const float* __restrict__ rp = p2 + (size_t)n * P2 * 3;
 
-  const int i = (blockIdx.x - n * nqb) * 256 + threadIdx.x;  // position in processing order
-  const bool in_range = i < (REDO ? (int)redo[1 + n] : P1);
-  const int q = in_range ? order[(size_t)n * P1 + i] : 0;
+  const bool in_range = i < positions;
+  const int q = in_range ? order[n * (REDO ? (size_t)redo_stride(P1) : (size_t)P1) + i] : 0;
   const size_t row = (size_t)n * P1 + q;
   int64_t* __restrict__ io = idxs + row * K;
   float* __restrict__ dout = dists + row * K;
@@ -650,7 +651,7 @@ void launch_knn_grid_redo(const void* p1, const void* p2, const int64_t* l1, con
                           int N, int P1, int P2, int K, int norm, int pad, const float* hdr,
                           const int32_t* cs, int cells_max, const float* records, const RedoList& r,
                           int64_t* idxs, void* dists, hipStream_t s) {
-  KgArgs a{p1, p2, l1, l2, r.queries, hdr, cs, (const int32_t*)records, cells_max, r.total, N, P1,
+  KgArgs a{p1, p2, l1, l2, r.queries, hdr, cs, (const int32_t*)records, cells_max, r.counts, N, P1,
            P2, K, kg_prefix(K, P2), pad, idxs, dists, s};
   if (norm == 1) kg_launch_k<1, true, true>(a);
   else kg_launch_k<2, true, true>(a);

@@ -27,6 +27,7 @@ namespace {
 // replay's state equals the real state at every real insertion), so the
 // slot layout and values are the single sequential pass's, bit for bit.  A
 // slice with more than HD_CAP candidates is recomputed by the merge.
+// only: where not null, the clouds it has no count for are left alone.
 //
 // Reference points reach the lanes through DPP: each 16-lane row of the wave
 // loads the same reference row with ordinary vector loads (lane k of a row:
@@ -105,14 +106,15 @@ HdLayout hd_layout(int64_t rows, int64_t S, int64_t K) {
 template <int DT, int NORM, int KC>
 __global__ __launch_bounds__(256) void knn_hd_slice_kernel(
     const float* __restrict__ p1, const float* __restrict__ p2, const int64_t* __restrict__ len1,
-    const int64_t* __restrict__ len2, int P1, int P2, int K, int nqb, int S, int slen,
-    int32_t* __restrict__ cnt, float* __restrict__ cd, int32_t* __restrict__ ci,
-    float* __restrict__ fd) {
+    const int64_t* __restrict__ len2, const uint32_t* __restrict__ only, int P1, int P2, int K,
+    int nqb, int S, int slen, int32_t* __restrict__ cnt, float* __restrict__ cd,
+    int32_t* __restrict__ ci, float* __restrict__ fd) {
   constexpr int G = DT / 64;
   __shared__ float s_d[4][32][64];
   const int sl = blockIdx.x % S;
   const int nb = blockIdx.x / S;
   const int n = nb / nqb;
+  if (only && only[n] == 0u) return;
   const int w = wave_id(), lane = lane_id();
   const int qw = (nb - n * nqb) * 256 + 64 * w;
   if (qw >= P1) return;  // the whole wave
@@ -229,7 +231,8 @@ __global__ __launch_bounds__(256) void knn_hd_slice_kernel(
 template <int DT, int NORM, int KC, bool SORT>
 __global__ __launch_bounds__(256) void knn_hd_merge_kernel(
     const float* __restrict__ p1, const float* __restrict__ p2, const int64_t* __restrict__ len1,
-    const int64_t* __restrict__ len2, int N, int P1, int P2, int K, int S, int slen, int pad_sentinel,
+    const int64_t* __restrict__ len2, const uint32_t* __restrict__ only, int N, int P1, int P2,
+    int K, int S, int slen, int pad_sentinel,
     const int32_t* __restrict__ cnt, const float* __restrict__ cd,
     const int32_t* __restrict__ ci, const float* __restrict__ fd, int64_t* __restrict__ idxs,
     float* __restrict__ dists) {
@@ -237,6 +240,7 @@ __global__ __launch_bounds__(256) void knn_hd_merge_kernel(
   if (row >= (int64_t)N * P1) return;  // the whole wave
   const int lane = lane_id();
   const int n = (int)(row / P1), q = (int)(row - (int64_t)n * P1);
+  if (only && only[n] == 0u) return;
   int64_t l1 = len1[n], l2 = len2[n];
   l1 = l1 < 0 ? 0 : (l1 > P1 ? P1 : l1);
   l2 = l2 < 0 ? 0 : (l2 > P2 ? P2 : l2);
@@ -324,7 +328,7 @@ namespace {
 template <int DT, int NORM, int KC>
 void launch_hd_kc(const void* p1, const void* p2, const int64_t* l1, const int64_t* l2, int N,
                   int P1, int P2, int K, int S, int pad, bool sort, int64_t* idxs, void* dists,
-                  void* ws, hipStream_t s) {
+                  void* ws, const uint32_t* only, hipStream_t s) {
   const int nqb = (P1 + 255) / 256;
   const int slen = (P2 - K + S - 1) / S;
   const HdLayout L = hd_layout((int64_t)N * P1, S, K);
@@ -333,26 +337,27 @@ void launch_hd_kc(const void* p1, const void* p2, const int64_t* l1, const int64
   int32_t* ci = (int32_t*)((char*)ws + L.idx);
   float* fd = (float*)((char*)ws + L.fill);
   hipLaunchKernelGGL((knn_hd_slice_kernel<DT, NORM, KC>), dim3(N * nqb * S), dim3(256), 0, s,
-                     (const float*)p1, (const float*)p2, l1, l2, P1, P2, K, nqb, S, slen, cnt, cd,
+                     (const float*)p1, (const float*)p2, l1, l2, only, P1, P2, K, nqb, S, slen,
+                     cnt, cd,
                      ci, fd);
   const unsigned mg = (unsigned)(((int64_t)N * P1 + 3) / 4);  // a wave per row
   if (sort)
     hipLaunchKernelGGL((knn_hd_merge_kernel<DT, NORM, KC, true>), dim3(mg), dim3(256), 0, s,
-                       (const float*)p1, (const float*)p2, l1, l2, N, P1, P2, K, S, slen, pad, cnt,
+                       (const float*)p1, (const float*)p2, l1, l2, only, N, P1, P2, K, S, slen, pad, cnt,
                        cd, ci, fd, idxs, (float*)dists);
   else
     hipLaunchKernelGGL((knn_hd_merge_kernel<DT, NORM, KC, false>), dim3(mg), dim3(256), 0, s,
-                       (const float*)p1, (const float*)p2, l1, l2, N, P1, P2, K, S, slen, pad, cnt,
+                       (const float*)p1, (const float*)p2, l1, l2, only, N, P1, P2, K, S, slen, pad, cnt,
                        cd, ci, fd, idxs, (float*)dists);
 }
 
 template <int DT, int NORM>
 void launch_hd_norm(const void* p1, const void* p2, const int64_t* l1, const int64_t* l2, int N,
                     int P1, int P2, int K, int S, int pad, bool sort, int64_t* idxs, void* dists,
-                    void* ws, hipStream_t s) {
-  if (K <= 8) launch_hd_kc<DT, NORM, 8>(p1, p2, l1, l2, N, P1, P2, K, S, pad, sort, idxs, dists, ws, s);
-  else if (K <= 16) launch_hd_kc<DT, NORM, 16>(p1, p2, l1, l2, N, P1, P2, K, S, pad, sort, idxs, dists, ws, s);
-  else launch_hd_kc<DT, NORM, 32>(p1, p2, l1, l2, N, P1, P2, K, S, pad, sort, idxs, dists, ws, s);
+                    void* ws, const uint32_t* only, hipStream_t s) {
+  if (K <= 8) launch_hd_kc<DT, NORM, 8>(p1, p2, l1, l2, N, P1, P2, K, S, pad, sort, idxs, dists, ws, only, s);
+  else if (K <= 16) launch_hd_kc<DT, NORM, 16>(p1, p2, l1, l2, N, P1, P2, K, S, pad, sort, idxs, dists, ws, only, s);
+  else launch_hd_kc<DT, NORM, 32>(p1, p2, l1, l2, N, P1, P2, K, S, pad, sort, idxs, dists, ws, only, s);
 }
 
 }  // namespace
@@ -363,13 +368,13 @@ int64_t hd_workspace_bytes(int64_t rows, int64_t S, int64_t K) {
 
 void launch_hd(const void* p1, const void* p2, const int64_t* l1, const int64_t* l2, int N, int P1,
                int P2, int D, int K, int norm, int S, int pad, bool sort, int64_t* idxs,
-               void* dists, void* ws, hipStream_t s) {
+               void* dists, void* ws, const uint32_t* only, hipStream_t s) {
   if (D == 128) {
-    if (norm == 1) launch_hd_norm<128, 1>(p1, p2, l1, l2, N, P1, P2, K, S, pad, sort, idxs, dists, ws, s);
-    else launch_hd_norm<128, 2>(p1, p2, l1, l2, N, P1, P2, K, S, pad, sort, idxs, dists, ws, s);
+    if (norm == 1) launch_hd_norm<128, 1>(p1, p2, l1, l2, N, P1, P2, K, S, pad, sort, idxs, dists, ws, only, s);
+    else launch_hd_norm<128, 2>(p1, p2, l1, l2, N, P1, P2, K, S, pad, sort, idxs, dists, ws, only, s);
   } else {
-    if (norm == 1) launch_hd_norm<64, 1>(p1, p2, l1, l2, N, P1, P2, K, S, pad, sort, idxs, dists, ws, s);
-    else launch_hd_norm<64, 2>(p1, p2, l1, l2, N, P1, P2, K, S, pad, sort, idxs, dists, ws, s);
+    if (norm == 1) launch_hd_norm<64, 1>(p1, p2, l1, l2, N, P1, P2, K, S, pad, sort, idxs, dists, ws, only, s);
+    else launch_hd_norm<64, 2>(p1, p2, l1, l2, N, P1, P2, K, S, pad, sort, idxs, dists, ws, only, s);
   }
 }
 

@@ -6,7 +6,8 @@
 // roundings) in order, and where no two of the first K + 1 are equal their
 // indices are the reference's.  Rows with equal distances, or values that are
 // not finite, are listed and replayed (knn_replay.hpp): the order of equal
-// distances depends on the MinK process's history.
+// distances depends on the MinK process's history.  Lists too long for that go
+// to the kernels that take a lane a row (kn_redo_limit).
 //
 // knn_near_setup_kernel, a workgroup a cloud: references as (x, y, z, index)
 //   records by cell of a G^3 grid, cells row-major in x, y, z (a line of
@@ -52,6 +53,11 @@ inline int kn_gmax(int64_t P2) {
   return g;
 }
 constexpr int KN_WAVES = 4;
+// Rows replayed one a workgroup at most, about where the lane-a-row kernels
+// take as long for all of them: a row takes 30-60 ns among 2048 references and
+// fewer, 0.11-0.17 us among 16384; those kernels 45-174 us (512 references, K =
+// 3 .. 32), 64-320 (2048), 200-1000 (16384).
+inline int64_t kn_redo_limit(int64_t P2, int64_t K) { return 1400 + (P2 < 2048 ? 40 : 80) * K; }
 constexpr int KN_PPT = 16;  // clouds of up to 1024 KN_PPT points stay in registers in the setup
 
 // ------------------------------------------------------------------- DPP
@@ -296,10 +302,9 @@ __global__ __launch_bounds__(1024) void knn_near_setup_kernel(
     const float* __restrict__ p1, const int64_t* __restrict__ len1, int P1,
     const float* __restrict__ p2, const int64_t* __restrict__ len2, int P2, int N, int K,
     int gmax, float* __restrict__ hdr, int32_t* __restrict__ cstart, float4* __restrict__ rrec,
-    float4* __restrict__ qrec, uint32_t* __restrict__ redo_counts) {
+    float4* __restrict__ qrec, RedoList redo) {
   __shared__ KnLds sm;
-  if (blockIdx.x == 0)
-    for (int i = threadIdx.x; i <= N; i += 1024) redo_counts[i] = 0u;
+  if ((int)blockIdx.x < N) redo_clear(redo, blockIdx.x);
   if ((int)blockIdx.x >= N) {
     const int n = blockIdx.x - N;
     const int64_t l1 = len1[n];
@@ -412,10 +417,15 @@ __global__ __launch_bounds__(256) void knn_near_kernel(
   const int blk = xcd_logical_block(blockIdx.x, gridDim.x);  // a cloud's blocks share an XCD's L2
   const int n = blk / nqb;
   int64_t l1 = len1[n], l2 = len2[n];
+  const int epoch = blockIdx.x >> 11;
+  const bool many = redo_many(redo, epoch);
   const int L1 = (int)(l1 < 0 ? 0 : (l1 > P1 ? P1 : l1));
   const int L2 = (int)(l2 < 0 ? 0 : (l2 > P2 ? P2 : l2));
   const int i0 = ((blk - n * nqb) * KN_WAVES + w) * 4;  // the wave's first position in query order
-  if (i0 >= P1) return;
+  if (i0 >= P1) {  // (a workgroup's 16 places are whole)
+    redo_mark<32>(redo, n, P1, i0 + g, 0, l16 == 0, false, false, 0);
+    return;
+  }
   const int i = i0 + g;
   const bool in_range = i < P1, act = i < L1;  // valid rows come first in the order
   int q = min(i, P1 - 1);
@@ -443,8 +453,8 @@ __global__ __launch_bounds__(256) void knn_near_kernel(
     const float4* __restrict__ rr = rrec + (size_t)n * P2;
     const bool fin = __float_as_int(h[7]) == 0 && __builtin_fabsf(qr[0]) < inf &&
                      __builtin_fabsf(qr[1]) < inf && __builtin_fabsf(qr[2]) < inf;
+    bool go = act && fin;  // rows that search
     again = act && !fin;
-    const bool go = act && fin;  // rows that search
     KnSides sides;
 #pragma unroll
     for (int b = 0; b < 4; ++b) sides.bit[b] = (lane >> b) & 1 ? inf : -inf;
@@ -555,6 +565,10 @@ __global__ __launch_bounds__(256) void knn_near_kernel(
       // without a ring the K nearest are often outside: only with many points
       open = open && cnt < (ring == 0 ? 4 * K : K) && ring < G;
     }
+    if (many) {  // (listed unsearched)
+      again = act;
+      go = false;
+    }
     sweep(box, go, false, box);
     if constexpr (R == 0) T = row_all(best[0].d, [](float a, float b) { return min_of(a, b); });
     // 2. the box of everything at or below the K-th distance
@@ -607,7 +621,7 @@ __global__ __launch_bounds__(256) void knn_near_kernel(
     }
   }
   const bool row_again = ((__ballot(again) >> (16 * g)) & 0xffff) != 0;
-  if (row_again && l16 == 0) redo_push(redo, n, P1, q);
+  redo_mark<32>(redo, n, P1, i, q, l16 == 0, row_again, w == 0 && (blk & 7) == 0, epoch);
 }
 
 struct KnLayout {
@@ -689,7 +703,7 @@ RedoList launch_knn_near(const void* p1, const void* p2, const int64_t* l1, cons
   float* hdr = (float*)(w + L.hdr);
   int32_t* cs = (int32_t*)(w + L.cstart);
   float4 *rrec = (float4*)(w + L.rrec), *qrec = (float4*)(w + L.qrec);
-  const RedoList redo = redo_at(w + L.redo, N, P1);
+  const RedoList redo = redo_at(w + L.redo, N, P1, kn_redo_limit(P2, K));
   // The queries' order pays (neighbouring rows share cells, and rows with
   // wide boxes one another's waves: 42 against 49 us at 16 x 2048 x 2048)
   // where it is made beside the references' grid; more queries than
@@ -697,13 +711,14 @@ RedoList launch_knn_near(const void* p1, const void* p2, const int64_t* l1, cons
   // for 34 against 36 us).
   const bool order = P1 <= P2;
   const int gmax = kn_gmax(P2), cells_max = gmax * gmax * gmax;
-  hipLaunchKernelGGL(knn_near_setup_kernel, dim3(order ? 2 * N : N), dim3(1024), 0, s, (const float*)p1, l1, P1,
-                     (const float*)p2, l2, P2, N, K, gmax, hdr, cs, rrec, qrec, redo.total);
+  hipLaunchKernelGGL(knn_near_setup_kernel, dim3(order ? 2 * N : N), dim3(1024), 0, s,
+                     (const float*)p1, l1, P1, (const float*)p2, l2, P2, N, K, gmax, hdr, cs, rrec,
+                     qrec, redo);
   const int nqb = (P1 + 4 * KN_WAVES - 1) / (4 * KN_WAVES);
 #define KNN_NEAR(NORM, R)                                                                        \
   hipLaunchKernelGGL((knn_near_kernel<NORM, R>), dim3(N * nqb), dim3(256), 0, s, l1, l2, hdr, cs, \
-                     rrec, (const float*)p1, order ? qrec : nullptr, cells_max, P1, P2, K, nqb, pad, redo,    \
-                     idxs, (float*)dists)
+                     rrec, (const float*)p1, order ? qrec : nullptr, cells_max, P1, P2, K, nqb,   \
+                     pad, redo, idxs, (float*)dists)
 #define KNN_NEAR_K(NORM)                \
   do {                                  \
     if (!sort) KNN_NEAR(NORM, 0);       \
@@ -714,7 +729,8 @@ RedoList launch_knn_near(const void* p1, const void* p2, const int64_t* l1, cons
   else KNN_NEAR_K(2);
 #undef KNN_NEAR_K
 #undef KNN_NEAR
-  launch_knn_redo(p1, p2, l1, l2, N, P1, P2, 3, K, norm, pad, sort, redo, idxs, dists, s);
+  launch_knn_redo(p1, p2, l1, l2, N, P1, P2, 3, K, norm, pad, sort, redo,
+                  order ? REDO_RECORDS : REDO_ROWS_3D, order ? qrec : nullptr, idxs, dists, s);
   if (grid_redo)
     launch_knn_grid_redo(p1, p2, l1, l2, N, P1, P2, K, norm, pad, hdr, cs, cells_max,
                          (const float*)rrec, redo, idxs, dists, s);

@@ -118,39 +118,98 @@ struct ReplayRow {
 };
 
 // Rows whose order the distances alone do not decide (equal distances, or
-// values that are not finite): a total count, the rows as n P1 + q in the
-// order of arrival, and per cloud a count and the query numbers.  Up to
-// REDO_LIMIT rows are replayed one a workgroup (launch_knn_redo); more go to
-// the lane-a-row kernel, cloud by cloud.
-constexpr int REDO_LIMIT = 2048;
-
+// values that are not finite) are flagged at their place in the processing
+// order.  Up to about `limit` of them are replayed one a workgroup
+// (launch_knn_redo); more go to the lane-a-row kernels, whose waves want
+// neighbouring queries: each group of 16 places with a flag is handed over
+// whole, in that order.  Flags are plain stores, and of the waves that list
+// rows a few count them: a count by every one took 25 ns a row (149 us instead
+// of 30 for the search of 64 x 1024 x 1024 points on a 256^3 lattice).  Which
+// way the rows go changes no result, so an estimate is enough.
 struct RedoList {
-  uint32_t* total;  // [1], then counts[N]
-  uint32_t* rows;   // [N P1]
-  int32_t* queries; // [N P1], cloud n's from n P1
+  uint32_t* guess;   // [2] about the number of listed rows; whether there are any
+  uint32_t* epochs;  // [REDO_EPOCHS] lines: about the number listed in the epoch before
+  uint32_t* counts;  // [N] queries of a cloud that the lane-a-row kernels take
+  uint8_t* flags;    // [N stride] places, cloud by cloud
+  int32_t* queries;  // [N stride] the listed rows n P1 + q by place, then those queries
+  uint32_t limit;
 };
-__device__ __forceinline__ void redo_push(const RedoList& r, int n, int P1, int q) {
-  const uint32_t a = atomicAdd(r.total, 1u);
-  r.rows[a] = (uint32_t)n * (uint32_t)P1 + (uint32_t)q;
-  const uint32_t b = atomicAdd(r.total + 1 + n, 1u);
-  r.queries[(size_t)n * P1 + b] = q;
+// places a cloud: whole groups of 16
+__host__ __device__ inline int64_t redo_stride(int64_t P1) { return (P1 + 15) / 16 * 16; }
+// Workgroups go by epochs, about as many at a time as the GPU holds.  Once more
+// rows than the limit were listed in the epoch before, the rows of a workgroup
+// may as well all be listed unsearched.  An epoch's count is a line of its own,
+// first read when the count is made: a line read before would be read again from
+// the L2 as it was (a load at device scope misses it: 1.5 us of 55 for 8 x 16384
+// queries).
+constexpr int REDO_EPOCHS = 64, REDO_LINE = 32;
+__device__ __forceinline__ bool redo_many(const RedoList& r, int epoch) {
+  return r.epochs[(epoch < REDO_EPOCHS ? epoch : REDO_EPOCHS - 1) * REDO_LINE] > r.limit;
 }
-inline int64_t redo_bytes(int64_t N, int64_t P1) {
-  auto up = [](int64_t x) { return (x + 255) / 256 * 256; };
-  return up((N + 1) * 4) + 2 * up(N * P1 * 4);
+// Every place gets its flag, the places past the cloud's rows too; `mark` is the
+// lane that has one.  Lists row q of cloud n, at `place`, where `again`.
+// counts: the wave is the one in SAMPLE that counts its rows.
+template <int SAMPLE>
+__device__ __forceinline__ void redo_mark(const RedoList& r, int n, int P1, int place, int q,
+                                          bool mark, bool again, bool counts, int epoch) {
+  const int64_t at = n * redo_stride(P1) + place;
+  if (mark) r.flags[at] = again ? 1 : 0;
+  const uint64_t m = __ballot(mark && again);
+  if (m == 0) return;
+  if (mark && again) {
+    r.queries[at] = (int32_t)((uint32_t)n * (uint32_t)P1 + (uint32_t)q);
+    r.guess[1] = 1u;
+  }
+  if (counts && lane_id() == __builtin_ctzll(m)) {
+    const uint32_t c = (uint32_t)(SAMPLE * __builtin_popcountll(m));
+    atomicAdd(r.guess, c);
+    if (epoch + 1 < REDO_EPOCHS) atomicAdd(r.epochs + (epoch + 1) * REDO_LINE, c);
+  }
 }
-inline RedoList redo_at(void* ws, int64_t N, int64_t P1) {
+// The kernel before clears the counts, cloud n's by (at least 64) threads of one
+// workgroup.
+__device__ __forceinline__ void redo_clear(const RedoList& r, int n) {
+  if (threadIdx.x == 0) r.counts[n] = 0u;
+  if (n == 0 && threadIdx.x < 2) r.guess[threadIdx.x] = 0u;
+  if (n == 0 && threadIdx.x < REDO_EPOCHS) r.epochs[threadIdx.x * REDO_LINE] = 0u;
+}
+inline RedoList redo_at(void* ws, int64_t N, int64_t P1, int64_t limit, int64_t* bytes = nullptr) {
   auto up = [](int64_t x) { return (x + 255) / 256 * 256; };
+  const int64_t places = N * redo_stride(P1);
   RedoList r;
-  r.total = (uint32_t*)ws;
-  r.rows = (uint32_t*)((char*)ws + up((N + 1) * 4));
-  r.queries = (int32_t*)((char*)r.rows + up(N * P1 * 4));
+  char* at = (char*)ws;
+  r.guess = (uint32_t*)at;
+  r.counts = r.guess + 2;
+  at += up((N + 2) * 4);
+  r.epochs = (uint32_t*)at;
+  at += REDO_EPOCHS * REDO_LINE * 4;
+  r.flags = (uint8_t*)at;
+  at += up(places);
+  r.queries = (int32_t*)at;
+  at += up(places * 4);
+  r.limit = (uint32_t)limit;
+  if (bytes) *bytes = at - (char*)ws;
   return r;
 }
+inline int64_t redo_bytes(int64_t N, int64_t P1) {
+  int64_t b;
+  redo_at(nullptr, N, P1, 0, &b);
+  return b;
+}
 
-// knn_redo.hip: the listed rows' MinK process (float), a workgroup a row
+// How the places of a RedoList's flags stand for queries.
+enum RedoPlaces {
+  REDO_ROWS,     // place p is row p, in no particular order
+  REDO_ROWS_3D,  // place p is row p, a 3-D point: put in spatial order first
+  REDO_RECORDS   // records (x, y, z, row) in spatial order
+};
+
+// knn_redo.hip: the listed rows' MinK process (float), a workgroup a row; or,
+// where they are more than the limit, the lists that the lane-a-row kernels
+// take.
 void launch_knn_redo(const void* p1, const void* p2, const int64_t* l1, const int64_t* l2, int N,
                      int P1, int P2, int D, int K, int norm, int pad, bool sort, const RedoList& r,
-                     int64_t* idxs, void* dists, hipStream_t s);
+                     RedoPlaces places, const float4* records, int64_t* idxs, void* dists,
+                     hipStream_t s);
 
 }  // namespace tpo
