@@ -422,8 +422,11 @@ __global__ __launch_bounds__(256) void knn_near_kernel(
   const int L1 = (int)(l1 < 0 ? 0 : (l1 > P1 ? P1 : l1));
   const int L2 = (int)(l2 < 0 ? 0 : (l2 > P2 ? P2 : l2));
   const int i0 = ((blk - n * nqb) * KN_WAVES + w) * 4;  // the wave's first position in query order
-  if (i0 >= P1) {  // (a workgroup's 16 places are whole)
-    redo_mark<32>(redo, n, P1, i0 + g, 0, l16 == 0, false, false, 0);
+  // the wave's four flags (a workgroup's 16 places are whole)
+  uint32_t* __restrict__ flags =
+      reinterpret_cast<uint32_t*>(redo.flags + n * redo_stride(P1) + i0);
+  if (i0 >= P1) {
+    if (lane == 0) *flags = 0u;
     return;
   }
   const int i = i0 + g;
@@ -453,8 +456,8 @@ __global__ __launch_bounds__(256) void knn_near_kernel(
     const float4* __restrict__ rr = rrec + (size_t)n * P2;
     const bool fin = __float_as_int(h[7]) == 0 && __builtin_fabsf(qr[0]) < inf &&
                      __builtin_fabsf(qr[1]) < inf && __builtin_fabsf(qr[2]) < inf;
-    bool go = act && fin;  // rows that search
-    again = act && !fin;
+    const bool go = act && fin && !many;  // rows that search (many: listed unsearched)
+    again = act && !go;
     KnSides sides;
 #pragma unroll
     for (int b = 0; b < 4; ++b) sides.bit[b] = (lane >> b) & 1 ? inf : -inf;
@@ -565,10 +568,6 @@ __global__ __launch_bounds__(256) void knn_near_kernel(
       // without a ring the K nearest are often outside: only with many points
       open = open && cnt < (ring == 0 ? 4 * K : K) && ring < G;
     }
-    if (many) {  // (listed unsearched)
-      again = act;
-      go = false;
-    }
     sweep(box, go, false, box);
     if constexpr (R == 0) T = row_all(best[0].d, [](float a, float b) { return min_of(a, b); });
     // 2. the box of everything at or below the K-th distance
@@ -620,8 +619,13 @@ __global__ __launch_bounds__(256) void knn_near_kernel(
       }
     }
   }
-  const bool row_again = ((__ballot(again) >> (16 * g)) & 0xffff) != 0;
-  redo_mark<32>(redo, n, P1, i, q, l16 == 0, row_again, w == 0 && (blk & 7) == 0, epoch);
+  const uint64_t any = __ballot(again);
+  if (any == 0) {
+    if (lane == 0) *flags = 0u;
+  } else {
+    redo_mark<32>(redo, n, P1, i, q, l16 == 0, ((any >> (16 * g)) & 0xffff) != 0,
+                  w == 0 && (blk & 7) == 0, epoch);
+  }
 }
 
 struct KnLayout {

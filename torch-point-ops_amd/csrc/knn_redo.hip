@@ -11,7 +11,7 @@
 // us among 16384 (K = 3 .. 32).  Lists past their limit become the lane-a-row
 // kernels' lists here: groups of 16 neighbouring queries, so that those kernels
 // meet the order they are made for.  8 x 16384 x 16384 points of a 16^3
-// lattice, K = 3, every row tied: 298 us with all steps; listed row by row as
+// lattice, K = 3, every row tied: 296 us with all steps; listed row by row as
 // they arrived 1388.
 #include "knn_order.hpp"
 #include "knn_replay.hpp"

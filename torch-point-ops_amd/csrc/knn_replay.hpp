@@ -144,7 +144,9 @@ __host__ __device__ inline int64_t redo_stride(int64_t P1) { return (P1 + 15) / 
 // queries).
 constexpr int REDO_EPOCHS = 64, REDO_LINE = 32;
 __device__ __forceinline__ bool redo_many(const RedoList& r, int epoch) {
-  return r.epochs[(epoch < REDO_EPOCHS ? epoch : REDO_EPOCHS - 1) * REDO_LINE] > r.limit;
+  typedef const __attribute__((address_space(4))) uint32_t* Scalar;  // (a scalar load)
+  const int line = (epoch < REDO_EPOCHS ? epoch : REDO_EPOCHS - 1) * REDO_LINE;
+  return ((Scalar)(uintptr_t)r.epochs)[line] > r.limit;
 }
 // Every place gets its flag, the places past the cloud's rows too; `mark` is the
 // lane that has one.  Lists row q of cloud n, at `place`, where `again`.
