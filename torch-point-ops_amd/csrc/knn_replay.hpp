@@ -142,7 +142,7 @@ __host__ __device__ inline int64_t redo_stride(int64_t P1) { return (P1 + 15) / 
 // first read when the count is made: a line read before would be read again from
 // the L2 as it was (a load at device scope misses it: 1.5 us of 55 for 8 x 16384
 // queries).
-constexpr int REDO_EPOCHS = 64, REDO_LINE = 32;
+constexpr int REDO_EPOCHS = 16, REDO_LINE = 32;  // (2 KB: small calls pay for them too)
 __device__ __forceinline__ bool redo_many(const RedoList& r, int epoch) {
   typedef const __attribute__((address_space(4))) uint32_t* Scalar;  // (a scalar load)
   const int line = (epoch < REDO_EPOCHS ? epoch : REDO_EPOCHS - 1) * REDO_LINE;
